@@ -19,6 +19,7 @@ namespace {
 
 constexpr int THREADS = 256;
 constexpr float MASK_FILL = -1e30f;  // src/deciax/kernels/attention/reference.py:8
+constexpr float LOG2E = 1.4426950408889634f;
 
 DX_DEVICE float wave_reduce_sum(float v) {
 #pragma unroll
@@ -72,53 +73,120 @@ layer_norm_f32_kernel(const float *__restrict__ x, const float *__restrict__ w, 
   for (int i = lane; i < d; i += 64) yr[i] = (xr[i] - mean) * r * w[i] + (b ? b[i] : 0.f);
 }
 
-// y[m, n] = (acc ? y[m, n] : 0) + act(x[m, :] . w[n, :] + bias[n]); 64 x 64 output tile, 4 x 4 per
-// thread, k in chunks of 16 through LDS. act: 0 identity, 1 exact GELU.
-__global__ void __launch_bounds__(THREADS)
+// fp32 products on the matrix core: v_mfma_f32_16x16x4_f32 (fp32 products and sums, 256 FLOP per cycle and
+// CU). Lane l supplies A row (l % 16) and B column (l % 16) at contraction index l / 16, and gets back column
+// l % 16, rows (l / 16) * 4 + r. Which four contraction indices meet in one MFMA is free, so a lane takes runs of
+// consecutive ones: its operands are 16-byte loads straight from global memory, no LDS.
+DX_DEVICE floatx4 mfma16_f32(float a, float b, floatx4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// y[m, n] = (acc ? y[m, n] : 0) + act(x[m, :] . w[n, :] + bias[n]); act: 0 identity, 1 exact GELU.
+// A wave computes 16 TM x 16 TN outputs over its share of k: KW waves of the workgroup split k in runs of 16 KC
+// (interleaved, so together they read whole cache lines) and add their sums through LDS; WM x WN such groups
+// stand side by side. A wave's lane (l % 16, l / 16) holds k values k0 + 16 c + 4 (l / 16) .. + 3 of its row, for
+// chunks c < KC, loaded one step ahead into the other half of its registers. Rows past m and n read the last
+// row (not stored). VEC: rows are 16-byte aligned, else elements are read one at a time.
+template <int TM, int TN, int KW, int WM, int WN, int KC, bool VEC>
+__global__ void __launch_bounds__(64 * KW * WM * WN)
 linear_f32_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
                   float *__restrict__ y, long m, int n, int k, long ldx, long ldw, long ldy, int act, int acc) {
-  __shared__ float xs[16][65];
-  __shared__ float ws[16][65];
-  const long m0 = (long)blockIdx.y * 64;
-  const int n0 = blockIdx.x * 64;
-  const int tid = threadIdx.x, tr = tid / 16, tc = tid % 16;
-  float c[4][4] = {};
-  for (int k0 = 0; k0 < k; k0 += 16) {
-    for (int idx = tid; idx < 64 * 16; idx += THREADS) {
-      const int r = idx / 16, kk = idx % 16;
-      const long gm = m0 + r;
-      const int gn = n0 + r, gk = k0 + kk;
-      xs[kk][r] = (gm < m && gk < k) ? x[gm * ldx + gk] : 0.f;
-      ws[kk][r] = (gn < n && gk < k) ? w[(long)gn * ldw + gk] : 0.f;
+  constexpr int STEP = 16 * KC;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kw = wave % KW, wn = wave / KW % WN, wm = wave / (KW * WN);
+  const int lr = lane & 15, lk = lane >> 4;
+  const long m0 = ((long)blockIdx.y * WM + wm) * (16 * TM);
+  const int n0 = ((int)blockIdx.x * WN + wn) * (16 * TN);
+  const float *xp[TM], *wp[TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) xp[i] = x + min(m0 + 16 * i + lr, m - 1) * ldx + 4 * lk;
+#pragma unroll
+  for (int j = 0; j < TN; ++j) wp[j] = w + (long)min(n0 + 16 * j + lr, n - 1) * ldw + 4 * lk;
+
+  auto load4 = [&](const float *p, int kk) __attribute__((always_inline)) {  // p[kk .. kk + 3], zeros from k on
+    floatx4 v = {0.f, 0.f, 0.f, 0.f};
+    const int left = k - 4 * lk - kk;
+    if (VEC && left >= 4) {
+      v = *reinterpret_cast<const floatx4 *>(p + kk);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (e < left) v[e] = p[kk + e];
     }
-    __syncthreads();
+    return v;
+  };
+  floatx4 c[TM][TN] = {};
+  floatx4 a0[TM][KC], b0[TN][KC], a1[TM][KC], b1[TN][KC];
+  auto load = [&](floatx4 (&a)[TM][KC], floatx4 (&b)[TN][KC], int kk) __attribute__((always_inline)) {
+    if (VEC && kk + STEP <= k) {
 #pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      float a[4], bb[4];
+      for (int s = 0; s < KC; ++s) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        a[i] = xs[kk][tr * 4 + i];
-        bb[i] = ws[kk][tc * 4 + i];
+        for (int i = 0; i < TM; ++i) a[i][s] = *reinterpret_cast<const floatx4 *>(xp[i] + kk + 16 * s);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) b[j][s] = *reinterpret_cast<const floatx4 *>(wp[j] + kk + 16 * s);
       }
+    } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int s = 0; s < KC; ++s) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) c[i][j] = fmaf(a[i], bb[j], c[i][j]);
+        for (int i = 0; i < TM; ++i) a[i][s] = load4(xp[i], kk + 16 * s);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) b[j][s] = load4(wp[j], kk + 16 * s);
+      }
     }
-    __syncthreads();
+  };
+  auto mma = [&](const floatx4 (&a)[TM][KC], const floatx4 (&b)[TN][KC]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < KC; ++s)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) c[i][j] = mfma16_f32(a[i][s][e], b[j][s][e], c[i][j]);
+  };
+  constexpr int STRIDE = STEP * KW;
+  int kk = kw * STEP;
+  if (kk < k) load(a0, b0, kk);
+  for (; kk < k; kk += 2 * STRIDE) {
+    const int k1 = kk + STRIDE, k2 = kk + 2 * STRIDE;
+    if (k1 < k) load(a1, b1, k1);
+    mma(a0, b0);
+    if (k1 >= k) break;
+    if (k2 < k) load(a0, b0, k2);
+    mma(a1, b1);
   }
+
+  auto store = [&](long gm, int gn, float v) __attribute__((always_inline)) {
+    if (gm >= m || gn >= n) return;
+    v += bias ? bias[gn] : 0.f;
+    if (act == 1) v = gelu_erf(v);
+    float *dst = y + gm * ldy + gn;
+    *dst = acc ? *dst + v : v;
+  };
+  if constexpr (KW == 1) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const long gm = m0 + tr * 4 + i;
-    if (gm >= m) continue;
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int gn = n0 + tc * 4 + j;
-      if (gn >= n) continue;
-      float v = c[i][j] + (bias ? bias[gn] : 0.f);
-      if (act == 1) v = gelu_erf(v);
-      float *dst = y + gm * ldy + gn;
-      *dst = acc ? *dst + v : v;
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) store(m0 + 16 * i + 4 * lk + r, n0 + 16 * j + lr, c[i][j][r]);
+  } else {
+    static_assert(WM == 1 && WN == 1, "k-split workgroups hold one tile");
+    constexpr int TILE = 256 * TM * TN;
+    __shared__ float part[KW * TILE];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          part[kw * TILE + (16 * i + 4 * lk + r) * (16 * TN) + 16 * j + lr] = c[i][j][r];
+    __syncthreads();
+    for (int idx = tid; idx < TILE; idx += 64 * KW) {
+      float v = 0.f;
+#pragma unroll
+      for (int q = 0; q < KW; ++q) v += part[q * TILE + idx];
+      store(m0 + idx / (16 * TN), n0 + idx % (16 * TN), v);
     }
   }
 }
@@ -184,6 +252,171 @@ mha_f32_kernel(const float *__restrict__ q, const float *__restrict__ k, const f
       out[((long)b * Q + qi) * ldo + (long)h * dh + d0 + threadIdx.x] = t / sum;
     }
     __syncthreads();
+  }
+}
+
+// The same on the matrix core, head_dim D = 16 N <= 128, 16-byte aligned rows. A workgroup takes 16 QB queries of
+// one (b, head); its WAVES waves take 16 SUB-key blocks in turn, each with its own running max m, row sum l and O,
+// merged through LDS at the end (no barrier in the key loop). Layouts (see mfma16_f32):
+//   S^T = K Q^T   contraction over head dims: lane (r, g) = (l % 16, l / 16) holds dims [4 N g, 4 N g + 4 N) of key
+//                 row r and of query r, MFMA j contracting dim 4 N g + j of the four groups. It gets back query r,
+//                 keys 4 g + 0..3 of the 16.
+//   O^T += V^T P^T MFMA t contracts keys 4 g + t, whose probabilities the lane already holds; V rows come as N
+//                 consecutive floats [N r, N r + N) of key 4 g + t, block c (c < N) taking float c, so the lane
+//                 ends up with the 4 N consecutive dims [4 N g, 4 N g + 4 N) of query r.
+// K of the next block is requested as soon as this block's scores are done, V at the start of its block.
+template <int N>
+DX_DEVICE void load_run(float (&v)[N], const float *p) {  // N consecutive floats, aligned as far as N allows
+  if constexpr (N % 4 == 0) {
+#pragma unroll
+    for (int i = 0; i < N; i += 4) {
+      const floatx4 t = *reinterpret_cast<const floatx4 *>(p + i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[i + e] = t[e];
+    }
+  } else if constexpr (N % 2 == 0) {
+#pragma unroll
+    for (int i = 0; i < N; i += 2) {
+      const float2 t = *reinterpret_cast<const float2 *>(p + i);
+      v[i] = t.x;
+      v[i + 1] = t.y;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = p[i];
+  }
+}
+
+template <int N, int QB, int WAVES, int SUB>
+__global__ void __launch_bounds__(64 * WAVES)
+mha_f32_mfma_kernel(const float *__restrict__ q, const float *__restrict__ k, const float *__restrict__ v,
+                    const uint8_t *__restrict__ key_mask, float *__restrict__ out, int Q, int K, long ldq, long ldk,
+                    long ldv, long ldo) {
+  constexpr int D = 16 * N, KB = 16 * SUB;
+  constexpr float NONE = -3e38f;  // running max before any key: below MASK_FILL
+  __shared__ float os[WAVES][16 * QB][D + 4];
+  __shared__ float ms[WAVES][16 * QB], ls[WAVES][16 * QB];
+  const int h = blockIdx.y, b = blockIdx.z, q0 = blockIdx.x * 16 * QB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
+  const float scale = 1.0f / sqrtf((float)D);
+  const float *kb = k + (long)b * K * ldk + (long)h * D + 4 * N * g;
+  const float *vb = v + (long)b * K * ldv + (long)h * D + N * r16;
+  const uint8_t *mb = key_mask + (long)b * K;
+
+  float qf[QB][4 * N];
+#pragma unroll
+  for (int u = 0; u < QB; ++u)
+    load_run<4 * N>(qf[u], q + ((long)b * Q + min(q0 + 16 * u + r16, Q - 1)) * ldq + (long)h * D + 4 * N * g);
+
+  float kf[SUB][4 * N];
+  auto load_k = [&](int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < SUB; ++s) load_run<4 * N>(kf[s], kb + (long)min(k0 + 16 * s + r16, K - 1) * ldk);
+  };
+  floatx4 o[QB][N] = {};
+  float mr[QB], l[QB];
+#pragma unroll
+  for (int u = 0; u < QB; ++u) {
+    mr[u] = NONE;
+    l[u] = 0.f;
+  }
+  int k0 = wave * KB;
+  if (k0 < K) load_k(k0);
+  for (; k0 < K; k0 += WAVES * KB) {
+    float vf[SUB][4][N];
+    uint32_t state[SUB];  // 2 bits per key of the lane's four: 0 masked, 1 visible, 2 past the last key
+#pragma unroll
+    for (int s = 0; s < SUB; ++s) {
+      state[s] = 0;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int key = k0 + 16 * s + 4 * g + t;
+        load_run<N>(vf[s][t], vb + (long)min(key, K - 1) * ldv);
+        state[s] |= (key >= K ? 2u : mb[key] ? 1u : 0u) << (2 * t);
+      }
+    }
+    floatx4 sc[QB][SUB];
+#pragma unroll
+    for (int u = 0; u < QB; ++u)
+#pragma unroll
+      for (int s = 0; s < SUB; ++s) sc[u][s] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 4 * N; ++j)
+#pragma unroll
+      for (int s = 0; s < SUB; ++s)
+#pragma unroll
+        for (int u = 0; u < QB; ++u) sc[u][s] = mfma16_f32(kf[s][j], qf[u][j], sc[u][s]);
+    if (k0 + WAVES * KB < K) load_k(k0 + WAVES * KB);
+#pragma unroll
+    for (int u = 0; u < QB; ++u) {
+      float mx = NONE;
+#pragma unroll
+      for (int s = 0; s < SUB; ++s)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const uint32_t st = (state[s] >> (2 * t)) & 3u;
+          const float z = st == 1u ? sc[u][s][t] * scale : st == 0u ? MASK_FILL : -INFINITY;
+          sc[u][s][t] = z;
+          mx = fmaxf(mx, z);
+        }
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      const float mn = fmaxf(mr[u], mx);
+      const float alpha = fast_exp2((mr[u] - mn) * LOG2E);
+      mr[u] = mn;
+      l[u] *= alpha;
+      if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {
+#pragma unroll
+        for (int c = 0; c < N; ++c) o[u][c] *= alpha;
+      }
+#pragma unroll
+      for (int s = 0; s < SUB; ++s)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const float p = fast_exp2((sc[u][s][t] - mn) * LOG2E);
+          sc[u][s][t] = p;
+          l[u] += p;
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < SUB; ++s)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int c = 0; c < N; ++c)
+#pragma unroll
+          for (int u = 0; u < QB; ++u) o[u][c] = mfma16_f32(vf[s][t][c], sc[u][s][t], o[u][c]);
+  }
+#pragma unroll
+  for (int u = 0; u < QB; ++u) {
+    l[u] += __shfl_xor(l[u], 16, 64);
+    l[u] += __shfl_xor(l[u], 32, 64);
+    if (g == 0) {
+      ms[wave][16 * u + r16] = mr[u];
+      ls[wave][16 * u + r16] = l[u];
+    }
+    // block c, register t is dim N (4 g + t) + c of query r16
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int c = 0; c < N; ++c) os[wave][16 * u + r16][N * (4 * g + t) + c] = o[u][c][t];
+  }
+  __syncthreads();
+  for (int idx = tid; idx < 16 * QB * D; idx += 64 * WAVES) {
+    const int qi = idx / D, d = idx % D;
+    if (q0 + qi >= Q) continue;
+    float mx = ms[0][qi];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) mx = fmaxf(mx, ms[w][qi]);
+    float num = 0.f, den = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float f = fast_exp2((ms[w][qi] - mx) * LOG2E);
+      num += os[w][qi][d] * f;
+      den += ls[w][qi] * f;
+    }
+    out[((long)b * Q + q0 + qi) * ldo + (long)h * D + d] = num / den;
   }
 }
 
@@ -315,10 +548,24 @@ hipError_t dx_layer_norm_f32_launch(const float *x, const float *w, const float 
   return hipGetLastError();
 }
 
+template <int TM, int TN, int KW, int WM, int WN, int KC>
+static void linear_run(const float *x, const float *w, const float *bias, float *y, long m, int n, int k, long ldx,
+                       long ldw, long ldy, int act, int acc, hipStream_t s) {
+  const bool vec = ((ldx | ldw) & 3) == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
+  const dim3 grid(blocks(n, 16 * TN * WN), blocks(m, 16 * TM * WM));
+  auto kern = vec ? linear_f32_kernel<TM, TN, KW, WM, WN, KC, true> : linear_f32_kernel<TM, TN, KW, WM, WN, KC, false>;
+  kern<<<grid, 64 * KW * WM * WN, 0, s>>>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc);
+}
+
 hipError_t dx_linear_f32_launch(const float *x, const float *w, const float *bias, float *y, long m, int n, int k,
                                 long ldx, long ldw, long ldy, int act, int acc, hipStream_t s) {
-  const dim3 grid(blocks(n, 64), blocks(m, 64));
-  linear_f32_kernel<<<grid, THREADS, 0, s>>>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc);
+  const long big = (m + 127) / 128 * ((n + 127) / 128), mid = (m + 31) / 32 * ((n + 31) / 32);
+  if (big >= 192)
+    linear_run<4, 4, 1, 2, 2, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s);
+  else if (mid >= 256)
+    linear_run<2, 2, 4, 1, 1, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s);
+  else
+    linear_run<1, 1, 16, 1, 1, 4>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s);
   return hipGetLastError();
 }
 
@@ -328,8 +575,34 @@ hipError_t dx_span_means_f32_launch(const float *x, const int32_t *spans, float 
   return hipGetLastError();
 }
 
+template <int N>
+static void mha_run(const float *q, const float *k, const float *v, const uint8_t *key_mask, float *out, int B, int Q,
+                    int K, int H, long ldq, long ldk, long ldv, long ldo, hipStream_t s) {
+  constexpr int SUB = N <= 4 ? 4 : 2;
+  if ((long)B * H * ((Q + 31) / 32) >= 512)
+    mha_f32_mfma_kernel<N, 2, 4, SUB><<<dim3((Q + 31) / 32, H, B), 256, 0, s>>>(q, k, v, key_mask, out, Q, K, ldq, ldk,
+                                                                              ldv, ldo);
+  else
+    mha_f32_mfma_kernel<N, 1, 8, SUB><<<dim3((Q + 15) / 16, H, B), 512, 0, s>>>(q, k, v, key_mask, out, Q, K, ldq, ldk,
+                                                                              ldv, ldo);
+}
+
 hipError_t dx_mha_f32_launch(const float *q, const float *k, const float *v, const uint8_t *key_mask, float *out,
                              int B, int Q, int K, int H, int dh, long ldq, long ldk, long ldv, long ldo, hipStream_t s) {
+  const uintptr_t addr = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v);
+  if (dh % 16 == 0 && dh <= 128 && ((ldq | ldk | ldv) & 3) == 0 && (addr & 15) == 0 && H <= 65535 && B <= 65535) {
+    switch (dh / 16) {
+      case 1: mha_run<1>(q, k, v, key_mask, out, B, Q, K, H, ldq, ldk, ldv, ldo, s); break;
+      case 2: mha_run<2>(q, k, v, key_mask, out, B, Q, K, H, ldq, ldk, ldv, ldo, s); break;
+      case 3: mha_run<3>(q, k, v, key_mask, out, B, Q, K, H, ldq, ldk, ldv, ldo, s); break;
+      case 4: mha_run<4>(q, k, v, key_mask, out, B, Q, K, H, ldq, ldk, ldv, ldo, s); break;
+      case 5: mha_run<5>(q, k, v, key_mask, out, B, Q, K, H, ldq, ldk, ldv, ldo, s); break;
+      case 6: mha_run<6>(q, k, v, key_mask, out, B, Q, K, H, ldq, ldk, ldv, ldo, s); break;
+      case 7: mha_run<7>(q, k, v, key_mask, out, B, Q, K, H, ldq, ldk, ldv, ldo, s); break;
+      default: mha_run<8>(q, k, v, key_mask, out, B, Q, K, H, ldq, ldk, ldv, ldo, s); break;
+    }
+    return hipGetLastError();
+  }
   const size_t shm = ((size_t)K + THREADS) * sizeof(float);
   mha_f32_kernel<<<(unsigned)(B * Q * H), THREADS, shm, s>>>(q, k, v, key_mask, out, Q, K, H, dh, ldq, ldk, ldv, ldo);
   return hipGetLastError();

@@ -161,3 +161,59 @@ def test_encoded_requests_through_head() -> None:
         assert ours["answers"]["mood"]["choice"] == theirs["answers"]["mood"]["choice"]
         assert ours["answers"]["late"]["noul"] == pytest.approx(theirs["answers"]["late"]["noul"], abs=2e-4)
         assert ours["answers"]["stars"]["score"] == pytest.approx(theirs["answers"]["stars"]["score"], abs=2e-4)
+
+
+@pytest.mark.parametrize("m,n,k,pad", [
+    (1, 1, 1, 0), (3, 17, 31, 0), (16, 16, 64, 0), (17, 1000, 1029, 3),   # 16 x 16 tiles, k over 16 waves
+    (300, 1000, 96, 0), (513, 515, 100, 1),                              # 32 x 32 tiles, k over 4 waves
+    (4097, 769, 130, 4), (20000, 200, 36, 0),                            # 128 x 128 tiles
+])
+def test_linear_f32_tiles(m: int, n: int, k: int, pad: int) -> None:
+    """Every tile shape at its edges, rows with and without 16-byte alignment, bias, GELU and accumulation, against
+    the product in 64 bits. A sum of k fp32 products in any order is within k 2^-24 sum |x w| of it."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    say(f"linear_f32 {m} x {n} x {k}, row padding {pad}")
+    r = rng(m + n + k)
+    x = torch.as_tensor(r.normal(size=(m, k + pad)).astype(np.float32)).cuda()[:, :k]
+    w = torch.as_tensor(r.normal(size=(n, k + pad)).astype(np.float32)).cuda()[:, :k]
+    b = torch.as_tensor(r.normal(size=n).astype(np.float32)).cuda()
+    want = x.double() @ w.double().t()
+    bound = (k + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + b.double().abs()) + 1e-30
+    assert ((K.linear_f32(x, w).double() - want).abs() <= bound).all()
+    base = torch.as_tensor(r.normal(size=(m, n)).astype(np.float32)).cuda()
+    got = K.linear_f32(x, w, b, gelu=True, out=base.clone(), accumulate=True).double()
+    act = torch.nn.functional.gelu(want + b.double())
+    # GELU has slope at most 1.13; erff and the three roundings after it add a few ulp of the result
+    assert ((got - base.double() - act).abs() <= 1.2 * bound + 2.0 ** -21 * (act.abs() + base.double().abs()) + 1e-6).all()
+
+
+@pytest.mark.parametrize("batch,nq,nk,heads,dh", [
+    (1, 1, 1, 1, 16), (2, 17, 65, 3, 32), (1, 6, 600, 16, 64), (2, 33, 130, 2, 48), (1, 5, 70, 2, 80), (1, 40, 64, 2, 96),
+    (2, 20, 31, 2, 112), (1, 50, 515, 4, 128), (8, 40, 127, 40, 64), (1, 9, 40, 2, 24),
+])
+def test_mha_f32_forms(batch: int, nq: int, nk: int, heads: int, dh: int) -> None:
+    """Matrix-core head dims, both workgroup forms and the general kernel (dh 24) against the masked softmax in 64
+    bits, with holes in the mask and one batch row that keeps no key (the uniform average)."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    say(f"mha_f32 {batch} x {nq} x {nk}, {heads} heads x {dh}")
+    r = rng(nq + nk + dh)
+    w = heads * dh
+    q, k, v = (torch.as_tensor(r.normal(size=(batch * t, w)).astype(np.float32)).cuda() for t in (nq, nk, nk))
+    mask = torch.as_tensor(r.random((batch, nk)) < 0.7).to(torch.uint8).cuda()
+    mask[:, 0] = 1
+    if batch > 1:
+        mask[-1] = 0
+    got = K.mha_f32(q, k, v, mask, batch=batch, heads=heads).double()
+    split = lambda t: t.double().view(batch, -1, heads, dh).transpose(1, 2)  # noqa: E731
+    s = split(q) @ split(k).transpose(-1, -2) / dh ** 0.5
+    p = torch.softmax(s.masked_fill(~mask.bool()[:, None, None, :], -1e30), -1)
+    want = (p @ split(v)).transpose(1, 2).reshape(batch * nq, w)
+    # scores of dh products: relative 2^-24 (dh + 4) of sum |q k|, a few units; the weights inherit it
+    err = (got - want).abs().max().item()
+    assert err < 4 * 2.0 ** -24 * (dh + 16) * float((split(q).abs() @ split(k).abs().transpose(-1, -2)).max()) / dh ** 0.5, err
