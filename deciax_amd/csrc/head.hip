@@ -101,38 +101,32 @@ linear_f32_kernel(const float *__restrict__ x, const float *__restrict__ w, cons
 #pragma unroll
   for (int j = 0; j < TN; ++j) wp[j] = w + (long)min(n0 + 16 * j + lr, n - 1) * ldw + 4 * lk;
 
-  auto load4 = [&](const float *p, int kk) __attribute__((always_inline)) {  // p[kk .. kk + 3], zeros from k on
-    floatx4 v = {0.f, 0.f, 0.f, 0.f};
-    const int left = k - 4 * lk - kk;
-    if (VEC && left >= 4) {
-      v = *reinterpret_cast<const floatx4 *>(p + kk);
+  auto load4 = [&](const float *p) __attribute__((always_inline)) {
+    if constexpr (VEC) {
+      return *reinterpret_cast<const floatx4 *>(p);
     } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (e < left) v[e] = p[kk + e];
+      const floatx4 v = {p[0], p[1], p[2], p[3]};
+      return v;
     }
-    return v;
   };
   floatx4 c[TM][TN] = {};
   floatx4 a0[TM][KC], b0[TN][KC], a1[TM][KC], b1[TN][KC];
+  // a whole step at kk
   auto load = [&](floatx4 (&a)[TM][KC], floatx4 (&b)[TN][KC], int kk) __attribute__((always_inline)) {
-    if (VEC && kk + STEP <= k) {
 #pragma unroll
-      for (int s = 0; s < KC; ++s) {
+    for (int s = 0; s < KC; ++s) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i) a[i][s] = *reinterpret_cast<const floatx4 *>(xp[i] + kk + 16 * s);
+      for (int i = 0; i < TM; ++i) a[i][s] = load4(xp[i] + kk + 16 * s);
 #pragma unroll
-        for (int j = 0; j < TN; ++j) b[j][s] = *reinterpret_cast<const floatx4 *>(wp[j] + kk + 16 * s);
-      }
-    } else {
-#pragma unroll
-      for (int s = 0; s < KC; ++s) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i) a[i][s] = load4(xp[i], kk + 16 * s);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) b[j][s] = load4(wp[j], kk + 16 * s);
-      }
+      for (int j = 0; j < TN; ++j) b[j][s] = load4(wp[j] + kk + 16 * s);
     }
+  };
+  auto part4 = [&](const float *p, int left) __attribute__((always_inline)) {  // the first `left` of 4, then zeros
+    floatx4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (e < left) v[e] = p[e];
+    return v;
   };
   auto mma = [&](const floatx4 (&a)[TM][KC], const floatx4 (&b)[TN][KC]) __attribute__((always_inline)) {
 #pragma unroll
@@ -144,16 +138,34 @@ linear_f32_kernel(const float *__restrict__ x, const float *__restrict__ w, cons
 #pragma unroll
           for (int j = 0; j < TN; ++j) c[i][j] = mfma16_f32(a[i][s][e], b[j][s][e], c[i][j]);
   };
-  constexpr int STRIDE = STEP * KW;
-  int kk = kw * STEP;
-  if (kk < k) load(a0, b0, kk);
-  for (; kk < k; kk += 2 * STRIDE) {
-    const int k1 = kk + STRIDE, k2 = kk + 2 * STRIDE;
-    if (k1 < k) load(a1, b1, k1);
+  // whole steps kw, kw + KW, ... (the prefetch past the last reloads it), then the partial one, if any
+  const int full = k / STEP;
+  const int mine = full > kw ? (full - kw - 1) / KW + 1 : 0;
+  auto at = [&](int t) { return (kw + min(t, mine - 1) * KW) * STEP; };
+  if (mine > 0) {
+    load(a0, b0, at(0));
+    int t = 0;
+    for (; t + 1 < mine; t += 2) {
+      load(a1, b1, at(t + 1));
+      __builtin_amdgcn_sched_barrier(0);  // the next step's loads go out before this step's products
+      mma(a0, b0);
+      load(a0, b0, at(t + 2));
+      __builtin_amdgcn_sched_barrier(0);
+      mma(a1, b1);
+    }
+    if (t < mine) mma(a0, b0);
+  }
+  if (k % STEP && kw == full % KW) {
+    const int kk = full * STEP;
+#pragma unroll
+    for (int s = 0; s < KC; ++s) {
+      const int left = k - kk - 16 * s - 4 * lk;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a0[i][s] = part4(xp[i] + kk + 16 * s, left);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) b0[j][s] = part4(wp[j] + kk + 16 * s, left);
+    }
     mma(a0, b0);
-    if (k1 >= k) break;
-    if (k2 < k) load(a0, b0, k2);
-    mma(a1, b1);
   }
 
   auto store = [&](long gm, int gn, float v) __attribute__((always_inline)) {
@@ -325,17 +337,13 @@ mha_f32_mfma_kernel(const float *__restrict__ q, const float *__restrict__ k, co
   if (k0 < K) load_k(k0);
   for (; k0 < K; k0 += WAVES * KB) {
     float vf[SUB][4][N];
-    uint32_t state[SUB];  // 2 bits per key of the lane's four: 0 masked, 1 visible, 2 past the last key
+    // one mask byte per lane covers the block (KB <= 64 keys); bit 16 s + 4 g + t is the lane's key (s, t)
+    const uint8_t mk = mb[min(k0 + min(lane, KB - 1), K - 1)];
 #pragma unroll
-    for (int s = 0; s < SUB; ++s) {
-      state[s] = 0;
+    for (int s = 0; s < SUB; ++s)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int key = k0 + 16 * s + 4 * g + t;
-        load_run<N>(vf[s][t], vb + (long)min(key, K - 1) * ldv);
-        state[s] |= (key >= K ? 2u : mb[key] ? 1u : 0u) << (2 * t);
-      }
-    }
+      for (int t = 0; t < 4; ++t) load_run<N>(vf[s][t], vb + (long)min(k0 + 16 * s + 4 * g + t, K - 1) * ldv);
+    const uint64_t vis = __builtin_amdgcn_ballot_w64(mk != 0) >> (4 * g);
     floatx4 sc[QB][SUB];
 #pragma unroll
     for (int u = 0; u < QB; ++u)
@@ -355,8 +363,8 @@ mha_f32_mfma_kernel(const float *__restrict__ q, const float *__restrict__ k, co
       for (int s = 0; s < SUB; ++s)
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-          const uint32_t st = (state[s] >> (2 * t)) & 3u;
-          const float z = st == 1u ? sc[u][s][t] * scale : st == 0u ? MASK_FILL : -INFINITY;
+          const float hidden = k0 + 16 * s + 4 * g + t < K ? MASK_FILL : -INFINITY;
+          const float z = ((vis >> (16 * s + t)) & 1u) && hidden == MASK_FILL ? sc[u][s][t] * scale : hidden;
           sc[u][s][t] = z;
           mx = fmaxf(mx, z);
         }
@@ -578,9 +586,11 @@ hipError_t dx_span_means_f32_launch(const float *x, const int32_t *spans, float 
 template <int N>
 static void mha_run(const float *q, const float *k, const float *v, const uint8_t *key_mask, float *out, int B, int Q,
                     int K, int H, long ldq, long ldk, long ldv, long ldo, hipStream_t s) {
-  constexpr int SUB = N <= 4 ? 4 : 2;
+  // keys per block: as many as leave registers for two waves per SIMD (the softmax of one beside the products of
+  // the other)
+  constexpr int SUB = N <= 4 ? 4 : 2, SUB2 = N <= 2 ? 4 : N <= 5 ? 2 : 1;
   if ((long)B * H * ((Q + 31) / 32) >= 512)
-    mha_f32_mfma_kernel<N, 2, 4, SUB><<<dim3((Q + 31) / 32, H, B), 256, 0, s>>>(q, k, v, key_mask, out, Q, K, ldq, ldk,
+    mha_f32_mfma_kernel<N, 2, 4, SUB2><<<dim3((Q + 31) / 32, H, B), 256, 0, s>>>(q, k, v, key_mask, out, Q, K, ldq, ldk,
                                                                               ldv, ldo);
   else
     mha_f32_mfma_kernel<N, 1, 8, SUB><<<dim3((Q + 15) / 16, H, B), 512, 0, s>>>(q, k, v, key_mask, out, Q, K, ldq, ldk,
