@@ -73,6 +73,47 @@ layer_norm_f32_kernel(const float *__restrict__ x, const float *__restrict__ w, 
   for (int i = lane; i < d; i += 64) yr[i] = (xr[i] - mean) * r * w[i] + (b ? b[i] : 0.f);
 }
 
+// The same with the row in registers (16-byte chunk c = lane + 64 i), so it is read once and all of it at once:
+// d <= 256 MAXC, a multiple of 4, rows and weights 16-byte aligned.
+template <int MAXC>
+__global__ void __launch_bounds__(THREADS)
+layer_norm_f32_row_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ b,
+                          float *__restrict__ y, long rows, int d, long ldx, long ldy, float eps) {
+  const long row = (long)blockIdx.x * (THREADS / 64) + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int lane = threadIdx.x & 63, nch = d / 4;
+  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+  const floatx4 *xr = reinterpret_cast<const floatx4 *>(x + row * ldx);
+  floatx4 v[MAXC];
+#pragma unroll
+  for (int i = 0; i < MAXC; ++i) v[i] = lane + 64 * i < nch ? xr[lane + 64 * i] : zero;
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < MAXC; ++i) s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
+  const float mean = wave_reduce_sum(s) / (float)d;
+  float q = 0.f;
+#pragma unroll
+  for (int i = 0; i < MAXC; ++i)
+    if (lane + 64 * i < nch) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[i][e] -= mean;
+        q += v[i][e] * v[i][e];
+      }
+    }
+  const float r = 1.0f / sqrtf(wave_reduce_sum(q) / (float)d + eps);
+  floatx4 *yr = reinterpret_cast<floatx4 *>(y + row * ldy);
+#pragma unroll
+  for (int i = 0; i < MAXC; ++i) {
+    const int c = lane + 64 * i;
+    if (c < nch) {
+      const floatx4 wc = reinterpret_cast<const floatx4 *>(w)[c];
+      const floatx4 bc = b ? reinterpret_cast<const floatx4 *>(b)[c] : zero;
+      yr[c] = v[i] * r * wc + bc;
+    }
+  }
+}
+
 // fp32 products on the matrix core: v_mfma_f32_16x16x4_f32 (fp32 products and sums, 256 FLOP per cycle and
 // CU). Lane l supplies A row (l % 16) and B column (l % 16) at contraction index l / 16, and gets back column
 // l % 16, rows (l / 16) * 4 + r. Which four contraction indices meet in one MFMA is free, so a lane takes runs of
@@ -204,18 +245,33 @@ linear_f32_kernel(const float *__restrict__ x, const float *__restrict__ w, cons
 }
 
 // out[b * O + o, :] = mean of x[b * S + s, :] over s in [spans[b, o, 0], spans[b, o, 1]) (within
-// [0, S)); an empty span gives 0 (head.py:28 divides by max(count, 1)).
+// [0, S)); an empty span gives 0 (head.py:28 divides by max(count, 1)). One workgroup per span and 256 columns.
 __global__ void __launch_bounds__(THREADS)
 span_means_f32_kernel(const float *__restrict__ x, const int32_t *__restrict__ spans, float *__restrict__ out, int S,
                       int O, int d, long ldx, long ldo) {
-  const int bo = blockIdx.x, b = bo / O;
+  const int bo = blockIdx.x, b = bo / O, i = blockIdx.y * THREADS + threadIdx.x;
   const int lo = max(spans[2 * bo], 0), hi = min(spans[2 * bo + 1], S);
+  if (i >= d) return;
   const float inv = 1.0f / (float)max(hi - lo, 1);
-  for (int i = threadIdx.x; i < d; i += THREADS) {
-    float s = 0.f;
-    for (int t = lo; t < hi; ++t) s += x[((long)b * S + t) * ldx + i];
-    out[(long)bo * ldo + i] = hi > lo ? s * inv : 0.f;
+  const float *p = x + ((long)b * S + lo) * ldx + i;
+  float s = 0.f;
+  int t = lo;
+  for (; t + 8 <= hi; t += 8, p += 8 * ldx) {  // eight rows in flight, added in order
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = p[e * ldx];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s += v[e];
   }
+  if (t < hi) {
+    float v[7];
+#pragma unroll
+    for (int e = 0; e < 7; ++e) v[e] = p[min(e, hi - 1 - t) * ldx];
+#pragma unroll
+    for (int e = 0; e < 7; ++e)
+      if (t + e < hi) s += v[e];
+  }
+  out[(long)bo * ldo + i] = hi > lo ? s * inv : 0.f;
 }
 
 // One workgroup per (b, query, head): scores over the K keys of batch row b into LDS, masked keys at
@@ -439,40 +495,75 @@ gather_rows_f32_kernel(const float *__restrict__ x, const int32_t *__restrict__ 
   for (int i = threadIdx.x; i < d; i += THREADS) dst[i] = acc ? dst[i] + src[i] : src[i];
 }
 
-// One workgroup per (b, question qi): logits[o] = options[b, o] . base[b, qi] / sqrt(W) over options
-// this question owns (owner == qi and option_mask), MASK_FILL elsewhere; routing = softmax over o;
-// summary[b, qi] = sum_o routing[o] * options[b, o] (head.py:76-85).
+// logits[o] = options[b, o] . base[b, qi] / sqrt(W) over the options question qi owns (owner == qi and option_mask),
+// MASK_FILL elsewhere; routing = softmax over o; summary[b, qi] = sum_o routing[o] * options[b, o] (head.py:76-85).
+// A workgroup takes FG questions of b and 256 columns of the summary, so the options are read once per FG questions
+// there. Its waves share out the dot products of the owned options (the others need none), which every column
+// block repeats: they are few next to the sum's rows.
+template <int FG>
 __global__ void __launch_bounds__(THREADS)
 routing_f32_kernel(const float *__restrict__ options, const float *__restrict__ base, const int32_t *__restrict__ owner,
                    const uint8_t *__restrict__ option_mask, float *__restrict__ summary, int O, int NQ, int W) {
-  extern __shared__ float p[];  // O routing weights
-  __shared__ float red[4];
-  const int qi = blockIdx.x % NQ, b = blockIdx.x / NQ;
-  const float *br = base + ((long)b * NQ + qi) * W;
+  extern __shared__ __attribute__((aligned(16))) float p[];  // [O][FG] routing weights
+  constexpr int WAVES = THREADS / 64;
+  const int b = blockIdx.z, f0 = blockIdx.y * FG, nf = min(FG, NQ - f0);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const float *ob = options + (long)b * O * W;
   const float inv = 1.0f / sqrtf((float)W);
-  float mx = MASK_FILL;
-  for (int o = threadIdx.x; o < O; o += THREADS) {
-    const float *orow = options + ((long)b * O + o) * W;
-    float s = 0.f;
-    for (int i = 0; i < W; ++i) s = fmaf(orow[i], br[i], s);
-    const bool owns = owner[(long)b * O + o] == qi && option_mask[(long)b * O + o];
-    s = owns ? s * inv : MASK_FILL;
-    p[o] = s;
-    mx = fmaxf(mx, s);
+  for (int i = threadIdx.x; i < O * FG; i += THREADS) p[i] = MASK_FILL;
+  __syncthreads();
+  int seen = 0;
+  for (int o0 = 0; o0 < O; o0 += 64) {
+    const int o = o0 + lane;
+    int rel = -1;
+    if (o < O && option_mask[(long)b * O + o]) rel = owner[(long)b * O + o] - f0;
+    for (uint64_t bits = __builtin_amdgcn_ballot_w64(rel >= 0 && rel < nf); bits; bits &= bits - 1) {
+      if (seen++ % WAVES != wave) continue;
+      const int j = __builtin_ctzll(bits), f = __builtin_amdgcn_readlane(rel, j);
+      const float *orow = ob + (long)(o0 + j) * W, *br = base + ((long)b * NQ + f0 + f) * W;
+      float s = 0.f;
+#pragma unroll 8
+      for (int i = lane; i < W; i += 64) s = fmaf(orow[i], br[i], s);
+      s = wave_reduce_sum(s);
+      if (lane == 0) p[(o0 + j) * FG + f] = s * inv;
+    }
   }
-  mx = block_max(mx, red);
-  float sum = 0.f;
-  for (int o = threadIdx.x; o < O; o += THREADS) {
-    const float e = expf(p[o] - mx);
-    p[o] = e;
-    sum += e;
+  __syncthreads();
+  for (int f = wave; f < nf; f += WAVES) {
+    float mx = MASK_FILL;
+    for (int o = lane; o < O; o += 64) mx = fmaxf(mx, p[o * FG + f]);
+    mx = wave_reduce_max(mx);
+    float sum = 0.f;
+    for (int o = lane; o < O; o += 64) {
+      const float e = expf(p[o * FG + f] - mx);
+      p[o * FG + f] = e;
+      sum += e;
+    }
+    sum = wave_reduce_sum(sum);
+    for (int o = lane; o < O; o += 64) p[o * FG + f] /= sum;
   }
-  sum = block_sum(sum, red);
-  for (int i = threadIdx.x; i < W; i += THREADS) {
-    float s = 0.f;
-    for (int o = 0; o < O; ++o) s += (p[o] / sum) * options[((long)b * O + o) * W + i];
-    summary[((long)b * NQ + qi) * W + i] = s;
+  __syncthreads();
+  const int i = blockIdx.x * THREADS + threadIdx.x;
+  if (i >= W) return;
+  float s[FG] = {};
+  int o = 0;
+  for (; o + 16 <= O; o += 16) {
+    float v[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) v[e] = ob[(long)(o + e) * W + i];
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+#pragma unroll
+      for (int f = 0; f < FG; ++f) s[f] += p[(o + e) * FG + f] * v[e];
   }
+  for (; o < O; ++o) {
+    const float v = ob[(long)o * W + i];
+#pragma unroll
+    for (int f = 0; f < FG; ++f) s[f] += p[o * FG + f] * v;
+  }
+#pragma unroll
+  for (int f = 0; f < FG; ++f)
+    if (f < nf) summary[((long)b * NQ + f0 + f) * W + i] = s[f];
 }
 
 // fields[b, qi] = base[b, qi] + summary_norm[b, qi] + glob[b] + type_emb[types[b, qi]]
@@ -552,7 +643,15 @@ unsigned blocks(long n, int per) { return (unsigned)((n + per - 1) / per); }
 
 hipError_t dx_layer_norm_f32_launch(const float *x, const float *w, const float *b, float *y, long rows, int d,
                                     long ldx, long ldy, float eps, hipStream_t s) {
-  layer_norm_f32_kernel<<<blocks(rows, THREADS / 64), THREADS, 0, s>>>(x, w, b, y, rows, d, ldx, ldy, eps);
+  const uintptr_t addr = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |
+                         reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(y);
+  const unsigned grid = blocks(rows, THREADS / 64);
+  if (d % 4 == 0 && d <= 4096 && ((ldx | ldy) & 3) == 0 && (addr & 15) == 0) {
+    auto kern = d <= 1024 ? layer_norm_f32_row_kernel<4> : layer_norm_f32_row_kernel<16>;
+    kern<<<grid, THREADS, 0, s>>>(x, w, b, y, rows, d, ldx, ldy, eps);
+    return hipGetLastError();
+  }
+  layer_norm_f32_kernel<<<grid, THREADS, 0, s>>>(x, w, b, y, rows, d, ldx, ldy, eps);
   return hipGetLastError();
 }
 
@@ -567,19 +666,40 @@ static void linear_run(const float *x, const float *w, const float *bias, float 
 
 hipError_t dx_linear_f32_launch(const float *x, const float *w, const float *bias, float *y, long m, int n, int k,
                                 long ldx, long ldw, long ldy, int act, int acc, hipStream_t s) {
-  const long big = (m + 127) / 128 * ((n + 127) / 128), mid = (m + 31) / 32 * ((n + 31) / 32);
-  if (big >= 192)
-    linear_run<4, 4, 1, 2, 2, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s);
-  else if (mid >= 256)
-    linear_run<2, 2, 4, 1, 1, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s);
-  else
-    linear_run<1, 1, 16, 1, 1, 4>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s);
+  // Each form's time is its rounds of waves over the 1024 SIMDs times a wave's share of one 64 x 64 x k product,
+  // and the smaller tiles re-read their operands more often: a 64 x 32, 32 x 32 or 16 x 16 wave runs at 0.7, 0.55
+  // or 0.22 of the 64 x 64 wave's rate (measured; us, 64 x 64 with k whole / split 2 / 4, 64 x 32, 32 x 32, 16 x 16):
+  //   23 x 1024 x 4096: 249 / 126 / 67, 35, 28, 20     200 x 1024 x 1024: 72 / 38 / 24, 16, 11, 18
+  //   512 x 1024 x 1024: 71 / 38 / 25, 17, 20, 36      600 x 2048 x 1024: 72 / 41 / 47, 48, 44, 80
+  //   1200 x 2048 x 1024: 74 / 80 / 71, 84, 84, 156    2000 x 1024 x 4096: 264 / 137 / 151, 225, 237, 566
+  //   32768 x 2048 x 1024: 1143 / 1327 / 1443, 1700, 2015, -
+  auto tiles = [&](int tm, int tn) { return (m + tm - 1) / tm * ((n + tn - 1) / tn); };
+  auto rounds = [](long waves) { return (double)((waves + 1023) / 1024); };
+  const long t64 = tiles(64, 64);
+  const double cost[6] = {rounds(t64),
+                          rounds(2 * t64) / 2,
+                          rounds(4 * t64) / 4,
+                          rounds(4 * tiles(64, 32)) / 8 * 1.45,
+                          rounds(4 * tiles(32, 32)) / 16 * 1.8,
+                          rounds(16 * tiles(16, 16)) / 256 * 4.5};
+  int best = 0;
+  for (int i = 1; i < 6; ++i)
+    if (cost[i] < cost[best]) best = i;
+  switch (best) {
+    case 0: linear_run<4, 4, 1, 4, 1, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s); break;
+    case 1: linear_run<4, 4, 2, 1, 1, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s); break;
+    case 2: linear_run<4, 4, 4, 1, 1, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s); break;
+    case 3: linear_run<4, 2, 4, 1, 1, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s); break;
+    case 4: linear_run<2, 2, 4, 1, 1, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s); break;
+    default: linear_run<1, 1, 16, 1, 1, 4>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s); break;
+  }
   return hipGetLastError();
 }
 
 hipError_t dx_span_means_f32_launch(const float *x, const int32_t *spans, float *out, int B, int S, int O, int d,
                                     long ldx, long ldo, hipStream_t s) {
-  span_means_f32_kernel<<<(unsigned)(B * O), THREADS, 0, s>>>(x, spans, out, S, O, d, ldx, ldo);
+  span_means_f32_kernel<<<dim3((unsigned)(B * O), blocks(d, THREADS)), THREADS, 0, s>>>(x, spans, out, S, O, d, ldx,
+                                                                                      ldo);
   return hipGetLastError();
 }
 
@@ -627,8 +747,14 @@ hipError_t dx_gather_rows_f32_launch(const float *x, const int32_t *idx, float *
 hipError_t dx_routing_f32_launch(const float *options, const float *base, const int32_t *owner,
                                  const uint8_t *option_mask, float *summary, int B, int O, int NQ, int W,
                                  hipStream_t s) {
-  routing_f32_kernel<<<(unsigned)(B * NQ), THREADS, (size_t)O * sizeof(float), s>>>(options, base, owner, option_mask,
-                                                                                    summary, O, NQ, W);
+  // eight questions per workgroup where that still fills the chip and their weights fit 64 KB of LDS
+  const unsigned cols = blocks(W, THREADS);
+  if (O <= 2048 && (long)B * blocks(NQ, 8) * cols >= 128)
+    routing_f32_kernel<8><<<dim3(cols, blocks(NQ, 8), B), THREADS, (size_t)O * 8 * sizeof(float), s>>>(
+        options, base, owner, option_mask, summary, O, NQ, W);
+  else
+    routing_f32_kernel<1><<<dim3(cols, NQ, B), THREADS, (size_t)O * sizeof(float), s>>>(options, base, owner,
+                                                                                      option_mask, summary, O, NQ, W);
   return hipGetLastError();
 }
 

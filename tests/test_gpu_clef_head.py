@@ -165,8 +165,8 @@ def test_encoded_requests_through_head() -> None:
 
 @pytest.mark.parametrize("m,n,k,pad", [
     (1, 1, 1, 0), (3, 17, 31, 0), (16, 16, 64, 0), (17, 1000, 1029, 3),   # 16 x 16 tiles, k over 16 waves
-    (300, 1000, 96, 0), (513, 515, 100, 1),                              # 32 x 32 tiles, k over 4 waves
-    (4097, 769, 130, 4), (20000, 200, 36, 0),                            # 128 x 128 tiles
+    (200, 1030, 95, 1), (300, 1000, 96, 0), (513, 515, 100, 1),           # 32 x 32 and 64 x 32 tiles, k over 4 waves
+    (601, 2047, 70, 0), (20000, 200, 36, 0), (4097, 1025, 130, 4),        # 64 x 64 tiles, k over 2, 4 and 1 waves
 ])
 def test_linear_f32_tiles(m: int, n: int, k: int, pad: int) -> None:
     """Every tile shape at its edges, rows with and without 16-byte alignment, bias, GELU and accumulation, against
