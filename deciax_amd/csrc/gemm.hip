@@ -6,6 +6,10 @@
 // wave owns a BM/2 x 128 quadrant in 32x32x16 MFMA blocks with fp32
 // accumulators (a single wave saturates the matrix core with this shape).
 //
+// Two kernels: gemm_nt_kernel, described here (256 x 256 tiles, which large M takes, and the 128-row tiles of the
+// residual-norm epilogue), and gemm_ring_kernel further down (smaller tiles, for launches that 256 x 256 tiles would
+// leave short of workgroups). dispatch() chooses by the tiles' rounds over the chip.
+//
 // Two data paths (256-row tiles, and 128-row tiles with K <= 8192, take the second):
 //
 // Register-staged. Per thread and K tile: 16-byte chunks arrive through buffer loads
@@ -62,11 +66,9 @@ struct Int {
 };
 
 constexpr int BK = 64;
-// Column tile: 256, or 128 for the 64-row tiles that serve small M (plain epilogues only). Every output
-// element runs the same MFMA chain in the same k order in either shape, so its value does not depend on
-// the tile configuration, hence not on M.
-template <int BM>
-constexpr int tile_n() { return BM == 64 ? 128 : 256; }
+// Column tile of gemm_nt_kernel. Every output element runs the same MFMA chain in the same k order in every tile
+// shape of this file, so its value does not depend on the tile configuration, hence not on M.
+constexpr int BN_NT = 256;
 constexpr int THREADS = 256;
 
 enum { EPI_BF16 = 0, EPI_F32 = 1, EPI_GATED = 2, EPI_QKV = 3, EPI_NORM = 4 };
@@ -168,16 +170,13 @@ template <int BM, int EPI, bool DTL, bool EB = false>
 __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
 gemm_nt_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, void *__restrict__ C, int M, int N,
                int K, long lda, long ldb, long ldc, int act, int group_m, QkvEpilogue qe, NormEpilogue ne) {
-  constexpr int BN = tile_n<BM>();
+  constexpr int BN = BN_NT;
   constexpr int TM = BM / 64, TN = BN / 64;  // 32x32 blocks per wave along m, n
-  // the narrow tiles have too few MFMAs per k-step for the fixed-slot schedules: the compiler schedules them
-  constexpr bool SMALL = BM == 64;
-  static_assert(!SMALL || EPI == EPI_BF16 || EPI == EPI_F32, "narrow tiles take the plain epilogues only");
   constexpr int STAGE = (BM + BN) * BK;
   constexpr int AC = BM * BK / 8 / THREADS, BC = BN * BK / 8 / THREADS;  // 16-byte chunks per thread
   constexpr int NC = AC + BC;
   constexpr int RATIO = NC / AC;  // chunk j is an A chunk iff j % RATIO == 0
-  static_assert((SMALL || NC % 4 == 0) && NC % AC == 0, "chunk schedule");
+  static_assert(NC % 4 == 0 && NC % AC == 0, "chunk schedule");
   constexpr int OUT_W = EPI == EPI_GATED ? BN / 2 : BN;
   constexpr int OUT_PITCH = OUT_W + 8;
   // 256-row direct-to-LDS tiles use a ring of 3 A and 2 B stages (5 x 32 KB = the whole 160 KB)
@@ -284,9 +283,9 @@ gemm_nt_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, v
   constexpr int GS = NM / NG;                          // MFMAs between two loads
   constexpr int W0 = (NC + 2) / 3, W1 = (NC + 1) / 3;  // writes per pre-barrier k-step
   constexpr int R0 = BM == 256 ? 6 : NM / 4;          // first fragment-read slot
-  static_assert(SMALL || (GS >= 2 && W0 <= NM && R0 + NR <= NM), "region schedule");
+  static_assert(GS >= 2 && W0 <= NM && R0 + NR <= NM, "region schedule");
 #define DX_REGION(nw, ng)                                                                          \
-  if constexpr (!SMALL) do {                                                                       \
+  do {                                                                                             \
     _Pragma("unroll") for (int t = 0; t < NM; ++t) {                                               \
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                           \
       if (t < (nw)) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);                             \
@@ -409,9 +408,9 @@ gemm_nt_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, v
     // their stage and half (P0) in the next k-step, at evenly spaced MFMA slots.
     constexpr int P3 = NI / 2, P0 = NI - NI / 2, P1 = NI - P3 - P0;
     constexpr int DR0 = R0;
-    static_assert(P1 >= 0 && (SMALL || DR0 + NR <= NM), "load schedule");
+    static_assert(P1 >= 0 && DR0 + NR <= NM, "load schedule");
 #define DX_DREGION(nl)                                                                             \
-  if constexpr (!SMALL) do {                                                                       \
+  do {                                                                                             \
     _Pragma("unroll") for (int t = 0; t < NM; ++t) {                                               \
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                           \
       if ((t * (nl)) % NM < (nl)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);               \
@@ -705,15 +704,254 @@ gemm_nt_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, v
   }
 }
 
+// s_waitcnt operand: at most `vm` vector-memory operations outstanding, every LDS operation done.
+constexpr int wait_imm(int vm) { return (vm & 15) | (vm >> 4) << 14 | 7 << 4; }
+
+// Small and middle M: deep-ring tiles. (32 TM WM) x (32 TN WN) x 64 tiles of WM x WN waves, each wave TM x TN
+// blocks, over an NST-stage ring of direct-to-LDS tiles: NST - 1 tiles stay in flight, which is what a weight
+// streamed once from HBM needs (a two-stage tile waits out a memory round trip per 64 k). All fragments of the next
+// tile are read into a second register set while this tile's are multiplied, so there is one wait and one barrier
+// per tile. The output goes straight from registers (8- or 16-byte pieces of a row): at these sizes it is small.
+// Each output's MFMA chain is that of gemm_nt_kernel, so its value does not depend on which kernel ran.
+//
+// B rows of a tile, so that each wave holds what its epilogue combines:
+//   plain   BN consecutive weight rows;
+//   gated   per wave 16 TN gate rows, then their up rows (blocks j and j + TN / 2), out of the 64-row packing;
+//   q|k|v   q|k tiles: per wave 16 TN first halves of rotary pairs, then their partners; v tiles: as plain.
+template <int TM, int TN, int WM, int WN, int NST, int EPI>
+__global__ void __launch_bounds__(64 * WM * WN)
+gemm_ring_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, void *__restrict__ C, int M, int N,
+                 int K, long lda, long ldb, long ldc, int act, int group_m, QkvEpilogue qe) {
+  constexpr int W = WM * WN, BM = 32 * TM * WM, BN = 32 * TN * WN;
+  constexpr int STAGE = (BM + BN) * BK;             // elements
+  constexpr int AI = BM / 8 / W, BI = BN / 8 / W;   // 1 KB loads per wave and tile (8 rows each)
+  constexpr int NI = AI + BI;
+  constexpr bool PAIRED = EPI == EPI_GATED || EPI == EPI_QKV;
+  static_assert(BM % (8 * W) == 0 && BN % (8 * W) == 0 && (NST - 1) * NI <= 63, "load schedule");
+  static_assert(!PAIRED || TN % 2 == 0, "paired epilogues hold both columns of a pair in one wave");
+  static_assert(EPI != EPI_NORM, "no residual-norm epilogue here");
+  __shared__ __attribute__((aligned(1024))) uint16_t smem[NST * STAGE];
+
+  const int num_m = (M + BM - 1) / BM, num_n = N / BN;
+  int tm, tn;
+  tile_coords(blockIdx.x, gridDim.x, num_m, num_n, group_m, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int lrow = lane & 31, lhalf = lane >> 5;
+  const bool v_tile = EPI == EPI_QKV && n0 >= qe.qk_cols;
+
+  // weight row of the tile's LDS row r
+  auto weight_row = [&](int r) {
+    if (!PAIRED || v_tile) return n0 + r;
+    const int in = r % (32 * TN), second = in / (16 * TN);
+    const int u = n0 / 2 + r / (32 * TN) * (16 * TN) + in % (16 * TN);  // pair index
+    if constexpr (EPI == EPI_GATED) return u / 64 * 128 + u % 64 + second * 64;
+    else return u / (qe.d / 2) * qe.d + u % (qe.d / 2) + second * (qe.d / 2);
+  };
+  const int row0 = weight_row(0);
+  // load j of a wave fills LDS rows [8 i, 8 i + 8), i = wave AI + j: lane l takes row 8 i + l / 8, chunk slot l % 8
+  int aoff[AI], boff[BI];
+#pragma unroll
+  for (int j = 0; j < AI; ++j) {
+    const int row = 8 * (wave * AI + j) + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
+    aoff[j] = (int)(row * lda * 2) + c * 16;
+  }
+  int brows = 0;  // weight rows the tile spans
+#pragma unroll
+  for (int j = 0; j < BI; ++j) {
+    const int row = 8 * (wave * BI + j) + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
+    boff[j] = (int)((weight_row(row) - row0) * ldb * 2) + c * 16;
+  }
+  brows = weight_row(BN - 1) - row0 + 1;
+  const int abytes = (int)((long)min(M - m0, BM) * lda * 2);  // rows past M read as zeros
+  const int bbytes = (int)((long)brows * ldb * 2);
+  const int KT = K / BK;
+  auto issue = [&](int t, int stage) __attribute__((always_inline)) {
+    // past the last tile: empty resources, so the loads count but touch no memory
+    const __amdgpu_buffer_rsrc_t ra = make_rsrc(A + (long)m0 * lda, t < KT ? abytes : 0);
+    const __amdgpu_buffer_rsrc_t rb = make_rsrc(B + (long)row0 * ldb, t < KT ? bbytes : 0);
+    uint16_t *base = smem + stage * STAGE;
+#pragma unroll
+    for (int j = 0; j < AI; ++j) lds_load16(ra, base + (wave * AI + j) * 512, aoff[j], t * BK * 2);
+#pragma unroll
+    for (int j = 0; j < BI; ++j) lds_load16(rb, base + BM * BK + (wave * BI + j) * 512, boff[j], t * BK * 2);
+  };
+  floatx16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  bf16x8 fa0[4][TM], fb0[4][TN], fa1[4][TM], fb1[4][TN];
+  // LDS rows of a wave start at multiples of 32, so the swizzle depends on the lane's row alone
+  int fo[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) fo[ks] = swz(lrow, ks * 2 + lhalf);
+  auto read = [&](bf16x8 (&fa)[4][TM], bf16x8 (&fb)[4][TN], int stage) __attribute__((always_inline)) {
+    const uint16_t *sa = smem + stage * STAGE + wm * (32 * TM * BK), *sb = smem + stage * STAGE + BM * BK + wn * (32 * TN * BK);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+        fa[ks][i] = as_bf16x8(*reinterpret_cast<const u32x4 *>(sa + i * 32 * BK + fo[ks]));
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        fb[ks][j] = as_bf16x8(*reinterpret_cast<const u32x4 *>(sb + j * 32 * BK + fo[ks]));
+    }
+  };
+  auto mm = [&](const bf16x8 (&fa)[4][TM], const bf16x8 (&fb)[4][TN]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = mfma32(fb[ks][j], fa[ks][i], acc[i][j]);
+  };
+#pragma unroll
+  for (int t = 0; t < NST; ++t) issue(t, t);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 1) * NI) : "memory");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  read(fa0, fb0, 0);
+  int stage = 0;  // of tile kt
+  // Tile kt's fragments are in fa / fb (or arriving); tile kt + 1 has landed once the NST - 2 younger tiles are all
+  // that is in flight; after the barrier every wave has read tile kt, whose stage takes tile kt + NST.
+  auto iteration = [&](int kt, auto &fa, auto &fb, auto &ga, auto &gb) __attribute__((always_inline)) {
+    // (the builtin, not inline asm: the compiler then knows that the fragments are there and does not wait again,
+    // for the next tile's reads too, before the first MFMA)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(wait_imm((NST - 2) * NI));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    const int freed = stage;
+    stage = stage + 1 == NST ? 0 : stage + 1;
+    read(ga, gb, stage);
+    issue(kt + NST, freed);
+    mm(fa, fb);
+    // among the MFMAs: the next tile's fragment reads, two or more per MFMA, then the loads, evenly spaced
+    constexpr int NR = 4 * (TM + TN), NM = 4 * TM * TN, RPM = (NR + NM - 1) / NM + 1, RM = (NR + RPM - 1) / RPM;
+    constexpr int LM = NM > RM ? NM - RM : 1, LPM = (NI + LM - 1) / LM;
+#pragma unroll
+    for (int t = 0; t < NM; ++t) {
+      if (t < RM) __builtin_amdgcn_sched_group_barrier(0x100, RPM, 0);
+      else if ((t - RM + 1) * NI / LM > (t - RM) * NI / LM) __builtin_amdgcn_sched_group_barrier(0x020, LPM, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int kt = 0;
+  for (; kt + 1 < KT; kt += 2) {
+    iteration(kt, fa0, fb0, fa1, fb1);
+    iteration(kt + 1, fa1, fb1, fa0, fb0);
+  }
+  if (kt < KT) iteration(kt, fa0, fb0, fa1, fb1);
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+
+  // lane (lrow, lhalf) holds row i 32 + lrow, columns j 32 + 8 q + 4 lhalf + 0..3 of its wave's quadrant in acc[i][j]
+  // registers 4 q .. 4 q + 3
+  uint16_t *Cb = reinterpret_cast<uint16_t *>(C);
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int row = m0 + (wm * TM + i) * 32 + lrow;
+    if (row >= M) continue;
+    if constexpr (EPI == EPI_F32 || EPI == EPI_BF16) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const long at = (long)row * ldc + n0 + (wn * TN + j) * 32 + q * 8 + lhalf * 4;
+          if constexpr (EPI == EPI_F32) {
+            const floatx4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+            *reinterpret_cast<floatx4 *>(reinterpret_cast<float *>(C) + at) = v;
+          } else {
+            u32x2 w;
+            w[0] = pack_bf2(acc[i][j][4 * q], acc[i][j][4 * q + 1]);
+            w[1] = pack_bf2(acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+            *reinterpret_cast<u32x2 *>(Cb + at) = w;
+          }
+        }
+    } else if constexpr (EPI == EPI_GATED) {
+      auto gated = [&](auto silu_c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < TN / 2; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const floatx16 &ga = acc[i][j], &ua = acc[i][j + TN / 2];
+            u32x2 w;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const uint32_t g2 = pack_bf2(ga[4 * q + 2 * h], ga[4 * q + 2 * h + 1]);
+              const uint32_t u2 = pack_bf2(ua[4 * q + 2 * h], ua[4 * q + 2 * h + 1]);
+              const float g0 = lo_bf(g2), g1 = hi_bf(g2);
+              const float a0 = round_bf(decltype(silu_c)::value ? silu(g0) : gelu_tanh(g0));
+              const float a1 = round_bf(decltype(silu_c)::value ? silu(g1) : gelu_tanh(g1));
+              w[h] = pack_bf2(a0 * lo_bf(u2), a1 * hi_bf(u2));
+            }
+            const int col = n0 / 2 + wn * (16 * TN) + j * 32 + q * 8 + lhalf * 4;
+            *reinterpret_cast<u32x2 *>(Cb + (long)row * ldc + col) = w;
+          }
+      };
+      if (act == DX_ACT_SILU) gated(Flag<true>());
+      else gated(Flag<false>());
+    } else {
+      if (v_tile) {
+        uint16_t *vcol = qe.vt + qe.vt_col[row];
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int col = n0 - qe.qk_cols + (wn * TN + j) * 32 + (r >> 2) * 8 + lhalf * 4 + (r & 3);
+            vcol[(long)col * qe.vt_ld] = f2bf(acc[i][j][r]);
+          }
+      } else {
+        const int half = qe.d / 2;
+        const long p = min(max(qe.pos[row], 0), qe.max_pos - 1);
+#pragma unroll
+        for (int j = 0; j < TN / 2; ++j) {
+          const int u = n0 / 2 + wn * (16 * TN) + j * 32, head = u / half, h0 = u % half;  // 32 pairs of one head
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int jc = h0 + q * 8 + lhalf * 4;
+            const u32x2 cs = *reinterpret_cast<const u32x2 *>(qe.cos + p * half + jc);
+            const u32x2 sn = *reinterpret_cast<const u32x2 *>(qe.sin + p * half + jc);
+            u32x2 o1, o2;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const uint32_t a2 = pack_bf2(acc[i][j][4 * q + 2 * h], acc[i][j][4 * q + 2 * h + 1]);
+              const uint32_t b2 = pack_bf2(acc[i][j + TN / 2][4 * q + 2 * h], acc[i][j + TN / 2][4 * q + 2 * h + 1]);
+              const float av[2] = {lo_bf(a2), hi_bf(a2)}, bv[2] = {lo_bf(b2), hi_bf(b2)};
+              const float cv[2] = {lo_bf(cs[h]), hi_bf(cs[h])}, sv[2] = {lo_bf(sn[h]), hi_bf(sn[h])};
+              float r1[2], r2[2];
+#pragma unroll
+              for (int e = 0; e < 2; ++e) {
+                r1[e] = round_bf(av[e] * cv[e]) - round_bf(bv[e] * sv[e]);
+                r2[e] = round_bf(bv[e] * cv[e]) + round_bf(av[e] * sv[e]);
+              }
+              o1[h] = pack_bf2(r1[0], r1[1]);
+              o2[h] = pack_bf2(r2[0], r2[1]);
+            }
+            uint16_t *dst = Cb + (long)row * ldc + head * qe.d + jc;
+            *reinterpret_cast<u32x2 *>(dst) = o1;
+            *reinterpret_cast<u32x2 *>(dst + half) = o2;
+          }
+        }
+      }
+    }
+  }
+}
+
 template <int BM, int EPI>
 hipError_t launch(const uint16_t *A, const uint16_t *B, void *C, long M, long N, long K, long lda, long ldb,
                   long ldc, int act, const QkvEpilogue &qe, const NormEpilogue &ne, hipStream_t s) {
-  const long num_m = (M + BM - 1) / BM, num_n = N / tile_n<BM>();
+  const long num_m = (M + BM - 1) / BM, num_n = N / BN_NT;
   const bool weight_cached = N * K * 2 <= (256L << 20);  // the weight fits the 256 MB Infinity Cache
   // 256-row tiles always take the direct-to-LDS ring: its A stages give long-K shapes the latency slack
   // (against the register-staged path: down K 14336 +3-8 % alone and -0.8 % step time in the 9B
-  // forward, K 36864 +4.5 %, 1344- and 448-tile down shapes +2.5 % / +1 %). 128-row tiles (M <= 1024)
-  // have two stages only, so long K keeps the register-staged path and its two tiles of slack there.
+  // forward, K 36864 +4.5 %, 1344- and 448-tile down shapes +2.5 % / +1 %). 128-row tiles (the
+  // residual-norm epilogue up to 1024 rows) have two stages only, so long K keeps the register-staged path and its two tiles of slack there.
   auto kern = gemm_nt_kernel<BM, EPI, true>;
   if constexpr (BM != 256)
     if (K > 8192) kern = gemm_nt_kernel<BM, EPI, false>;
@@ -738,18 +976,81 @@ hipError_t launch(const uint16_t *A, const uint16_t *B, void *C, long M, long N,
   return hipGetLastError();
 }
 
+template <int TM, int TN, int WM, int WN, int NST, int EPI>
+hipError_t launch_ring(const uint16_t *A, const uint16_t *B, void *C, long M, long N, long K, long lda, long ldb,
+                       long ldc, int act, const QkvEpilogue &qe, hipStream_t s) {
+  const long num_m = (M + 32 * TM * WM - 1) / (32 * TM * WM), num_n = N / (32 * TN * WN);
+  // the row tiles of one weight column stand together (8 at most), so that they share it in one XCD's L2
+  gemm_ring_kernel<TM, TN, WM, WN, NST, EPI><<<dim3((unsigned)(num_m * num_n)), dim3(64 * WM * WN), 0, s>>>(
+      A, B, C, (int)M, (int)N, (int)K, lda, ldb, ldc, act, 8, qe);
+  return hipGetLastError();
+}
+
+// Tile choice. Below the power limit these GEMMs run at the rate tiles reach LDS from L2: about 50 GB/s per CU with
+// every CU loading (some 120 cache lines in flight per CU at 550 to 900 cycles, measured on tiles from 32 x 32 to
+// 256 x 256). So a launch takes its rounds of tiles over the 256 CUs times a tile's rows of A and B, BM + BN, and
+// the smallest tile that still fits one round wins. Past two rounds the tiles drift apart and half of the last
+// round overlaps. Over 54 shapes (N x K of the 9B projections, M from 8 to 3300) the choice is within 0.8% of the
+// best measured form on average. us before (64 x 128, 128 x 256 or 256 x 256 tiles) -> now:
+//   3584 x 14336:  M 64 156 -> 38   M 200 156 -> 52   M 517 182 -> 89    M 1300 232 -> 149   M 3300 276 (unchanged)
+//   28672 x 3584:  M 64  75 -> 40   M 200  75 -> 57   M 517 182 -> 128   M 1000 254 -> 162
+//   8192 x 3584:   M 64  47 -> 17   M 200  68 -> 24   M 517  66 -> 41    M 1000  64 -> 55
+struct TileForm {
+  int bm, bn;
+};
+double tile_cost(TileForm f, long M, long N) {
+  const long tiles = (M + f.bm - 1) / f.bm * (N / f.bn), up = (tiles + 255) / 256;
+  const double rounds = up <= 2 ? (double)up : fmax(tiles / 256.0, up - 0.5);
+  return rounds * (f.bm + f.bn) * (f.bm > f.bn ? 0.97 : 1.0);  // rows of A are the ones that stay in L2
+}
+
 template <int EPI>
 hipError_t dispatch(const uint16_t *A, const uint16_t *B, void *C, long M, long N, long K, long lda, long ldb,
                     long ldc, int act, hipStream_t s, const QkvEpilogue &qe = QkvEpilogue{},
                     const NormEpilogue &ne = NormEpilogue{}) {
-  // Small M: halve the row tile so more workgroups exist. For the plain epilogues, 64 x 128 tiles when the
-  // 128 x 256 ones would leave three quarters of the CUs idle (under 64 tiles: o and down of one 9B
-  // request of up to 512 tokens; its forward -12 to -16% at 128-512 tokens, unchanged from 768 on).
-  if constexpr (EPI == EPI_BF16 || EPI == EPI_F32)
-    if (M <= 1024 && (M + 127) / 128 * (N / tile_n<128>()) < 64)
-      return launch<64, EPI>(A, B, C, M, N, K, lda, ldb, ldc, act, qe, ne, s);
-  if (M <= 1024) return launch<128, EPI>(A, B, C, M, N, K, lda, ldb, ldc, act, qe, ne, s);
-  return launch<256, EPI>(A, B, C, M, N, K, lda, ldb, ldc, act, qe, ne, s);
+  if constexpr (EPI == EPI_NORM) {
+    if (M <= 1024) return launch<128, EPI>(A, B, C, M, N, K, lda, ldb, ldc, act, qe, ne, s);
+    return launch<256, EPI>(A, B, C, M, N, K, lda, ldb, ldc, act, qe, ne, s);
+  } else {
+    constexpr bool PAIRED = EPI == EPI_GATED || EPI == EPI_QKV;
+    // 256 x 256 first, then the ring forms of this epilogue (paired ones need an even TN, so they lack the
+    // narrowest); q|k|v tiles must not straddle the end of the q|k columns
+    static const TileForm forms[] = {{256, 256}, {256, 128}, {192, 128}, {128, 128}, {96, 128}, {64, 128},
+                                     {128, 64},  {64, 64},   {192, 64},  {96, 64},   {64, 32},  {32, PAIRED ? 64 : 32}};
+    int best = 0;
+    double least = tile_cost(forms[0], M, N);
+    for (int i = 1; i < 12; ++i) {
+      if (PAIRED && i >= 8 && i <= 10) continue;
+      if (EPI == EPI_QKV && qe.qk_cols % forms[i].bn) continue;
+      const double c = tile_cost(forms[i], M, N);
+      if (c < least) {
+        least = c;
+        best = i;
+      }
+    }
+#define DX_RING(...) return launch_ring<__VA_ARGS__, EPI>(A, B, C, M, N, K, lda, ldb, ldc, act, qe, s)
+    switch (best) {
+      case 1: DX_RING(4, 2, 2, 2, 3);
+      case 2: DX_RING(3, 2, 2, 2, 4);
+      case 3: DX_RING(2, 2, 2, 2, 4);
+      case 4: DX_RING(3, 2, 1, 2, 5);
+      case 5: DX_RING(1, 2, 2, 2, 6);
+      case 6: DX_RING(1, 2, 4, 1, 6);
+      case 7: DX_RING(1, 2, 2, 1, 5);
+    }
+    if constexpr (PAIRED) {
+      if (best == 11) DX_RING(1, 2, 1, 1, 5);
+    } else {
+      switch (best) {
+        case 8: DX_RING(3, 1, 2, 2, 5);
+        case 9: DX_RING(3, 1, 1, 2, 7);
+        case 10: DX_RING(1, 1, 2, 1, 6);
+        case 11: DX_RING(1, 1, 1, 1, 8);
+      }
+    }
+#undef DX_RING
+    return launch<256, EPI>(A, B, C, M, N, K, lda, ldb, ldc, act, qe, ne, s);
+  }
 }
 
 }  // namespace

@@ -909,3 +909,65 @@ def test_fused_residual_norm_forward_bit_identical() -> None:
         gemma.FUSED_NORM = default
     assert np.array_equal(out[True][0], out[False][0])
     assert np.array_equal(out[True][1], out[False][1])
+
+
+# Rows whose choice of GEMM tile covers every form at N = 3584 (32 x 32, 64 x 32, 64 x 64, 96 x 64, 128 x 64, 96 x 128,
+# 128 x 128, 192 x 128, 256 x 128 and 256 x 256 tiles; 192 x 64 and 64 x 128 at the widths below), one row either side
+# of a tile edge among them; K of one and of five 64-deep tiles, fewer than the ring's stages.
+FORM_ROWS = (1, 32, 33, 65, 100, 129, 200, 300, 400, 513, 600, 769, 1000, 1300, 1537, 2100, 3300)
+
+
+@pytest.mark.parametrize("k", [64, 320, 1088])
+def test_gemm_tile_forms_agree(k: int) -> None:
+    """Every tile form gives each row bit for bit what the 256 x 256 form gives it: plain bf16 and fp32, gated with
+    both activations, at row strides wider than the row."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    say(f"GEMM tile forms, K={k}")
+    r = rng(k)
+    big = 8192
+    a = to_dev(bf16_np(r.normal(size=(big, k + 8)).astype(np.float32)))[:, :k]
+    for n in (3584, 4608, 1280):
+        w = to_dev(bf16_np(r.normal(size=(n, k)).astype(np.float32) * 0.1))
+        want = {dt: K.linear(a, w, out_dtype=dt) for dt in (torch.bfloat16, torch.float32)}
+        gated = {act: K.gated_linear(a, w, act) for act in ("gelu_tanh", "silu")}
+        for m in FORM_ROWS:
+            for dt, y in want.items():
+                got = torch.full((m + 1, n + 8), float("nan"), dtype=dt, device=a.device)
+                K.linear(a[:m], w, out=got[:m, :n], out_dtype=dt)
+                assert torch.equal(got[:m, :n], y[:m]), f"M={m} N={n} K={k} {dt}"
+                assert torch.isnan(got[m]).all() and torch.isnan(got[:, n:]).all(), f"M={m} N={n}: wrote outside"
+            for act, y in gated.items():
+                assert torch.equal(K.gated_linear(a[:m], w, act), y[:m]), f"gated M={m} N={n} K={k} {act}"
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(16, 8, 256), (32, 16, 128), (2, 1, 64), (6, 3, 64)])
+def test_qkv_rope_tile_forms_agree(hq: int, hkv: int, d: int) -> None:
+    """Every tile form of the q|k|v projection equals linear -> rope -> transpose_v bit for bit (head counts whose
+    q|k columns are not a multiple of 128 included)."""
+    import torch
+
+    from deciax_amd import gemma
+    from deciax_amd import kernels as K
+
+    hidden, width, qk_w = 192, (hq + 2 * hkv) * d, (hq + hkv) * d
+    r = rng(hq + d)
+    w = to_dev(bf16_np(r.normal(size=(width, hidden)) * 0.1))
+    cos_b, sin_b = gemma.rope_tables(4096, d, 10000.0)
+    cos, sin = gemma._bits_to_tensor(cos_b, w.device), gemma._bits_to_tensor(sin_b, w.device)
+    for rows in FORM_ROWS:
+        say(f"qkv_rope forms hq={hq} hkv={hkv} d={d} rows={rows}")
+        lengths = [rows] if rows < 60 else [rows - 45, 45]
+        batch = gemma.pack_batch([r.integers(0, 100, n).tolist() for n in lengths], [[] for _ in lengths])
+        x = to_dev(bf16_np(r.normal(size=(rows, hidden))))
+        ref = K.rope(K.linear(x, w), batch.positions, cos, sin, num_heads=hq + hkv, head_dim=d)
+        vt_ref = torch.zeros((hkv * d, batch.vt_ld), dtype=torch.bfloat16, device=x.device)
+        K.transpose_v(ref[:, qk_w:], vt_ref, batch.seq_start, batch.seq_len, batch.vt_start, batch.max_len,
+                      num_kv_heads=hkv, head_dim=d)
+        qk = torch.zeros((rows, width), dtype=torch.bfloat16, device=x.device)
+        vt = torch.zeros_like(vt_ref)
+        K.qkv_rope(x, w, qk, vt, batch.positions, batch.vt_col, cos, sin, num_q_heads=hq, num_kv_heads=hkv, head_dim=d)
+        assert torch.equal(qk[:, :qk_w].view(torch.int16), ref[:, :qk_w].contiguous().view(torch.int16)), rows
+        assert not qk[:, qk_w:].any() and torch.equal(vt.view(torch.int16), vt_ref.view(torch.int16)), rows
