@@ -56,7 +56,9 @@ constexpr int SHORT_SEQ = 3072;
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float NEG_BIG = -1e30f;  // the reference's MASK_FILL (reference.py:8)
 
-enum { MODE_FIXED = 0, MODE_ONLINE = 1 };
+// MODE_CAP: running max with a soft-cap (those beyond the fixed shift). A mode of its own: the sixteen tanhf of a
+// block would otherwise sit in the loop of every launch without one.
+enum { MODE_FIXED = 0, MODE_ONLINE = 1, MODE_CAP = 2 };
 
 DX_DEVICE bool visible(int qi, int key, int len, int window, int causal) {
   if (key >= len) return false;
@@ -267,6 +269,8 @@ attn_bf16_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
 
   const float c2inv = 1.f / (-2.f * LOG2E * softcap);
   const float c3 = 0.5f * LOG2E * softcap;
+  // running-max form: scores (soft-capped ones carry the scale already) to log2 units
+  const float to_log2 = MODE == MODE_CAP ? LOG2E : scale * LOG2E;
 
   // Which 32-key blocks this wave's rows see: active = some key visible, masked = some key hidden.
   auto block_state = [&](const int kbase, bool &need_mask) {
@@ -290,6 +294,20 @@ attn_bf16_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
     vhi = window > 0 ? min(qi + window, len - 1) : len - 1;
     vlo = window > 0 ? qi - window : 0;
   }
+
+  // Running-max form: the row's maximum (its 32-key halves sit in lanes l and l ^ 32) joins mrun, and O follows.
+  auto raise_max = [&](const float tmax) __attribute__((always_inline)) {
+    const float mnew = fmaxf(mrun, fmaxf(tmax, __shfl_xor(tmax, 32, 64)));
+    if (__builtin_amdgcn_ballot_w64(mnew != mrun)) {
+      const float alpha = fast_exp2(mrun - mnew);
+      mrun = mnew;
+      lsum *= alpha;
+#pragma unroll
+      for (int i = 0; i < NDB; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
+    }
+  };
 
   // One 32-key block kb of the tile in stage sk (K, then V^T at sk + KST): S^T = K Q^T, softmax,
   // O^T += V^T P^T. MASKED evaluates the causal / window / length mask and skips blocks no row sees.
@@ -332,28 +350,21 @@ attn_bf16_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
         lsum += p;
       }
     } else {
-      float tmax = NEG_BIG;
+      if constexpr (MODE == MODE_CAP) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        float t = s[r] * scale;
-        if (softcap > 0.f) t = softcap * tanhf(t / softcap);
-        t *= LOG2E;
-        if constexpr (M) t = keep(r) ? t : NEG_BIG;
-        s[r] = t;
-        tmax = fmaxf(tmax, t);
+        for (int r = 0; r < 16; ++r) s[r] = softcap * tanhf(s[r] * scale / softcap);
       }
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-      const float mnew = fmaxf(mrun, tmax);
-      const float alpha = fast_exp2(mrun - mnew);
-      mrun = mnew;
-      lsum *= alpha;
-#pragma unroll
-      for (int i = 0; i < NDB; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
+      float smax = NEG_BIG;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        float p = fast_exp2(s[r] - mnew);
+        if constexpr (M) smax = keep(r) ? fmaxf(smax, s[r]) : smax;
+        else smax = fmaxf(smax, s[r]);
+      }
+      const float tmax = fmaxf(smax * to_log2, NEG_BIG);
+      raise_max(tmax);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        float p = fast_exp2(__builtin_fmaf(s[r], to_log2, -mrun));
         if constexpr (M) p = keep(r) ? p : 0.f;
         s[r] = p;
         lsum += p;
@@ -379,13 +390,65 @@ attn_bf16_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
     stream_sched<2 * NDB>();
   };
 
+  // Both blocks of a 64-key tile without masked keys, running-max form: one maximum and one pass over O for the
+  // tile. The softmax's vector instructions bound this form, and that pass was a third of them (head_dim 128).
+  auto tile64 = [&](const uint16_t *sk) __attribute__((always_inline)) {
+    floatx16 s[2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[kb][r] = 0.f;
+      const int krow = kb * 32 + kperm(lrow);
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) {
+        const int lo = ((ks * 2 + lhalf) ^ k_swz<D>(krow)) << 3;
+        s[kb] = mfma32(as_bf16x8(*reinterpret_cast<const u32x4 *>(sk + krow * D + lo)), qf[ks], s[kb]);
+      }
+    }
+    stream_sched<2 * NKS>();
+    float smax = NEG_BIG;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) smax = fmaxf(smax, s[kb][r]);
+    raise_max(fmaxf(smax * to_log2, NEG_BIG));
+    bf16x8 pf[4];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        s[kb][r] = fast_exp2(__builtin_fmaf(s[kb][r], to_log2, -mrun));
+        lsum += s[kb][r];
+      }
+#pragma unroll
+      for (int h2 = 0; h2 < 2; ++h2) {
+        u32x4 w;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] = pack_bf2(s[kb][8 * h2 + 2 * i], s[kb][8 * h2 + 2 * i + 1]);
+        pf[2 * kb + h2] = as_bf16x8(w);
+      }
+    }
+    const uint16_t *sv = sk + KST;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int h2 = 0; h2 < 4; ++h2)
+        o[db] = mfma32(as_bf16x8(*reinterpret_cast<const u32x4 *>(sv + vt_off<TK>(db * 32 + lrow, 2 * h2 + lhalf))),
+                       pf[h2], o[db]);
+    stream_sched<4 * NDB>();
+  };
+
   // Ring of NSTAGE tiles: tile kt sits in stage (kt - kt0) % NSTAGE, and tile kt + NSTAGE - 1 is
   // fetched while tile kt is multiplied (clamped: the last tiles reload themselves harmlessly).
   auto tile = [&](const int kt, auto masked) {
     issue(min(kt + NSTAGE - 1, kt1 - 1), (kt - kt0 + NSTAGE - 1) % NSTAGE);
     const uint16_t *sk = smem + ((kt - kt0) % NSTAGE) * STAGE;
+    if constexpr (MODE == MODE_ONLINE && TK == 64 && !decltype(masked)::value) {
+      tile64(sk);
+    } else {
 #pragma unroll
-    for (int kb = 0; kb < TK / 32; ++kb) block(sk, kt * TK + kb * 32, kb, masked);
+      for (int kb = 0; kb < TK / 32; ++kb) block(sk, kt * TK + kb * 32, kb, masked);
+    }
     // tile kt + 1 has landed in every wave's share (the NSTAGE - 2 younger tiles may stay in flight)
     // and every wave is done reading tile kt, whose stage the next iteration refills. A plain s_barrier:
     // __syncthreads would also wait for the younger tiles' loads (its fence waits for all LDS writes).
@@ -868,16 +931,20 @@ vt_zero_tails_kernel(uint16_t *__restrict__ Vt, const int32_t *__restrict__ seq_
   if (row < vt_rows && j < ((len + 63) & ~63)) Vt[(long)row * vt_ld + vt_start[blockIdx.x] + j] = 0;
 }
 
+inline bool fixed_shift(const AttnArgs &a) { return a.softcap > 0.f && a.softcap <= 56.f; }
+
 template <int D, int G, int W, int NS>
 hipError_t launch_bf16_dgw(const AttnArgs &a, hipStream_t s) {
   constexpr int BQ = 32 * (W / G);
   const unsigned ntiles = (a.max_seq_len + BQ - 1) / BQ;
   const dim3 grid = a.max_seq_len <= SHORT_SEQ ? dim3(a.hkv, a.num_seqs, ntiles) : dim3(ntiles, a.hkv, a.num_seqs);
-  const bool fixed = a.softcap > 0.f && a.softcap <= 56.f;
-  auto kern = a.key_bits ? (fixed ? attn_bf16_kernel<D, G, MODE_FIXED, true, W, NS>
-                                  : attn_bf16_kernel<D, G, MODE_ONLINE, true, W, NS>)
-                         : (fixed ? attn_bf16_kernel<D, G, MODE_FIXED, false, W, NS>
-                                  : attn_bf16_kernel<D, G, MODE_ONLINE, false, W, NS>);
+  auto kern = a.key_bits ? (fixed_shift(a) ? attn_bf16_kernel<D, G, MODE_FIXED, true, W, NS>
+                                           : attn_bf16_kernel<D, G, MODE_ONLINE, true, W, NS>)
+                         : (fixed_shift(a) ? attn_bf16_kernel<D, G, MODE_FIXED, false, W, NS>
+                                           : attn_bf16_kernel<D, G, MODE_ONLINE, false, W, NS>);
+  if constexpr (W == 8)
+    if (a.softcap > 0.f && !fixed_shift(a))
+      kern = a.key_bits ? attn_bf16_kernel<D, G, MODE_CAP, true, W, NS> : attn_bf16_kernel<D, G, MODE_CAP, false, W, NS>;
   kern<<<grid, dim3(64 * W), 0, s>>>(
       static_cast<const uint16_t *>(a.q), static_cast<const uint16_t *>(a.k), static_cast<const uint16_t *>(a.v),
       static_cast<uint16_t *>(a.out), a.seq_start, a.seq_len, a.vt_start, a.vt_seq_stride, a.max_seq_len,
@@ -896,6 +963,7 @@ inline long mean_key_span(const AttnArgs &a) {
 
 template <int D, int G>
 hipError_t launch_bf16_dg(const AttnArgs &a, hipStream_t s) {
+  if (a.softcap > 0.f && !fixed_shift(a)) return launch_bf16_dgw<D, G, 8, 4>(a, s);  // the one form built with MODE_CAP
   if constexpr (D == 128)
     if (mean_key_span(a) <= 2048) return launch_bf16_dgw<D, G, 4, 2>(a, s);
   return launch_bf16_dgw<D, G, 8, 4>(a, s);
