@@ -181,8 +181,7 @@ int attn_prefill(const void *q, const void *k, const void *v, const uint8_t *key
   const int64_t vec = dtype == DX_BF16 ? 8 : 4;
   REQUIRE(v_row_stride % vec == 0 && v_row_stride >= (int64_t)num_kv_heads * head_dim,
           "attention: bad v row stride %ld", (long)v_row_stride);
-  // the matrix-core fp32 kernel (head_dim 64 and 128) reads a 32-key block of K or V through a buffer
-  // resource with 32-bit byte offsets; the head_dim 256 kernel addresses with 64-bit pointers
+  // row strides whose 32-key block would not fit 32-bit byte offsets: never taken at head_dim 64 and 128
   if (dtype == DX_F32)
     SUPPORTED(head_dim > 128 || (k_row_stride < (INT64_C(1) << 24) && v_row_stride < (INT64_C(1) << 24)),
               "attention: fp32 k / v row strides of 2^24 elements or more are not supported at head_dim %d",

@@ -1,5 +1,4 @@
-// Causal GQA prefill attention for gfx950: a bf16 MFMA path, an fp32 MFMA path (head_dim <= 128) and
-// an fp32 VALU path (head_dim 256).
+// Causal GQA prefill attention for gfx950: a bf16 MFMA path and an fp32 MFMA path.
 //
 // Algorithm (the reference's blocked causal GQA attention,
 // src/deciax/kernels/attention/blocked.py:9-32, in the online form of its TPU
@@ -40,7 +39,7 @@
 
 namespace {
 
-constexpr int THREADS = 256;        // fp32 path and the V^T transpose
+constexpr int THREADS = 256;        // the V^T transpose and the mask words
 constexpr int BKV = 64;     // V^T block alignment of dx_transpose_v
 // bf16 path: waves per workgroup and LDS ring depth. The long form, 8 waves (two per SIMD, 32 query rows
 // each) over a 4-stage ring (128 KB), runs one workgroup per CU. The short form, 4 waves over a 2-stage
@@ -553,154 +552,51 @@ attn_bf16_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
   }
 }
 
-// fp32 path: VALU flash attention, TPQ threads per query row.
-template <int D, int TPQ>
-__global__ void __launch_bounds__(THREADS)
+// fp32 path, on the matrix core: v_mfma_f32_16x16x4_f32 (fp32 products and sums). A workgroup takes
+// 16 QB query rows of one head; its WAVES waves take blocks of 16 SUB keys in turn, each with its own running max,
+// row sum and O, merged through LDS at the end, so no barrier runs in the key loop. Operands go from global memory
+// straight to MFMA lanes (the query tile, which every wave reads, through LDS). With r = lane % 16, g = lane / 16:
+//   S^T = K Q^T    the four contraction indices of MFMA 4 c + e are dims 16 c + 4 g + e, so a lane reads 16 bytes
+//                  of key row r per chunk c and a load covers 64 bytes of 16 rows. It gets back query r, keys
+//                  4 g + 0..3. D / 32 partial sums per score: no MFMA waits for the one before, and 32 roundings
+//                  in a row instead of D (error against 64 bits 1.9e-7, one chain 4.3e-7).
+//   O^T += V^T P^T MFMA t contracts keys 4 g + t, whose probabilities the lane holds; output block 4 a + e is dims
+//                  64 a + 4 r + e, so a load covers 256 bytes of 4 rows, and the lane ends up with the 16
+//                  consecutive dims 64 a + 16 g + .. of query r.
+// K of the next block is requested when this block's scores are done, V at the start of its block: each has half a
+// block of MFMAs to land. What bounds it: the MFMAs and, at QB = 1 and head_dim 256, the 32 bytes per cycle and CU
+// that K and V take from L2 (QB = 2 halves them).
+// Measured, before (VALU kernel at head_dim 256, LDS-staged 32x32x2 MFMAs below it; us) -> now:
+//   head_dim 256: 2 x 701, 8/4 heads, soft-capped 575 -> 82    4 x 1024, 32/8 heads 7890 -> 948 (73 TFLOP/s)
+//   head_dim 128: 2 x 701, soft-capped 75 -> 43                4 x 1024, 32/8 heads 901 -> 454
+//   head_dim 64:  2 x 701, soft-capped 45 -> 36                4 x 1024, 32/8 heads 550 -> 223
+// with soft-capping the error at head_dim 64 and 128 fell from 2.0e-6 to 1.9e-7 (tanhf for the rcp / exp2 form).
+DX_DEVICE floatx4 mfma16_f32(float a, float b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+template <int D, int QB, int WAVES, int SUB>
+__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(1, 1)))
 attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V,
-                float *__restrict__ O, const int32_t *__restrict__ seq_start, const int32_t *__restrict__ seq_len,
-                int max_seq_len, int hq, int hkv, long q_stride, long k_stride, long v_stride, long o_stride,
-                float scale, float softcap, int window, int causal, const uint8_t *__restrict__ key_mask) {
-  constexpr int QPB = THREADS / TPQ;
-  constexpr int DPT = D / TPQ;
-  constexpr int TK = 32;
-  __shared__ __attribute__((aligned(16))) float ks[TK * D];
-  __shared__ __attribute__((aligned(16))) float vs[TK * D];
+                    float *__restrict__ O, const int32_t *__restrict__ seq_start, const int32_t *__restrict__ seq_len,
+                    int max_seq_len, int hq, int hkv, long q_stride, long k_stride, long v_stride, long o_stride,
+                    float scale, float softcap, int window, int causal, const uint8_t *__restrict__ key_mask) {
+  constexpr int C = D / 16, A = D / 64, KB = 16 * SUB, BQ = 16 * QB, OP = D + 4;
+  constexpr int NC = D / 32;  // partial sums per score
+  static_assert(D % 64 == 0 && KB <= 64, "tile shape");
+  __shared__ __attribute__((aligned(16))) float os[WAVES * BQ * OP];
+  __shared__ float ms[WAVES][BQ], ls[WAVES][BQ];
 
-  const int b = blockIdx.y, h = blockIdx.z, g = h / (hq / hkv);
+  const int b = blockIdx.y, h = blockIdx.x % hq, g_kv = h / (hq / hkv);
   const int len = min(max(seq_len[b], 0), max_seq_len);
-  const int ntiles = (max_seq_len + QPB - 1) / QPB;
-  const int q0 = (ntiles - 1 - (int)blockIdx.x) * QPB;
-  if (q0 >= len) return;
-  const long start = seq_start[b];
-  const int tid = threadIdx.x, part = tid % TPQ;
-  const int qi = q0 + tid / TPQ;
-
-  float q[DPT], o[DPT];
-  {
-    const float *qp = Q + (start + min(qi, len - 1)) * q_stride + (long)h * D + part * DPT;
-#pragma unroll
-    for (int d = 0; d < DPT; ++d) {
-      q[d] = qp[d];
-      o[d] = 0.f;
-    }
-  }
-  const int qlast = min(q0 + QPB, len) - 1;
-  int klo, khi;
-  if (causal) {
-    khi = qlast + 1;
-    klo = window > 0 ? max(0, q0 - window + 1) : 0;
-  } else {
-    khi = window > 0 ? min(len, qlast + window + 1) : len;
-    klo = window > 0 ? max(0, q0 - window) : 0;
-  }
-  float m = NEG_BIG, l = 0.f;
-  for (int k0 = (klo / TK) * TK; k0 < khi; k0 += TK) {
-    __syncthreads();
-    for (int idx = tid; idx < TK * D / 4; idx += THREADS) {
-      const int row = idx / (D / 4), c = idx % (D / 4);
-      const long key = start + min(k0 + row, len - 1);
-      reinterpret_cast<float4 *>(ks)[idx] = *reinterpret_cast<const float4 *>(K + key * k_stride + (long)g * D + c * 4);
-      reinterpret_cast<float4 *>(vs)[idx] = *reinterpret_cast<const float4 *>(V + key * v_stride + (long)g * D + c * 4);
-    }
-    __syncthreads();
-    float sc[TK];
-    uint32_t vis = 0;
-    float tmax = NEG_BIG;
-#pragma unroll
-    for (int j = 0; j < TK; ++j) {
-      float s = 0.f;
-#pragma unroll
-      for (int d = 0; d < DPT; ++d) s = fmaf(q[d], ks[j * D + part * DPT + d], s);
-#pragma unroll
-      for (int off = 1; off < TPQ; off <<= 1) s += __shfl_xor(s, off, 64);
-      s *= scale;
-      if (softcap > 0.f) s = softcap * tanhf(s / softcap);
-      // key_mask (nullable) hides keys of row start + key; read only for keys inside the sequence
-      const bool v = visible(qi, k0 + j, len, window, causal) && (!key_mask || key_mask[start + k0 + j]);
-      vis |= (uint32_t)v << j;
-      sc[j] = s;
-      if (v) tmax = fmaxf(tmax, s);
-    }
-    const float mnew = fmaxf(m, tmax);
-    const float alpha = expf(m - mnew);
-    l *= alpha;
-#pragma unroll
-    for (int d = 0; d < DPT; ++d) o[d] *= alpha;
-#pragma unroll
-    for (int j = 0; j < TK; ++j) {
-      const float p = ((vis >> j) & 1u) ? expf(sc[j] - mnew) : 0.f;
-      l += p;
-#pragma unroll
-      for (int d = 0; d < DPT; ++d) o[d] = fmaf(p, vs[j * D + part * DPT + d], o[d]);
-    }
-    m = mnew;
-  }
-  if (qi < len) {
-    float *op = O + (start + qi) * o_stride + (long)h * D + part * DPT;
-#pragma unroll
-    for (int d = 0; d < DPT; ++d) op[d] = l > 0.f ? o[d] / l : 0.f;  // a row that sees no key: zeros
-  }
-}
-
-// fp32 path on the matrix core, head_dim <= 128: v_mfma_f32_32x32x2_f32 (fp32 products and sums).
-// A workgroup takes 32 query rows of one head. Its F_WAVES waves split the 32-key blocks (wave w takes
-// blocks w, w + F_WAVES, ...), each staging its block in an LDS region of its own, and merge their
-// online-softmax states (running max, row sum, O) at the end, so no barrier runs inside the key loop.
-//   S^T = K Q^T: D / 2 MFMAs, MFMA j contracting head dims j (lanes 0-31) and D / 2 + j (lanes
-//   32-63). Lane l then holds query l % 32 and keys (r / 4) 8 + (l / 32) 4 + r % 4 of the block.
-//   O^T += V^T P^T: MFMA step i contracts the two keys the lane halves hold in register i, so each lane
-//   feeds its own probabilities as the B operand and reads V[key][d] for its half's key.
-// The next block's K and V are requested from global memory into registers at the start of this block
-// and go to LDS once the region's previous reads are done (K after this block's PV, V at the start of the
-// next block; LDS operations of one wave complete in order), so each load has a whole block to land.
-constexpr int F_WAVES = 4;
-
-DX_DEVICE floatx16 mfma32_f32(float a, float b, floatx16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
-template <int D>
-__global__ void __launch_bounds__(64 * F_WAVES) __attribute__((amdgpu_waves_per_eu(1, 1)))
-attn_f32_mfma_kernel(const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V,
-                     float *__restrict__ O, const int32_t *__restrict__ seq_start, const int32_t *__restrict__ seq_len,
-                     int max_seq_len, int hq, int hkv, long q_stride, long k_stride, long v_stride, long o_stride,
-                     float scale, float softcap, int window, int causal, const uint8_t *__restrict__ key_mask) {
-  static_assert(D == 64 || D == 128, "fp32 matrix-core attention covers head_dim 64 and 128");
-  constexpr int KP = D + 4;    // K row pitch (floats): 16 lanes reading 16 bytes of 16 rows cover all 64 banks
-  constexpr int VP = D + 8;    // V row pitch: the lane halves read rows 4 apart, on disjoint banks
-  constexpr int REGION = 32 * KP + 32 * VP;  // floats per wave
-  constexpr int DH = D / 2;
-  constexpr int NDB = D / 32;
-  constexpr int LPL = 32 * (D / 4) / 64;     // 16-byte chunks of a 32 x D block per lane
-  constexpr int OP = 33;                     // merge: O^T [D][32] at pitch 33, then m [32] and l [32]
-  static_assert(D * OP + 64 <= REGION, "merge state fits the wave's region");
-  __shared__ __attribute__((aligned(16))) float smem[F_WAVES * REGION];
-
-  const int b = blockIdx.y, h = blockIdx.z, g = h / (hq / hkv);
-  const int len = min(max(seq_len[b], 0), max_seq_len);
-  const int ntiles = (max_seq_len + 31) / 32;
-  const int q0 = (ntiles - 1 - (int)blockIdx.x) * 32;  // heaviest (last) query tiles first
+  const int ntiles = (max_seq_len + BQ - 1) / BQ;
+  const int q0 = (ntiles - 1 - (int)blockIdx.x / hq) * BQ;  // heaviest (last) query tiles first
   if (q0 >= len) return;
   const long start = seq_start[b];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lrow = lane & 31, hh = lane >> 5;
-  const int qi = q0 + lrow;
-  float *const ks = smem + wave * REGION;
-  float *const vs = ks + 32 * KP;
+  const int r = lane & 15, g = lane >> 4;
 
-  float qf[DH];
-  {
-    const float *qp = Q + (start + min(qi, len - 1)) * q_stride + (long)h * D + hh * DH;
-#pragma unroll
-    for (int j = 0; j < DH; j += 4) {
-      const float4 v = *reinterpret_cast<const float4 *>(qp + j);
-      qf[j] = v.x;
-      qf[j + 1] = v.y;
-      qf[j + 2] = v.z;
-      qf[j + 3] = v.w;
-    }
-  }
-  const int qlast = min(q0 + 31, len - 1);
+  const int qlast = min(q0 + BQ, len) - 1;
   int klo, khi;
   if (causal) {
     khi = qlast + 1;
@@ -709,168 +605,176 @@ attn_f32_mfma_kernel(const float *__restrict__ Q, const float *__restrict__ K, c
     khi = window > 0 ? min(len, qlast + window + 1) : len;
     klo = window > 0 ? max(0, q0 - window) : 0;
   }
-  const int kb0 = klo / 32, kb1 = (khi + 31) / 32;
+  const float *const kp = K + start * k_stride + (long)g_kv * D + 4 * g;
+  const float *const vp = V + start * v_stride + (long)g_kv * D + 4 * r;
 
-  // chunk c = lane + 64 t of a block: key row c / (D / 4) = t RPT + lane / (D / 4), columns
-  // 4 (lane % (D / 4)) .. + 3. Each block's K and V rows come through buffer resources based at the
-  // block's first key, so the per-lane offsets are loop-invariant and rows past the sequence read zeros
-  // (their scores are masked).
-  constexpr int RPT = 64 / (D / 4);  // key rows per chunk step t
-  const int crow = lane / (D / 4), ccol = (lane % (D / 4)) * 4;
-  const int koff = (int)((crow * k_stride + ccol) * 4), voff = (int)((crow * v_stride + ccol) * 4);
-  const float *const kseq = K + start * k_stride + (long)g * D;
-  const float *const vseq = V + start * v_stride + (long)g * D;
-  float4 kr[LPL], vr[LPL];
-  auto rsrc = [&](const float *base, long stride, int kb) {
-    // the block's rows only (32-bit byte counts); wave-uniform, which the compiler is told so that the
-    // descriptor stays in scalar registers (a vector one costs a waterfall loop around every load)
-    const long rows = __builtin_amdgcn_readfirstlane(min(max(len - kb * 32, 0), 32));
-    return __builtin_amdgcn_make_buffer_rsrc((void *)(base + (long)kb * 32 * stride), (short)0,
-                                             (int)(rows * stride * 4), 0x00020000);
-  };
-  auto fetch_k = [&](int kb) {
-    const __amdgpu_buffer_rsrc_t r = rsrc(kseq, k_stride, kb);
-#pragma unroll
-    for (int t = 0; t < LPL; ++t)
-      kr[t] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, koff, (int)(t * RPT * k_stride * 4), 0));
-  };
-  auto fetch_v = [&](int kb) {
-    const __amdgpu_buffer_rsrc_t r = rsrc(vseq, v_stride, kb);
-#pragma unroll
-    for (int t = 0; t < LPL; ++t)
-      vr[t] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, (int)(t * RPT * v_stride * 4), 0));
-  };
-  auto put_k = [&]() {
-#pragma unroll
-    for (int t = 0; t < LPL; ++t) *reinterpret_cast<float4 *>(ks + (t * RPT + crow) * KP + ccol) = kr[t];
-  };
-  auto put_v = [&]() {
-#pragma unroll
-    for (int t = 0; t < LPL; ++t) *reinterpret_cast<float4 *>(vs + (t * RPT + crow) * VP + ccol) = vr[t];
-  };
-
-  floatx16 o[NDB];
-#pragma unroll
-  for (int i = 0; i < NDB; ++i)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
-  float m = NEG_BIG, l = 0.f;  // running max (log2 units) and this lane's share of the row sum
-  const float cap2 = softcap > 0.f ? 2.f * LOG2E / softcap : 0.f;
-
-  int kb = kb0 + wave;
-  if (kb < kb1) {
-    fetch_k(kb);
-    put_k();
-    fetch_v(kb);
-  }
-  for (; kb < kb1; kb += F_WAVES) {
-    put_v();
-    const int nb = kb + F_WAVES;
-    const bool more = nb < kb1;
-    if (more) {  // the next block's K and V load during this whole block
-      fetch_k(nb);
-      fetch_v(nb);
-    }
-    floatx16 s;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = 0.f;
-    {
-      // every K fragment of the block is requested before the first MFMA: one LDS round trip per block
-      // instead of one per four MFMAs of the dependent chain
-      const float *kp = ks + lrow * KP + hh * DH;
-      float4 kv[DH / 4];
-#pragma unroll
-      for (int j = 0; j < DH / 4; ++j) kv[j] = *reinterpret_cast<const float4 *>(kp + 4 * j);
-      __builtin_amdgcn_sched_barrier(0);  // the scheduler would otherwise sink each read to its MFMAs
-#pragma unroll
-      for (int j = 0; j < DH / 4; ++j) {
-        s = mfma32_f32(kv[j].x, qf[4 * j], s);
-        s = mfma32_f32(kv[j].y, qf[4 * j + 1], s);
-        s = mfma32_f32(kv[j].z, qf[4 * j + 2], s);
-        s = mfma32_f32(kv[j].w, qf[4 * j + 3], s);
-      }
-    }
-    // score r is key kb 32 + (r / 4) 8 + 4 hh + r % 4 of query qi. The softcap and key-mask tests are
-    // taken once per block, outside the per-score loops.
-    const int kbase = kb * 32 + 4 * hh;
-    if (softcap > 0.f) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        float x = s[r] * scale;
-        x = softcap - 2.f * softcap * fast_rcp(1.f + fast_exp2(x * cap2));  // cap tanh(x / cap)
-        s[r] = x * LOG2E;
-      }
-    } else {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float x = s[r] * scale;
-        s[r] = x * LOG2E;
-      }
-    }
-    uint32_t vis = 0;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) vis |= (uint32_t)visible(qi, kbase + (r >> 2) * 8 + (r & 3), len, window, causal) << r;
-    if (key_mask) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r)  // read only for visible keys, which lie inside the sequence
-        if (((vis >> r) & 1u) && !key_mask[start + kbase + (r >> 2) * 8 + (r & 3)]) vis &= ~(1u << r);
-    }
-    float tmax = NEG_BIG;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) tmax = ((vis >> r) & 1u) ? fmaxf(tmax, s[r]) : tmax;
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    const float mnew = fmaxf(m, tmax);
-    const float alpha = fast_exp2(m - mnew);
-    m = mnew;
-    l *= alpha;
-    if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {  // some row's running max moved
-#pragma unroll
-      for (int i = 0; i < NDB; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float p = ((vis >> r) & 1u) ? fast_exp2(s[r] - mnew) : 0.f;
-      s[r] = p;
-      l += p;
-    }
-#pragma unroll
-    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        o[db] = mfma32_f32(vs[((i >> 2) * 8 + 4 * hh + (i & 3)) * VP + db * 32 + lrow], s[i], o[db]);
-    if (more) put_k();
-  }
-
-  // merge the waves' states: wave w writes O^T, m and the row sum into its region, then every thread
-  // combines (query, head-dim) elements, consecutive threads taking consecutive head dims
-  l += __shfl_xor(l, 32, 64);
-  __syncthreads();  // every wave is done with its K / V region
-#pragma unroll
-  for (int db = 0; db < NDB; ++db)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) ks[(db * 32 + (r >> 2) * 8 + 4 * hh + (r & 3)) * OP + lrow] = o[db][r];
-  if (hh == 0) {
-    ks[D * OP + lrow] = m;
-    ks[D * OP + 32 + lrow] = l;
+  // the query tile, in the space that takes the waves' O later
+  for (int idx = tid; idx < BQ * (D / 4); idx += 64 * WAVES) {
+    const int q = idx / (D / 4), d = idx % (D / 4) * 4;
+    *reinterpret_cast<floatx4 *>(os + q * OP + d) =
+        *reinterpret_cast<const floatx4 *>(Q + (start + min(q0 + q, len - 1)) * q_stride + (long)h * D + d);
   }
   __syncthreads();
-  for (int idx = tid; idx < 32 * D; idx += 64 * F_WAVES) {
-    const int q = idx / D, d = idx % D;
-    if (q0 + q >= len) continue;
-    float mx = NEG_BIG;
+  const float *const qs = os + r * OP + 4 * g;
+  floatx4 kf[SUB][C];
+  auto load_k = [&](int k0) __attribute__((always_inline)) {  // rows past the sequence read its last one (masked)
 #pragma unroll
-    for (int w = 0; w < F_WAVES; ++w) mx = fmaxf(mx, smem[w * REGION + D * OP + q]);
-    float acc = 0.f, sum = 0.f;
+    for (int s = 0; s < SUB; ++s) {
+      const float *p = kp + (long)min(k0 + 16 * s + r, len - 1) * k_stride;
 #pragma unroll
-    for (int w = 0; w < F_WAVES; ++w) {
-      const float *st = smem + w * REGION;
-      const float f = fast_exp2(st[D * OP + q] - mx);
-      acc += st[d * OP + q] * f;
-      sum += st[D * OP + 32 + q] * f;
+      for (int c = 0; c < C; ++c) kf[s][c] = *reinterpret_cast<const floatx4 *>(p + 16 * c);
     }
-    O[(start + q0 + q) * o_stride + (long)h * D + d] = sum > 0.f ? acc / sum : 0.f;  // no visible key: zeros
+  };
+  floatx4 o[QB][C];
+  float m[QB], l[QB];
+#pragma unroll
+  for (int u = 0; u < QB; ++u) {
+    m[u] = NEG_BIG;
+    l[u] = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) o[u][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+  int k0 = klo / KB * KB + wave * KB;
+  if (k0 < khi) load_k(k0);
+  for (; k0 < khi; k0 += WAVES * KB) {
+    floatx4 vf[SUB][4][A];
+    // one mask byte per lane covers the block; bit 16 s + 4 g + t is the lane's key (s, t)
+    const uint8_t mk = key_mask ? key_mask[start + min(k0 + min(lane, KB - 1), len - 1)] : (uint8_t)1;
+#pragma unroll
+    for (int s = 0; s < SUB; ++s)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const float *p = vp + (long)min(k0 + 16 * s + 4 * g + t, len - 1) * v_stride;
+#pragma unroll
+        for (int a = 0; a < A; ++a) vf[s][t][a] = *reinterpret_cast<const floatx4 *>(p + 64 * a);
+      }
+    __builtin_amdgcn_sched_barrier(0);  // V's loads go out before the products
+    floatx4 part[QB][SUB][NC];
+#pragma unroll
+    for (int u = 0; u < QB; ++u)
+#pragma unroll
+      for (int s = 0; s < SUB; ++s)
+#pragma unroll
+        for (int n = 0; n < NC; ++n) part[u][s][n] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      floatx4 qf[QB];
+#pragma unroll
+      for (int u = 0; u < QB; ++u) qf[u] = *reinterpret_cast<const floatx4 *>(qs + 16 * u * OP + 16 * c);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int s = 0; s < SUB; ++s)
+#pragma unroll
+          for (int u = 0; u < QB; ++u) {
+            floatx4 &acc = part[u][s][(4 * c + e) % NC];
+            acc = mfma16_f32(kf[s][c][e], qf[u][e], acc);
+          }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    load_k(k0 + WAVES * KB);
+    floatx4 sc[QB][SUB];
+#pragma unroll
+    for (int u = 0; u < QB; ++u)
+#pragma unroll
+      for (int s = 0; s < SUB; ++s) {
+#pragma unroll
+        for (int w = NC / 2; w >= 1; w /= 2)
+#pragma unroll
+          for (int n = 0; n < w; ++n) part[u][s][n] += part[u][s][n + w];
+        sc[u][s] = part[u][s][0];
+      }
+    const uint64_t bits = __builtin_amdgcn_ballot_w64(mk != 0) >> (4 * g);
+#pragma unroll
+    for (int u = 0; u < QB; ++u) {
+      const int qi = q0 + 16 * u + r;
+      if (softcap > 0.f) {
+#pragma unroll
+        for (int s = 0; s < SUB; ++s)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) sc[u][s][t] = softcap * tanhf(sc[u][s][t] * scale / softcap);
+      } else {
+#pragma unroll
+        for (int s = 0; s < SUB; ++s) sc[u][s] *= scale;
+      }
+      uint32_t vis = 0;
+      float mx = NEG_BIG;
+#pragma unroll
+      for (int s = 0; s < SUB; ++s)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const bool v = visible(qi, k0 + 16 * s + 4 * g + t, len, window, causal) && ((bits >> (16 * s + t)) & 1u);
+          vis |= (uint32_t)v << (4 * s + t);
+          mx = v ? fmaxf(mx, sc[u][s][t]) : mx;
+        }
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      const float mn = fmaxf(m[u], mx);
+      const float alpha = expf(m[u] - mn);
+      m[u] = mn;
+      l[u] *= alpha;
+      if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {  // some row's running max moved
+#pragma unroll
+        for (int c = 0; c < C; ++c) o[u][c] *= alpha;
+      }
+#pragma unroll
+      for (int s = 0; s < SUB; ++s)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const float p = ((vis >> (4 * s + t)) & 1u) ? expf(sc[u][s][t] - mn) : 0.f;
+          sc[u][s][t] = p;
+          l[u] += p;
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < SUB; ++s)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int a = 0; a < A; ++a)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int u = 0; u < QB; ++u) o[u][4 * a + e] = mfma16_f32(vf[s][t][a][e], sc[u][s][t], o[u][4 * a + e]);
+  }
+#pragma unroll
+  for (int u = 0; u < QB; ++u) {
+    l[u] += __shfl_xor(l[u], 16, 64);
+    l[u] += __shfl_xor(l[u], 32, 64);
+    if (u == 0) __syncthreads();  // the query tile is no longer read
+    if (g == 0) {
+      ms[wave][16 * u + r] = m[u];
+      ls[wave][16 * u + r] = l[u];
+    }
+    float *row = os + (wave * BQ + 16 * u + r) * OP + 16 * g;
+#pragma unroll
+    for (int a = 0; a < A; ++a)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<floatx4 *>(row + 64 * a + 4 * i) =
+            floatx4{o[u][4 * a][i], o[u][4 * a + 1][i], o[u][4 * a + 2][i], o[u][4 * a + 3][i]};
+  }
+  __syncthreads();
+  for (int idx = tid; idx < BQ * (D / 4); idx += 64 * WAVES) {
+    const int q = idx / (D / 4), d = idx % (D / 4) * 4;
+    if (q0 + q >= len) continue;
+    float mx = ms[0][q];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) mx = fmaxf(mx, ms[w][q]);
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    float sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float f = expf(ms[w][q] - mx);
+      acc += *reinterpret_cast<const floatx4 *>(os + (w * BQ + q) * OP + d) * f;
+      sum += ls[w][q] * f;
+    }
+    floatx4 v = {0.f, 0.f, 0.f, 0.f};  // a row that sees no key: zeros
+    if (sum > 0.f) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = acc[e] / sum;
+    }
+    *reinterpret_cast<floatx4 *>(O + (start + q0 + q) * o_stride + (long)h * D + d) = v;
   }
 }
 
@@ -979,25 +883,27 @@ hipError_t launch_bf16_d(const AttnArgs &a, hipStream_t s) {
   return hipErrorInvalidValue;
 }
 
-template <int D, int TPQ>
-hipError_t launch_f32_d(const AttnArgs &a, hipStream_t s) {
-  constexpr int QPB = THREADS / TPQ;
-  const dim3 grid((a.max_seq_len + QPB - 1) / QPB, a.num_seqs, a.hq);
-  attn_f32_kernel<D, TPQ><<<grid, dim3(THREADS), 0, s>>>(
+template <int D, int QB, int W>
+hipError_t launch_f32_dqw(const AttnArgs &a, hipStream_t s) {
+  const dim3 grid((unsigned)((a.max_seq_len + 16 * QB - 1) / (16 * QB)) * a.hq, a.num_seqs);
+  attn_f32_kernel<D, QB, W, 1><<<grid, dim3(64 * W), 0, s>>>(
       static_cast<const float *>(a.q), static_cast<const float *>(a.k), static_cast<const float *>(a.v),
       static_cast<float *>(a.out), a.seq_start, a.seq_len, a.max_seq_len, a.hq, a.hkv, a.q_stride, a.k_stride,
       a.v_stride, a.out_stride, a.scale, a.softcap, a.window, a.causal, a.key_mask);
   return hipGetLastError();
 }
 
+// Head_dim 64 and 128: 32 queries, 8 waves (two per SIMD; 4 waves, or 32 keys a step, measured 10 to 60% slower).
+// Head_dim 256 has registers for 4 waves: 32 queries where that fills the CUs (4 x 1000, 8 heads 412 against 463 us),
+// else 16 (1 x 97, 8 heads 17 against 22 us; 2 x 200, 4 heads 20 against 30).
 template <int D>
-hipError_t launch_f32_mfma_d(const AttnArgs &a, hipStream_t s) {
-  const dim3 grid((a.max_seq_len + 31) / 32, a.num_seqs, a.hq);
-  attn_f32_mfma_kernel<D><<<grid, dim3(64 * F_WAVES), 0, s>>>(
-      static_cast<const float *>(a.q), static_cast<const float *>(a.k), static_cast<const float *>(a.v),
-      static_cast<float *>(a.out), a.seq_start, a.seq_len, a.max_seq_len, a.hq, a.hkv, a.q_stride, a.k_stride,
-      a.v_stride, a.out_stride, a.scale, a.softcap, a.window, a.causal, a.key_mask);
-  return hipGetLastError();
+hipError_t launch_f32_d(const AttnArgs &a, hipStream_t s) {
+  if constexpr (D < 256) {
+    return launch_f32_dqw<D, 2, 8>(a, s);
+  } else {
+    const long tiles = (long)((a.max_seq_len + 31) / 32) * a.hq * a.num_seqs;
+    return tiles >= 256 ? launch_f32_dqw<D, 2, 4>(a, s) : launch_f32_dqw<D, 1, 4>(a, s);
+  }
 }
 
 // Thread t packs word t % words of sequence t / words: bit j <- key_mask[seq_start + 32 w + j] != 0 for keys
@@ -1040,11 +946,9 @@ hipError_t dx_attn_bf16(const AttnArgs &a, hipStream_t s) {
 
 hipError_t dx_attn_f32(const AttnArgs &a, hipStream_t s) {
   switch (a.d) {
-    case 64: return launch_f32_mfma_d<64>(a, s);
-    case 128: return launch_f32_mfma_d<128>(a, s);
-    // head_dim 256 keeps the VALU kernel (the matrix-core one would hold 128 query registers per lane),
-    // 16 threads per query
-    case 256: return launch_f32_d<256, 16>(a, s);
+    case 64: return launch_f32_d<64>(a, s);
+    case 128: return launch_f32_d<128>(a, s);
+    case 256: return launch_f32_d<256>(a, s);
   }
   return hipErrorInvalidValue;
 }

@@ -382,6 +382,40 @@ def test_attention_fp32_config1() -> None:
     np.testing.assert_allclose(got[0], want, rtol=1e-4, atol=1e-4)
 
 
+# (lengths, hq, hkv, d, window, softcap, causal): tiles of 16 (head_dim 256, fewer than 256 tiles of 32) and of 32
+# queries, 16-key blocks split over 4 (head_dim 256) or 8 waves; ends of tiles, fewer blocks than waves, empty
+# sequences, one launch at and one below the switch of the tile height
+F32_CASES = [
+    ([1, 15, 16, 17, 31, 32, 33, 0, 130], 4, 2, 256, 0, 50.0, True),
+    ([257, 300], 2, 1, 256, 40, 0.0, True),
+    ([145, 64], 4, 4, 256, 33, 0.0, False),
+    ([512, 512, 512, 500], 4, 1, 256, 0, 20.0, True),     # 64 tiles x 4 heads: 32 queries
+    ([480, 33, 480, 480], 4, 4, 256, 0, 0.0, False),      # 60 tiles x 4 heads: 16 queries
+    ([1, 15, 16, 17, 127, 128, 129, 0, 300], 8, 2, 128, 0, 50.0, True),
+    ([200, 131], 4, 4, 128, 17, 0.0, False),
+    ([1, 31, 33, 127, 129, 0, 300], 6, 6, 64, 0, 0.0, False),
+    ([200, 131], 8, 4, 64, 40, 80.0, True),
+]
+
+
+@pytest.mark.parametrize("lengths,hq,hkv,d,window,softcap,causal", F32_CASES)
+def test_attention_fp32_tiles(lengths, hq, hkv, d, window, softcap, causal) -> None:
+    """fp32 within 1e-4, the bound of the fp32 cases above (scores are sums of d <= 256 products and weights sum
+    to one: the rounding of either stays below d 2^-24 = 2e-5 of the operands' magnitude)."""
+    from deciax_amd import kernels as K
+    from oracle.attention import attention_packed
+
+    say(f"attention fp32 tiles lengths={lengths} hq={hq} hkv={hkv} d={d} window={window} softcap={softcap} causal={causal}")
+    q, k, v, starts = _packed_case(d + window, lengths, hq, hkv, d, dtype="f32", scale=1.0)
+    rows = q.shape[0]
+    out = K.attention_varlen(*(to_dev(a.reshape(rows, -1), "f32") for a in (q, k, v)), i32(starts), i32(lengths),
+                             max(lengths), num_q_heads=hq, num_kv_heads=hkv, head_dim=d, scale=d ** -0.5,
+                             softcap=softcap, window=window, causal=causal)
+    want = attention_packed(q, k, v, starts, lengths, scale=d ** -0.5, softcap_value=softcap, window=window,
+                            causal=causal, bf16=False)
+    np.testing.assert_allclose(to_np(out).reshape(want.shape), want, rtol=1e-4, atol=1e-4)
+
+
 @pytest.mark.parametrize("window", [0, 64])
 def test_attention_fp32_window_softcap(window: int) -> None:
     from deciax_amd import kernels as K
