@@ -47,8 +47,13 @@ constexpr int BKV = 64;     // V^T block alignment of dx_transpose_v
 // epilogue and barrier waits overlap the other's key loop; it halves the query rows per staged K/V tile.
 // Head_dim 128 takes the short form when a query row sees 2048 keys or fewer on average (window <= 2048,
 // or causal sequences up to 4096): 27B heads, 8 x 2048 -4%, window 512 -12 to -15%, window 1024 -5 to
-// -10%, 16 x 3400 -2%; on longer spans it measured +0.2 to +1.1% (4 x 16384). Head_dim 256 keeps the long
-// form everywhere: the short one measured 6-11% slower on every shape but window 512 (within 1.5%).
+// -10%, 16 x 3400 -2%; on longer spans it measured +0.2 to +1.1% (4 x 16384). Head_dim 64 takes it up to 4096
+// keys: its 32 KB ring puts two workgroups on a CU too, and half the query rows spread small launches further
+// (12 heads: 2 x 1021 35 -> 30 us, 4 x 2048 83 -> 72, 1 x 2048 42 -> 32, 8 x 1021 49 -> 47; 4 x 8192 +2.8%).
+// Head_dim 256: the short form measured 6-11% slower. Where the long one has at most a workgroup per CU, four waves
+// over the same 4-stage ring (one per SIMD) halve what the longest workgroup has to do: 16/8 heads, 1 x 736 40 -> 31
+// us, 1 x 2000 102 -> 84, 1 x 3300 161 -> 133 (208 workgroups of 8 waves), 4 x 1000 63 -> 59 (256); 1 x 4500 (288)
+// is even, 8 x 1000 (512) 84 -> 114. Two waves measured like four. All forms give the same bits.
 // bf16 grid order switch (see attn_bf16_kernel). Whole units per XCD measured 3-9% faster at 3257-4096
 // tokens (16 sequences, 9B and 27B heads), 2% slower at 8 x 3072 and 15% slower at 8 x 2048.
 constexpr int SHORT_SEQ = 3072;
@@ -135,7 +140,7 @@ struct Flag {
 // 32 w + j) hides keys beyond the causal / window rule. Tiles that hold a masked key take the masked body,
 // and a query row that sees no key is written as zeros.
 template <int D, int G, int MODE, bool KM, int WAVES, int NSTAGE>
-__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES * NSTAGE == 16 ? 1 : 2, 2)))
 attn_bf16_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ Vt,
                  uint16_t *__restrict__ O, const int32_t *__restrict__ seq_start,
                  const int32_t *__restrict__ seq_len, const int32_t *__restrict__ vt_start, long vt_seq_stride,
@@ -868,8 +873,12 @@ inline long mean_key_span(const AttnArgs &a) {
 template <int D, int G>
 hipError_t launch_bf16_dg(const AttnArgs &a, hipStream_t s) {
   if (a.softcap > 0.f && !fixed_shift(a)) return launch_bf16_dgw<D, G, 8, 4>(a, s);  // the one form built with MODE_CAP
-  if constexpr (D == 128)
-    if (mean_key_span(a) <= 2048) return launch_bf16_dgw<D, G, 4, 2>(a, s);
+  if constexpr (D <= 128)
+    if (mean_key_span(a) <= (D == 64 ? 4096 : 2048)) return launch_bf16_dgw<D, G, 4, 2>(a, s);
+  if constexpr (D == 256) {
+    const long rows = 32 * (8 / G), long_form = (a.max_seq_len + rows - 1) / rows * a.hkv * a.num_seqs;
+    if (long_form <= 256) return launch_bf16_dgw<D, G, 4, 4>(a, s);
+  }
   return launch_bf16_dgw<D, G, 8, 4>(a, s);
 }
 

@@ -285,6 +285,48 @@ def test_attention_head_dim_128_short_and_long_forms_agree(hq: int, hkv: int) ->
         close(got[s + qpos], want, 2e-2, MEAN_REL["flash"])
 
 
+@pytest.mark.parametrize("hq,hkv,d,window,softcap,causal,longer", [
+    (16, 8, 256, 0, 50.0, True, 8192),      # at most 256 workgroups of 8 waves: 4 waves
+    (8, 2, 256, 300, 0.0, True, 16384),
+    (4, 4, 256, 0, 0.0, False, 16384),
+    (12, 12, 64, 0, 0.0, False, 8192),      # 4096 keys or fewer a row: 4 waves over two stages
+    (8, 2, 64, 0, 50.0, True, 16384),
+])
+def test_attention_forms_agree(hq: int, hkv: int, d: int, window: int, softcap: float, causal: bool,
+                               longer: int) -> None:
+    """Small launches at head_dim 256 and short spans at head_dim 64 run 4-wave workgroups, the others 8-wave ones,
+    over the same rows and keys in the same order: bit for bit the same output. A larger declared max_seq_len flips
+    the form; rows of the small form against the oracle."""
+    import torch
+
+    from deciax_amd import kernels as K
+    from oracle.attention import attention_seq
+
+    lengths = [700, 1, 33, 450]
+    say(f"attention forms hq={hq} hkv={hkv} d={d} window={window} softcap={softcap} causal={causal}")
+    q, k, v, starts = _packed_case(31 + d + hkv, lengths, hq, hkv, d)
+    rows = q.shape[0]
+    qd, kd, vd = (to_dev(a.reshape(rows, -1)) for a in (q, k, v))
+    padded = [(n + 63) // 64 * 64 for n in lengths]
+    vt_start = np.concatenate([[0], np.cumsum(padded)[:-1]])
+    vt = torch.zeros((hkv * d, int(sum(padded))), dtype=torch.bfloat16, device="cuda")
+    K.transpose_v(vd, vt, i32(starts), i32(lengths), i32(vt_start), max(lengths), num_kv_heads=hkv, head_dim=d)
+
+    def run(max_len: int) -> np.ndarray:
+        return to_np(K.attention_vt(qd, kd, vt, i32(starts), i32(lengths), i32(vt_start), max_len, num_q_heads=hq,
+                                    num_kv_heads=hkv, head_dim=d, scale=d ** -0.5, softcap=softcap, window=window,
+                                    causal=causal))
+
+    small = run(max(lengths))
+    np.testing.assert_array_equal(small, run(longer))
+    got = small.reshape(rows, hq, d)
+    for s, n in zip(starts, lengths):
+        qpos = np.unique(np.array([0, n // 2, n - 1]))
+        want = attention_seq(q[s:s + n], k[s:s + n], v[s:s + n], scale=d ** -0.5, softcap_value=softcap,
+                             window=window, causal=causal, query_pos=qpos, rounding="flash")
+        close(got[s + qpos], want, 2e-2)
+
+
 LONG_CASES = [
     # (hq, hkv, d, window, lengths): 24 or 48 (sequence, KV head) units, dealt out whole to the XCDs
     (16, 8, 256, 4096, [300, 5000, 4097]),
