@@ -74,6 +74,18 @@ int validate_attn(const void *q, const void *k, const void *v, const void *out, 
   return DX_OK;
 }
 
+int validate_attn_v(int32_t head_dim, int32_t num_kv_heads, int64_t k_row_stride, int64_t v_row_stride, int32_t dtype) {
+  const int64_t vec = dtype == DX_BF16 ? 8 : 4;
+  REQUIRE(v_row_stride % vec == 0 && v_row_stride >= (int64_t)num_kv_heads * head_dim,
+          "attention: bad v row stride %ld", (long)v_row_stride);
+  // row strides whose 32-key block would not fit 32-bit byte offsets: never taken at head_dim 64 and 128
+  if (dtype == DX_F32)
+    SUPPORTED(head_dim > 128 || (k_row_stride < (INT64_C(1) << 24) && v_row_stride < (INT64_C(1) << 24)),
+              "attention: fp32 k / v row strides of 2^24 elements or more are not supported at head_dim %d",
+              head_dim);
+  return DX_OK;
+}
+
 // The bf16 kernel reads one sequence's K rows and one KV head's V^T block through buffer resources whose
 // byte ranges and per-lane offsets are 32-bit: len * k_stride * 2 bytes of K, and
 // ((D - 1) * vt_ld + len rounded up to 64) * 2 bytes of V^T. Larger spans would wrap.
@@ -178,14 +190,8 @@ int attn_prefill(const void *q, const void *k, const void *v, const uint8_t *key
   int st = validate_attn(q, k, v, out, seq_start, seq_len, num_seqs, max_seq_len, num_q_heads, num_kv_heads,
                          head_dim, q_row_stride, k_row_stride, out_row_stride, scale, softcap, window, dtype);
   if (st) return st;
-  const int64_t vec = dtype == DX_BF16 ? 8 : 4;
-  REQUIRE(v_row_stride % vec == 0 && v_row_stride >= (int64_t)num_kv_heads * head_dim,
-          "attention: bad v row stride %ld", (long)v_row_stride);
-  // row strides whose 32-key block would not fit 32-bit byte offsets: never taken at head_dim 64 and 128
-  if (dtype == DX_F32)
-    SUPPORTED(head_dim > 128 || (k_row_stride < (INT64_C(1) << 24) && v_row_stride < (INT64_C(1) << 24)),
-              "attention: fp32 k / v row strides of 2^24 elements or more are not supported at head_dim %d",
-              head_dim);
+  st = validate_attn_v(head_dim, num_kv_heads, k_row_stride, v_row_stride, dtype);
+  if (st) return st;
   if (num_seqs == 0 || max_seq_len == 0) return DX_OK;
   AttnArgs a{q, k, v, out, seq_start, seq_len, nullptr, num_seqs, max_seq_len, num_q_heads, num_kv_heads, head_dim,
              q_row_stride, k_row_stride, v_row_stride, out_row_stride, 0, scale, softcap, window, causal ? 1 : 0};
@@ -268,6 +274,63 @@ int dx_attn_prefill_masked(const void *q, const void *k, const void *v, const ui
   return attn_prefill(q, k, v, key_mask, out, seq_start, seq_len, num_seqs, max_seq_len, num_q_heads, num_kv_heads,
                       head_dim, q_row_stride, k_row_stride, v_row_stride, out_row_stride, scale, softcap, window,
                       causal, dtype, workspace, workspace_bytes, stream);
+}
+
+int64_t dx_attn_padded_workspace(int32_t batch, int32_t len, int32_t num_kv_heads, int32_t head_dim, int32_t dtype) {
+  if (dtype != DX_BF16 || batch <= 0 || len <= 0) return 0;
+  // V^T and the mask bits as the masked form lays them out, then the sequence descriptors
+  return align_up(dx_attn_prefill_masked_workspace(batch, len, num_kv_heads, head_dim, dtype), 256) + 8 * (int64_t)batch;
+}
+
+int dx_attn_padded(const void *q, const void *k, const void *v, const uint8_t *key_mask, void *out, int32_t batch,
+                   int32_t len, int32_t num_q, int32_t num_k, int32_t num_q_heads, int32_t num_kv_heads,
+                   int32_t head_dim, int64_t q_row_stride, int64_t k_row_stride, int64_t v_row_stride,
+                   int64_t out_row_stride, float scale, float softcap, int32_t window, int32_t causal, int32_t dtype,
+                   void *workspace, int64_t workspace_bytes, void *stream) {
+  REQUIRE(key_mask, "attention: key_mask must not be null");
+  REQUIRE(batch >= 0 && len >= 0 && num_q >= 0 && num_q <= len && num_k >= 1 && num_k <= len,
+          "attention: %d queries and %d keys in padded rows of %d", num_q, num_k, len);
+  const int32_t *some = reinterpret_cast<const int32_t *>(key_mask);  // descriptors follow in the workspace
+  int st = validate_attn(q, k, v, out, some, some, batch, len, num_q_heads, num_kv_heads, head_dim, q_row_stride,
+                         k_row_stride, out_row_stride, scale, softcap, window, dtype);
+  if (!st) st = validate_attn_v(head_dim, num_kv_heads, k_row_stride, v_row_stride, dtype);
+  if (st) return st;
+  REQUIRE((int64_t)batch * len <= INT32_MAX, "attention: %d padded sequences of %d rows", batch, len);
+  if (batch == 0 || num_q == 0) return DX_OK;
+  hipStream_t s = as_stream(stream);
+  AttnArgs a{q, k, v, out, nullptr, nullptr, nullptr, batch, len, num_q_heads, num_kv_heads, head_dim,
+             q_row_stride, k_row_stride, v_row_stride, out_row_stride, 0, scale, softcap, window, causal ? 1 : 0};
+  AttnArgs rows = a;  // token-major values, for the rows that see no key
+  hipError_t e;
+  if (dtype == DX_F32) {
+    a.key_mask = key_mask;
+    e = dx_attn_f32(a, s);
+  } else {
+    const int64_t seq_stride = align_up(len, 64), vt_ld = seq_stride * batch;
+    st = check_bf16_ranges(len, k_row_stride, head_dim, vt_ld);
+    if (st) return st;
+    const int64_t vt_bytes = dx_attn_prefill_workspace(batch, len, num_kv_heads, head_dim, DX_BF16);
+    const int64_t masked = dx_attn_prefill_masked_workspace(batch, len, num_kv_heads, head_dim, DX_BF16);
+    const int64_t need = dx_attn_padded_workspace(batch, len, num_kv_heads, head_dim, DX_BF16);
+    REQUIRE(workspace && aligned16(workspace), "attention: bf16 needs a 16-byte aligned workspace");
+    REQUIRE(workspace_bytes >= need, "attention: workspace of %ld bytes, need %ld", (long)workspace_bytes, (long)need);
+    char *ws = static_cast<char *>(workspace);
+    uint32_t *bits = reinterpret_cast<uint32_t *>(ws + align_up(vt_bytes, 256));
+    int32_t *starts = reinterpret_cast<int32_t *>(ws + align_up(masked, 256)), *lens = starts + batch;
+    a.key_words = key_mask_words(len);
+    a.key_bits = bits;
+    a.v = workspace;
+    a.v_stride = vt_ld;
+    a.vt_seq_stride = seq_stride;
+    a.seq_start = starts;
+    a.seq_len = lens;
+    e = dx_prepare_padded_launch(static_cast<const uint16_t *>(v), static_cast<uint16_t *>(workspace), key_mask, bits,
+                                 starts, lens, batch, len, a.key_words, num_kv_heads, head_dim, v_row_stride,
+                                 seq_stride, vt_ld, s);
+    if (e == hipSuccess) e = dx_attn_bf16(a, s);
+  }
+  if (e == hipSuccess) e = dx_fill_unseen_launch(rows, key_mask, num_q, num_k, dtype == DX_F32, s);
+  return check_launch(e, "padded attention launch");
 }
 
 int dx_attn_prefill_vt(const void *q, const void *k, const void *vt, void *out, const int32_t *seq_start,

@@ -593,11 +593,11 @@ attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, const 
   __shared__ float ms[WAVES][BQ], ls[WAVES][BQ];
 
   const int b = blockIdx.y, h = blockIdx.x % hq, g_kv = h / (hq / hkv);
-  const int len = min(max(seq_len[b], 0), max_seq_len);
+  const int len = seq_len ? min(max(seq_len[b], 0), max_seq_len) : max_seq_len;  // null: a padded batch
   const int ntiles = (max_seq_len + BQ - 1) / BQ;
   const int q0 = (ntiles - 1 - (int)blockIdx.x / hq) * BQ;  // heaviest (last) query tiles first
   if (q0 >= len) return;
-  const long start = seq_start[b];
+  const long start = seq_start ? (long)seq_start[b] : (long)b * max_seq_len;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
 
@@ -783,21 +783,48 @@ attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, const 
   }
 }
 
+// What one launch prepares for a padded batch (every sequence max_seq_len rows, back to back) beside the transpose:
+// the sequence descriptors and the mask words. Null key_mask: a packed batch, descriptors given.
+struct PaddedPrep {
+  const uint8_t *key_mask = nullptr;
+  uint32_t *bits = nullptr;
+  int32_t *seq_start = nullptr, *seq_len = nullptr;
+  int words = 0;
+};
+
 // V rows -> V^T tiles. Grid: (64-row tiles of the longest sequence, sequences,
-// kv heads x D/64). Rows past seq_len up to the next multiple of 64 are
-// written as zeros, so P.V never multiplies a zero probability by stale data.
+// kv heads x D/64; with a PaddedPrep one more, whose workgroup x packs the 64 keys of tile x). Rows past seq_len up
+// to the next multiple of 64 are written as zeros, so P.V never multiplies a zero probability by stale data.
+template <bool PADDED>
 __global__ void __launch_bounds__(THREADS)
 transpose_v_kernel(const uint16_t *__restrict__ V, uint16_t *__restrict__ Vt, const int32_t *__restrict__ seq_start,
                    const int32_t *__restrict__ seq_len, const int32_t *__restrict__ vt_start, long vt_seq_stride,
-                   int max_seq_len, int d, long v_stride, long vt_ld) {
+                   int max_seq_len, int d, long v_stride, long vt_ld, PaddedPrep pp) {
+  if constexpr (PADDED) {
+    if (blockIdx.z == gridDim.z - 1) {
+      const int b = blockIdx.y, key = (int)blockIdx.x * 64 + (int)threadIdx.x;
+      if (threadIdx.x >= 64) return;
+      const uint64_t m = __builtin_amdgcn_ballot_w64(key < max_seq_len && pp.key_mask[(long)b * max_seq_len + min(key, max_seq_len - 1)] != 0);
+      if (threadIdx.x == 0) {
+        uint32_t *w = pp.bits + (long)b * pp.words + 2 * blockIdx.x;
+        w[0] = (uint32_t)m;
+        w[1] = (uint32_t)(m >> 32);
+        if (blockIdx.x == 0) {
+          pp.seq_start[b] = b * max_seq_len;
+          pp.seq_len[b] = max_seq_len;
+        }
+      }
+      return;
+    }
+  }
   __shared__ uint16_t tile[64][66];
   const int b = blockIdx.y;
-  const int len = min(max(seq_len[b], 0), max_seq_len);
+  const int len = PADDED ? max_seq_len : min(max(seq_len[b], 0), max_seq_len);
   const int p0 = blockIdx.x * 64;
   if (p0 >= len) return;
   const int dblocks = d / 64;
   const int g = blockIdx.z / dblocks, d0 = (blockIdx.z % dblocks) * 64;
-  const long start = seq_start[b];
+  const long start = PADDED ? (long)b * max_seq_len : seq_start[b];
   const long vts = vt_start ? (long)vt_start[b] : (long)b * vt_seq_stride;
   const int tid = threadIdx.x;
   {
@@ -915,6 +942,61 @@ hipError_t launch_f32_d(const AttnArgs &a, hipStream_t s) {
   }
 }
 
+DX_DEVICE float as_float(float v) { return v; }
+DX_DEVICE float as_float(uint16_t v) { return bf2f(v); }
+DX_DEVICE void put(float *p, float v) { *p = v; }
+DX_DEVICE void put(uint16_t *p, float v) { *p = f2bf(v); }
+
+// Padded batch: query rows that see no key get the mean of the sequence's num_k value rows (softmax of equal
+// scores). A workgroup looks at 64 rows. Row i sees keys [lo(i), hi(i)), and hi grows by one a row at most: the last
+// kept key below hi(first row), found by all threads, and the 64 mask bytes from there on tell for each row whether
+// its last kept key reaches lo(i). Almost every workgroup ends there; the others read the values.
+template <typename T>
+__global__ void __launch_bounds__(THREADS)
+fill_unseen_kernel(const T *__restrict__ V, T *__restrict__ O, const uint8_t *__restrict__ key_mask, int len, int num_q,
+                   int num_k, int hq, int hkv, int d, long v_stride, long o_stride, int window, int causal) {
+  __shared__ int last_kept[THREADS / 64];
+  __shared__ uint64_t unseen;
+  const int b = blockIdx.y, i0 = blockIdx.x * 64, tid = threadIdx.x, lane = tid & 63;
+  const uint8_t *mask = key_mask + (long)b * len;
+  auto lo = [&](int i) { return window <= 0 ? 0 : max(0, causal ? i - window + 1 : i - window); };
+  auto hi = [&](int i) { return causal ? min(i + 1, num_k) : window > 0 ? min(i + window + 1, num_k) : num_k; };
+  const int h0 = hi(i0);
+  int last = -1;
+  for (int k = h0 - 1 - tid; k >= lo(i0) && last < 0; k -= THREADS)
+    if (mask[k]) last = k;
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) last = max(last, __shfl_xor(last, off, 64));
+  if (lane == 0) last_kept[tid >> 6] = last;
+  __syncthreads();
+  if (tid < 64) {
+    for (int w = 0; w < THREADS / 64; ++w) last = max(last, last_kept[w]);
+    const uint64_t next = __builtin_amdgcn_ballot_w64(h0 + lane < num_k && mask[min(h0 + lane, num_k - 1)] != 0);
+    const int i = i0 + lane, n = hi(i) - h0;  // 0 <= n < 64
+    const uint64_t below = next & ((1ull << n) - 1);
+    if (below) last = h0 + 63 - __builtin_clzll(below);
+    const uint64_t u = __builtin_amdgcn_ballot_w64(i < num_q && last < lo(i));
+    if (lane == 0) unseen = u;
+  }
+  __syncthreads();
+  if (!unseen) return;
+  const int group = hq / hkv;
+  for (int c = tid; c < hkv * d; c += THREADS) {
+    const T *v = V + (long)b * len * v_stride + c;
+    float part[8] = {};
+    int k = 0;
+    for (; k + 8 <= num_k; k += 8)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) part[e] += as_float(v[(long)(k + e) * v_stride]);
+    for (; k < num_k; ++k) part[0] += as_float(v[(long)k * v_stride]);
+    const float mean = (((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]))) / num_k;
+    for (uint64_t u = unseen; u; u &= u - 1) {
+      T *out = O + ((long)b * len + i0 + __builtin_ctzll(u)) * o_stride + (long)(c / d) * group * d + c % d;
+      for (int j = 0; j < group; ++j) put(out + j * d, mean);
+    }
+  }
+}
+
 // Thread t packs word t % words of sequence t / words: bit j <- key_mask[seq_start + 32 w + j] != 0 for keys
 // inside the sequence, 0 past its length.
 __global__ void __launch_bounds__(THREADS)
@@ -973,7 +1055,31 @@ hipError_t dx_transpose_v_launch(const uint16_t *v, uint16_t *vt, const int32_t 
                                  const int32_t *vt_start, long vt_seq_stride, int num_seqs, int max_seq_len, int hkv,
                                  int d, long v_stride, long vt_ld, hipStream_t s) {
   const dim3 grid((max_seq_len + 63) / 64, num_seqs, hkv * (d / 64));
-  transpose_v_kernel<<<grid, dim3(THREADS), 0, s>>>(v, vt, seq_start, seq_len, vt_start, vt_seq_stride, max_seq_len,
-                                                   d, v_stride, vt_ld);
+  transpose_v_kernel<false><<<grid, dim3(THREADS), 0, s>>>(v, vt, seq_start, seq_len, vt_start, vt_seq_stride,
+                                                          max_seq_len, d, v_stride, vt_ld, PaddedPrep{});
+  return hipGetLastError();
+}
+
+hipError_t dx_prepare_padded_launch(const uint16_t *v, uint16_t *vt, const uint8_t *key_mask, uint32_t *bits,
+                                    int32_t *seq_start, int32_t *seq_len, int batch, int len, int words, int hkv, int d,
+                                    long v_stride, long vt_seq_stride, long vt_ld, hipStream_t s) {
+  const dim3 grid((len + 63) / 64, batch, hkv * (d / 64) + 1);
+  transpose_v_kernel<true><<<grid, dim3(THREADS), 0, s>>>(v, vt, nullptr, nullptr, nullptr, vt_seq_stride, len, d,
+                                                         v_stride, vt_ld,
+                                                         PaddedPrep{key_mask, bits, seq_start, seq_len, words});
+  return hipGetLastError();
+}
+
+hipError_t dx_fill_unseen_launch(const AttnArgs &a, const uint8_t *key_mask, int num_q, int num_k, bool f32,
+                                 hipStream_t s) {
+  const dim3 grid((num_q + 63) / 64, a.num_seqs);
+  if (f32)
+    fill_unseen_kernel<<<grid, dim3(THREADS), 0, s>>>(static_cast<const float *>(a.v), static_cast<float *>(a.out),
+                                                     key_mask, a.max_seq_len, num_q, num_k, a.hq, a.hkv, a.d, a.v_stride,
+                                                     a.out_stride, a.window, a.causal);
+  else
+    fill_unseen_kernel<<<grid, dim3(THREADS), 0, s>>>(static_cast<const uint16_t *>(a.v), static_cast<uint16_t *>(a.out),
+                                                     key_mask, a.max_seq_len, num_q, num_k, a.hq, a.hkv, a.d, a.v_stride,
+                                                     a.out_stride, a.window, a.causal);
   return hipGetLastError();
 }

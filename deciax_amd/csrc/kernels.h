@@ -52,7 +52,7 @@ hipError_t dx_vt_zero_tails_launch(uint16_t *vt, const int32_t *seq_len, const i
 struct AttnArgs {
   const void *q, *k, *v;  // v: token-major (fp32 path) or transposed (bf16 path)
   void *out;
-  const int32_t *seq_start, *seq_len, *vt_start;
+  const int32_t *seq_start, *seq_len, *vt_start;  // fp32 path: null start and length for a padded batch
   int num_seqs, max_seq_len, hq, hkv, d;
   long q_stride, k_stride, v_stride, out_stride;  // v_stride = vt_ld on the bf16 path
   long vt_seq_stride;                              // used when vt_start == nullptr
@@ -70,6 +70,15 @@ hipError_t dx_pack_key_bits_launch(const uint8_t *key_mask, const int32_t *seq_s
 hipError_t dx_transpose_v_launch(const uint16_t *v, uint16_t *vt, const int32_t *seq_start, const int32_t *seq_len,
                                  const int32_t *vt_start, long vt_seq_stride, int num_seqs, int max_seq_len, int hkv,
                                  int d, long v_stride, long vt_ld, hipStream_t s);
+
+// Padded batch (sequence b = rows [b len, b len + len)): V^T as dx_transpose_v_launch leaves it, the mask as bits
+// (words 32-bit words a sequence) and the sequence descriptors, in one launch.
+hipError_t dx_prepare_padded_launch(const uint16_t *v, uint16_t *vt, const uint8_t *key_mask, uint32_t *bits,
+                                    int32_t *seq_start, int32_t *seq_len, int batch, int len, int words, int hkv, int d,
+                                    long v_stride, long vt_seq_stride, long vt_ld, hipStream_t s);
+// Rows below num_q that see no key of the first num_k: the mean of those keys' values (a.v token-major).
+hipError_t dx_fill_unseen_launch(const AttnArgs &a, const uint8_t *key_mask, int num_q, int num_k, bool f32,
+                                 hipStream_t s);
 
 hipError_t dx_rmsnorm_launch(const uint16_t *x, const uint16_t *w, uint16_t *y, const uint8_t *mask, long rows,
                              int d, long ldx, long ldy, float eps, hipStream_t s);

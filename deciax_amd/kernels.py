@@ -490,25 +490,6 @@ def attention_masked(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, key_mask
     return out
 
 
-def _visible_counts(mask: torch.Tensor, nq: int, causal: bool, window: int) -> torch.Tensor:
-    """[B, K] key mask -> [B, nq] number of keys each query row sees (index bookkeeping for the rows
-    that see none)."""
-    b, nk = mask.shape
-    cs = torch.nn.functional.pad(torch.cumsum(mask.to(torch.int32), dim=1), (1, 0))  # cs[:, j] = keys < j
-    i = torch.arange(nq, device=mask.device)
-    if causal:
-        hi = torch.clamp(i + 1, max=nk)
-        lo = torch.clamp(i - window + 1, min=0) if window > 0 else torch.zeros_like(i)
-    elif window > 0:
-        hi = torch.clamp(i + window + 1, max=nk)
-        lo = torch.clamp(i - window, min=0)
-    else:
-        hi = torch.full_like(i, nk)
-        lo = torch.zeros_like(i)
-    lo = torch.minimum(lo, hi)
-    return cs[:, hi] - cs[:, lo]
-
-
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, key_mask: torch.Tensor, *, causal: bool = False,
               window: int = 0, softcap: float = 0.0, scale: float | None = None) -> torch.Tensor:
     """[B, Q, H, D] queries against [B, K, Hkv, D] keys and values with a [B, K] key mask ->
@@ -557,29 +538,18 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, key_mask: torch
         vp = torch.zeros_like(kp)
         mp = torch.zeros((b, length), dtype=torch.bool, device=q.device)
         qp[:, :nq], kp[:, :nk], vp[:, :nk], mp[:, :nk] = q, k, v, mask
-    starts = torch.arange(b, device=q.device, dtype=torch.int32) * length
-    lengths = torch.full((b,), length, device=q.device, dtype=torch.int32)
-    rows = b * length
-    kw = dict(num_q_heads=hq, num_kv_heads=hkv, head_dim=d, scale=scale, softcap=softcap, window=window,
-              causal=causal)
-    args = (qp.reshape(rows, hq * d), kp.reshape(rows, hkv * d), vp.reshape(rows, hkv * d))
-    # Always the key-mask kernel: tiles whose keys the mask keeps run its unmasked body, so a full mask
-    # costs about what the maskless kernel does, bit for bit the same output, and asking whether the mask
-    # is full would stall the stream for a host round trip.
-    out = attention_masked(*args, mp.reshape(rows), starts, lengths, length, **kw)
-    out = out.reshape(b, length, hq, d)[:, :nq]
-    empty = _visible_counts(mask, nq, causal, window) == 0
-    if bool(empty.any()):
-        # softmax over K equal scores: the average of every value row, which the kernel computes for a
-        # zero query attending all K keys
-        kz = torch.zeros((b * nk, hq * d), dtype=q.dtype, device=q.device)
-        uniform = attention_varlen(kz, k.reshape(b * nk, hkv * d).contiguous(), v.reshape(b * nk, hkv * d).contiguous(),
-                                   torch.arange(b, device=q.device, dtype=torch.int32) * nk,
-                                   torch.full((b,), nk, device=q.device, dtype=torch.int32), nk, num_q_heads=hq,
-                                   num_kv_heads=hkv, head_dim=d, scale=scale, causal=False)
-        uniform = uniform.reshape(b, nk, hq, d)[:, :1].expand(b, nq, hq, d)
-        out = torch.where(empty[:, :, None, None], uniform, out)
-    return out.contiguous()
+    # The key-mask kernel always: tiles whose keys the mask keeps run its unmasked body, so a full mask costs about
+    # what the maskless kernel does. Rows that see no key are found and filled on the device. Nothing here asks the
+    # device for a value, which would stall the stream for a host round trip.
+    code = DX_BF16 if q.dtype == BF16 else DX_F32
+    out = torch.empty((b * length, hq * d), dtype=q.dtype, device=q.device)
+    ws_bytes = _lib.lib().dx_attn_padded_workspace(b, length, hkv, d, code)
+    ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=q.device)
+    qp, kp, vp = (t.reshape(b * length, h * d) for t, h in ((qp, hq), (kp, hkv), (vp, hkv)))
+    call("dx_attn_padded", _ptr(qp), _ptr(kp), _ptr(vp), _ptr(mp.contiguous().view(torch.uint8)), _ptr(out), b, length,
+         nq, nk, hq, hkv, d, _rows(qp, "q"), _rows(kp, "k"), _rows(vp, "v"), _rows(out, "out"), float(scale),
+         float(softcap), int(window), int(bool(causal)), code, _ptr(ws), ws.numel(), _stream())
+    return out.reshape(b, length, hq, d)[:, :nq].contiguous()
 
 
 FLASH_HEAD_DIM = 64  # the reference TPU kernel's fixed head size (pallas.py:18)

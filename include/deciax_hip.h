@@ -138,7 +138,7 @@ int dx_attn_prefill_noalloc(const void *q, const void *k, const void *v,
  * attention of src/deciax/kernels/attention/reference.py:11-42. Every query
  * row below seq_len is computed; a row that sees no key is written as zeros
  * (the reference returns the uniform average of all values there, an
- * artefact of the finite MASK_FILL; the Python layer restores it). Workspace
+ * artefact of the finite MASK_FILL; dx_attn_padded restores it). Workspace
  * size from dx_attn_prefill_masked_workspace (V^T plus the mask as bits). */
 int dx_attn_prefill_masked(const void *q, const void *k, const void *v,
                            const uint8_t *key_mask, void *out,
@@ -155,6 +155,26 @@ int dx_attn_prefill_masked(const void *q, const void *k, const void *v,
 int64_t dx_attn_prefill_masked_workspace(int32_t num_seqs, int32_t max_seq_len,
                                          int32_t num_kv_heads, int32_t head_dim,
                                          int32_t dtype);
+
+/* dx_attn_prefill_masked over a padded batch: sequence b is rows [b * len,
+ * (b + 1) * len) of q, k, v, out and key_mask, its first num_q rows are
+ * queries and its first num_k rows keys (the mask is 0 past them). A query
+ * row that sees no key gets what the reference's finite MASK_FILL gives it,
+ * the mean of the num_k value rows (blocked.py:23-27). Three launches at most
+ * and no host round trip. Workspace size from dx_attn_padded_workspace. */
+int dx_attn_padded(const void *q, const void *k, const void *v,
+                   const uint8_t *key_mask, void *out, int32_t batch,
+                   int32_t len, int32_t num_q, int32_t num_k,
+                   int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                   int64_t q_row_stride, int64_t k_row_stride,
+                   int64_t v_row_stride, int64_t out_row_stride, float scale,
+                   float softcap, int32_t window, int32_t causal,
+                   int32_t dtype, void *workspace, int64_t workspace_bytes,
+                   void *stream);
+
+int64_t dx_attn_padded_workspace(int32_t batch, int32_t len,
+                                 int32_t num_kv_heads, int32_t head_dim,
+                                 int32_t dtype);
 
 /* Same as dx_attn_prefill (bf16 only), with V already transposed: position
  * p of sequence s, kv head g, dim d at vt[(g * head_dim + d) * vt_ld +

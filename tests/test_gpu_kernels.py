@@ -582,6 +582,47 @@ def test_attention_arbitrary_key_mask(nq, nk, hq, hkv, d, causal, window, softca
             np.testing.assert_allclose(a[bi], want, rtol=1e-4, atol=1e-4)
 
 
+# (nq, nk, hq, hkv, d, causal, window, dtype): key masks below hide whole tiles of 64 rows, ends of windows and all
+# keys; nk below and above nq, one row, lengths off and on the 64-row tiles
+UNSEEN_CASES = [
+    (200, 200, 4, 2, 64, True, 0, "bf16"),
+    (193, 193, 4, 4, 128, True, 9, "bf16"),
+    (130, 64, 4, 1, 256, False, 5, "bf16"),
+    (64, 130, 8, 2, 64, False, 0, "bf16"),
+    (1, 65, 2, 2, 64, True, 0, "bf16"),
+    (200, 129, 4, 2, 128, True, 70, "f32"),
+    (129, 200, 2, 2, 256, False, 3, "f32"),
+]
+
+
+@pytest.mark.parametrize("nq,nk,hq,hkv,d,causal,window,dtype", UNSEEN_CASES)
+def test_attention_rows_that_see_no_key(nq, nk, hq, hkv, d, causal, window, dtype) -> None:
+    """Rows without a visible key take the mean of all values, the others the oracle's attention, under masks that
+    keep everything, nothing, a prefix, a suffix, one key, and runs with gaps wider than a window."""
+    from deciax_amd import kernels as K
+    from oracle.attention import attention_seq
+
+    say(f"attention unseen rows nq={nq} nk={nk} hq={hq} hkv={hkv} d={d} causal={causal} window={window} {dtype}")
+    r = rng(nq + 3 * nk + d)
+    j = np.arange(nk)
+    mask = np.stack([j >= 0, j < 0, j < nk // 3, j >= min(nk - 1, 66), j == nk // 2, (j // 17) % 3 == 1])
+    b = mask.shape[0]
+    q = r.normal(size=(b, nq, hq, d)).astype(np.float32)
+    k = r.normal(size=(b, nk, hkv, d)).astype(np.float32)
+    v = r.normal(size=(b, nk, hkv, d)).astype(np.float32)
+    if dtype == "bf16":
+        q, k, v = bf16_np(q), bf16_np(k), bf16_np(v)
+    got = to_np(K.attention(to_dev(q, dtype), to_dev(k, dtype), to_dev(v, dtype), i32(mask.astype(np.int32)),
+                            causal=causal, window=window))
+    for bi in range(b):
+        want = attention_seq(q[bi], k[bi], v[bi], scale=d ** -0.5, softcap_value=0.0, window=window, causal=causal,
+                             bf16=dtype == "bf16", key_mask=mask[bi], rounding="flash")
+        if dtype == "bf16":
+            close(got[bi], want, 2e-2)
+        else:
+            np.testing.assert_allclose(got[bi], want, rtol=1e-4, atol=1e-4)
+
+
 @pytest.mark.parametrize("b,s,heads,window,dtype", [(2, 200, 4, 0, "bf16"), (2, 257, 3, 32, "bf16"),
                                                      (1, 96, 2, 8, "f32")])
 def test_flash_attention_packed_interface(b: int, s: int, heads: int, window: int, dtype: str) -> None:
