@@ -244,6 +244,194 @@ linear_f32_kernel(const float *__restrict__ x, const float *__restrict__ w, cons
   }
 }
 
+// Large products: fp32 operands as sums of three bf16 (x = h + m + l, each the bf16 nearest to what is left: 24 bits
+// or more), multiplied by six bf16 MFMAs: h h into one fp32 accumulator, l h, h l, m m, m h, h m into another, 2^-8
+// of its size, so that one rounding per 16 k counts. What is left out (m l, l m, l l) is below 2^-25 of |x w|, less
+// than the rounding of an fp32 product. Error against 64 bits at k = 1024 / 4096: 1.3e-7 / 2.9e-7 (fp32 MFMAs in one
+// chain 4.0e-7 / 8.2e-7; both accumulators in one 3.4e-7 / 7.2e-7, 4% faster).
+// Tile (64 TM) x (64 TN) of 2 x 2 waves, 16 k per step. A step's fp32 chunks arrive in registers one step ahead, are
+// split once per workgroup and go to the other half of the LDS. What bounds it: the bf16 MFMAs, 6 / 16 of the cycles
+// of fp32 ones, at the rate the large bf16 GEMMs reach (1.2 PFLOP/s of them). Two register sets, or the split spread
+// between the MFMAs, measured the same or slower; 32 k per step 20% slower.
+// An infinity, a NaN or a value past the largest bf16 leaves its row or column of the accumulators not finite (inf -
+// inf): a wave that finds one multiplies its part again with fp32 MFMAs.
+DX_DEVICE void split3(const floatx4 &v, u32x2 (&p)[3]) {
+  float a[4] = {v[0], v[1], v[2], v[3]};
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t w = pack_bf2(a[2 * i], a[2 * i + 1]);
+      p[t][i] = w;
+      if (t < 2) {
+        a[2 * i] -= lo_bf(w);
+        a[2 * i + 1] -= hi_bf(w);
+      }
+    }
+  }
+}
+
+template <int TM, int TN>
+__global__ void __launch_bounds__(256, 2)
+linear_split_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
+                    float *__restrict__ y, long m, int n, int k, long ldx, long ldw, long ldy, int act, int acc_y,
+                    int vec_y) {
+  constexpr int BM = 64 * TM, BN = 64 * TN, ROWS = BM + BN, BK = 16;
+  constexpr int CPR = BK / 4, RPP = 256 / CPR;          // 16-byte chunks per row; rows per pass of the workgroup
+  constexpr int AP = BM / RPP, BP = BN / RPP;           // chunks per thread
+  // planes [h, m, l][k / 8][row][8]: fragment reads run over consecutive rows, and the two halves of a write's rows
+  // fall on different banks (+3% over [row][16])
+  constexpr int HALF = ROWS * 8 + 64, PLANE = 2 * HALF, STAGE = 3 * PLANE;  // bf16 elements
+  __shared__ __attribute__((aligned(1024))) uint16_t smem[2 * STAGE];
+
+  const int num_n = (n + BN - 1) / BN, nblocks = gridDim.x;
+  // each XCD (workgroups go round-robin over 8) takes a contiguous run of tiles, the tiles of one row block together
+  const int per = nblocks / 8, rem = nblocks % 8, xcd = blockIdx.x % 8, idx = blockIdx.x / 8;
+  const int tile = xcd < rem ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
+  const long m0 = (long)(tile / num_n) * BM;
+  const int n0 = tile % num_n * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1, lrow = lane & 31, lhalf = lane >> 5;
+  const int arows = (int)min((long)BM, m - m0), brows = min(BN, n - n0);
+  // rows past m and n read as zeros
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)(x + m0 * ldx), (short)0, (int)(((long)(arows - 1) * ldx + k) * 4), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)(w + (long)n0 * ldw), (short)0, (int)(((long)(brows - 1) * ldw + k) * 4), 0x00020000);
+  const int prow = tid / CPR, pc = tid % CPR;
+  const int xoff = (int)((prow * ldx + 4 * pc) * 4), woff = (int)((prow * ldw + 4 * pc) * 4);
+  const int xstep = (int)(RPP * ldx * 4), wstep = (int)(RPP * ldw * 4);
+  floatx4 st[AP + BP];
+  auto load = [&](int kk) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < AP; ++j)
+      st[j] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rx, xoff + j * xstep, kk * 4, 0));
+#pragma unroll
+    for (int j = 0; j < BP; ++j)
+      st[AP + j] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rw, woff + j * wstep, kk * 4, 0));
+  };
+  const int dst = pc / 2 * HALF + prow * 8 + pc % 2 * 4;
+  // chunks at k or past it (the next row's values) count as zeros: w's are cleared
+  auto put = [&](int stage, int kk) __attribute__((always_inline)) {
+    const bool live = kk + 4 * pc < k;
+#pragma unroll
+    for (int j = 0; j < AP + BP; ++j) {
+      floatx4 v = st[j];
+      if (j >= AP) v = live ? v : floatx4{0.f, 0.f, 0.f, 0.f};
+      u32x2 p[3];
+      split3(v, p);
+      uint16_t *d = smem + stage * STAGE + dst + (j < AP ? j * RPP : BM + (j - AP) * RPP) * 8;
+#pragma unroll
+      for (int t = 0; t < 3; ++t) *reinterpret_cast<u32x2 *>(d + t * PLANE) = p[t];
+    }
+  };
+  floatx16 c[TM][TN], small[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) c[i][j][r] = small[i][j][r] = 0.f;
+  auto mma = [&](int stage) __attribute__((always_inline)) {
+    const uint16_t *pa = smem + stage * STAGE + lhalf * HALF + (wm * 32 * TM + lrow) * 8;
+    const uint16_t *pb = smem + stage * STAGE + lhalf * HALF + (BM + wn * 32 * TN + lrow) * 8;
+    bf16x8 a[3][TM], b[3][TN];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a[t][i] = as_bf16x8(*reinterpret_cast<const u32x4 *>(pa + t * PLANE + 32 * i * 8));
+#pragma unroll
+      for (int j = 0; j < TN; ++j) b[t][j] = as_bf16x8(*reinterpret_cast<const u32x4 *>(pb + t * PLANE + 32 * j * 8));
+    }
+    constexpr int PA[6] = {0, 2, 0, 1, 1, 0}, PB[6] = {0, 0, 2, 1, 0, 1};
+#pragma unroll
+    for (int t = 0; t < 6; ++t)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          floatx16 &acc = t == 0 ? c[i][j] : small[i][j];
+          acc = mfma32(b[PB[t]][j], a[PA[t]][i], acc);
+        }
+  };
+  const int steps = (k + BK - 1) / BK;
+  load(0);
+  put(0, 0);
+  load(min(BK, (steps - 1) * BK));
+  __syncthreads();
+  for (int t = 0; t < steps; ++t) {
+    mma(t & 1);
+    put((t + 1) & 1, (t + 1) * BK);  // past the end: zeros or old chunks that nothing reads
+    load(min(t + 2, steps - 1) * BK);
+    __syncthreads();
+  }
+
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        c[i][j][r] += small[i][j][r];
+        bad = bad || !(fabsf(c[i][j][r]) < INFINITY);
+      }
+  if (__builtin_amdgcn_ballot_w64(bad)) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) c[i][j][r] = 0.f;
+    for (int k0 = 0; k0 < k; k0 += 2) {
+      const int kk = k0 + lhalf;
+      float a[TM], b[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+        a[i] = kk < k ? x[min(m0 + wm * 32 * TM + 32 * i + lrow, m - 1) * ldx + kk] : 0.f;
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        b[j] = kk < k ? w[(long)min(n0 + wn * 32 * TN + 32 * j + lrow, n - 1) * ldw + kk] : 0.f;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) c[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[j], a[i], c[i][j], 0, 0, 0);
+    }
+  }
+
+  // lane (lrow, lhalf) holds row 32 i + lrow, columns 32 j + 8 q + 4 lhalf + 0..3 in registers 4 q .. 4 q + 3
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const long row = m0 + wm * 32 * TM + 32 * i + lrow;
+    if (row >= m) continue;
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int col = n0 + wn * 32 * TN + 32 * j + 8 * q + 4 * lhalf;
+        float *out = y + row * ldy + col;
+        floatx4 v = {c[i][j][4 * q], c[i][j][4 * q + 1], c[i][j][4 * q + 2], c[i][j][4 * q + 3]};
+        if (vec_y && col + 4 <= n) {
+          if (bias) v += *reinterpret_cast<const floatx4 *>(bias + col);
+          if (act == 1) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = gelu_erf(v[e]);
+          }
+          if (acc_y) v += *reinterpret_cast<const floatx4 *>(out);
+          *reinterpret_cast<floatx4 *>(out) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if (col + e >= n) continue;
+            float s = v[e] + (bias ? bias[col + e] : 0.f);
+            if (act == 1) s = gelu_erf(s);
+            out[e] = acc_y ? out[e] + s : s;
+          }
+        }
+      }
+  }
+}
+
 // out[b * O + o, :] = mean of x[b * S + s, :] over s in [spans[b, o, 0], spans[b, o, 1]) (within
 // [0, S)); an empty span gives 0 (head.py:28 divides by max(count, 1)). One workgroup per span and 256 columns.
 __global__ void __launch_bounds__(THREADS)
@@ -664,6 +852,14 @@ static void linear_run(const float *x, const float *w, const float *bias, float 
   kern<<<grid, 64 * KW * WM * WN, 0, s>>>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc);
 }
 
+template <int TM, int TN>
+static void split_run(const float *x, const float *w, const float *bias, float *y, long m, int n, int k, long ldx,
+                      long ldw, long ldy, int act, int acc, hipStream_t s) {
+  const int vec_y = (ldy & 3) == 0 && ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(bias)) & 15) == 0;
+  linear_split_kernel<TM, TN><<<blocks(n, 64 * TN) * blocks(m, 64 * TM), 256, 0, s>>>(x, w, bias, y, m, n, k, ldx, ldw,
+                                                                                     ldy, act, acc, vec_y);
+}
+
 hipError_t dx_linear_f32_launch(const float *x, const float *w, const float *bias, float *y, long m, int n, int k,
                                 long ldx, long ldw, long ldy, int act, int acc, hipStream_t s) {
   // Each form's time is its rounds of waves over the 1024 SIMDs times a wave's share of one 64 x 64 x k product,
@@ -685,6 +881,23 @@ hipError_t dx_linear_f32_launch(const float *x, const float *w, const float *bia
   int best = 0;
   for (int i = 1; i < 6; ++i)
     if (cost[i] < cost[best]) best = i;
+  // In the same unit (71 us at k = 1024), the split forms: 128 x 128 tiles 46 us a round of 256 workgroups, 128 x 64
+  // tiles 27 us and 4 (us, the best of the above -> 128 x 128, 128 x 64):
+  //   600 x 2048 x 1024: 42 -> 47, 32      1200 x 2048 x 1024: 70 -> 50, 47    2000 x 1024 x 4096: 141 -> 162, 119
+  //   4096 x 1024 x 1024: 86 -> 57, 57     4096 x 2048 x 4096: 535 -> 350, 402 32768 x 1024 x 4096: 2093 -> 1375, 1584
+  //   512 x 2048 x 1024: 27 -> 47, 32      600 x 1024 x 4096: 70 -> 162, 105
+  // They read whole 16-byte chunks of a row through 32-bit offsets.
+  const bool chunks = k >= 64 && ((k | ldx | ldw) & 3) == 0 && ldx <= (1 << 20) && ldw <= (1 << 20) &&
+                      ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
+  if (chunks) {
+    const long wide = (tiles(128, 128) + 255) / 256, slim = (tiles(128, 64) + 255) / 256;
+    const double wide_cost = wide * (46 / 71.), slim_cost = (27 * slim + 4) / 71.;
+    if (fmin(wide_cost, slim_cost) < cost[best]) {
+      if (wide_cost <= slim_cost) split_run<2, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s);
+      else split_run<2, 1>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s);
+      return hipGetLastError();
+    }
+  }
   switch (best) {
     case 0: linear_run<4, 4, 1, 4, 1, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s); break;
     case 1: linear_run<4, 4, 2, 1, 1, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s); break;

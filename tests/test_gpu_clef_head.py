@@ -190,6 +190,61 @@ def test_linear_f32_tiles(m: int, n: int, k: int, pad: int) -> None:
     assert ((got - base.double() - act).abs() <= 1.2 * bound + 2.0 ** -21 * (act.abs() + base.double().abs()) + 1e-6).all()
 
 
+@pytest.mark.parametrize("m,n,k,pad,scale", [
+    (1300, 2000, 100, 4, 1.0), (4097, 1025, 132, 0, 1.0), (1281, 2050, 64, 8, 1e-30),   # 128 x 128 tiles
+    (600, 2048, 68, 0, 1.0), (577, 2049, 80, 4, 1e30), (641, 2047, 1028, 0, 1.0),       # 128 x 64 tiles
+])
+def test_linear_f32_split_tiles(m: int, n: int, k: int, pad: int, scale: float) -> None:
+    """The three-bf16 products at the edges of their tiles and of a 16-wide step, with bias, GELU and accumulation and
+    rows that hold NaN past k, against 64 bits. The six products leave out 2^-25 |x w|, and the two accumulators take
+    k / 16 and 5 k / 16 roundings, the second of terms 2^-8 the size: within the bound k 2^-24 sum |x w| of an fp32
+    sum, and its 2-norm within that of torch's fp32 product."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    say(f"linear_f32 split {m} x {n} x {k}, row padding {pad}, scale {scale}")
+    r = rng(m + n + k)
+    x = torch.as_tensor((r.normal(size=(m, k + pad)) * scale).astype(np.float32)).cuda()
+    w = torch.as_tensor(r.normal(size=(n, k + pad)).astype(np.float32)).cuda()
+    x[:, k:] = w[:, k:] = float("nan")
+    x, w = x[:, :k], w[:, :k]
+    b = torch.as_tensor((r.normal(size=n) * scale).astype(np.float32)).cuda()
+    want = x.double() @ w.double().t()
+    bound = (k + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + b.double().abs()) + 1e-38
+    got = K.linear_f32(x, w).double()
+    assert ((got - want).abs() <= bound).all()
+    assert (got - want).norm() <= ((x @ w.t()).double() - want).norm()
+    if scale != 1.0:
+        return
+    base = torch.as_tensor(r.normal(size=(m, n)).astype(np.float32)).cuda()
+    got = K.linear_f32(x, w, b, gelu=True, out=base.clone(), accumulate=True).double()
+    act = torch.nn.functional.gelu(want + b.double())
+    assert ((got - base.double() - act).abs() <= 1.2 * bound + 2.0 ** -21 * (act.abs() + base.double().abs()) + 1e-6).all()
+
+
+def test_linear_f32_split_not_finite() -> None:
+    """Infinities, NaN and values past the largest bf16 give what fp32 products give."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    say("linear_f32 split, values that are not finite")
+    r = rng(5)
+    m, n, k = 1300, 2000, 100
+    x = torch.as_tensor(r.normal(size=(m, k)).astype(np.float32)).cuda()
+    w = torch.as_tensor((r.normal(size=(n, k)) * 1e-3).astype(np.float32)).cuda()
+    x[3, 5], x[700, 99], x[1299, 0], w[17, 50], w[1999, 3] = np.inf, -np.inf, np.nan, np.inf, np.nan
+    x[40, 7] = x[1290, 64] = 3.395e38  # rounds to infinity in bf16
+    want = x.double() @ w.double().t()
+    got = K.linear_f32(x, w).double()
+    torch.testing.assert_close(got.isnan(), want.isnan())
+    torch.testing.assert_close(got.isinf(), want.isinf())
+    live = want.isfinite()
+    bound = (k + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    assert ((got - want).abs() <= bound)[live].all() and (got.sign() == want.sign())[want.isinf()].all()
+
+
 @pytest.mark.parametrize("batch,nq,nk,heads,dh", [
     (1, 1, 1, 1, 16), (2, 17, 65, 3, 32), (1, 6, 600, 16, 64), (2, 33, 130, 2, 48), (1, 5, 70, 2, 80), (1, 40, 64, 2, 96),
     (2, 20, 31, 2, 112), (1, 50, 515, 4, 128), (8, 40, 127, 40, 64), (1, 9, 40, 2, 24),
