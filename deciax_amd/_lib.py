@@ -97,6 +97,8 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "dx_linear_f32": (
         c_int, [_p, _p, _p, _p, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int32, c_int32, _p]),
     "dx_span_means_f32": (c_int, [_p, _p, _p, c_int32, c_int32, c_int32, c_int64, c_int64, c_int64, _p]),
+    "dx_span_means_gather_f32": (
+        c_int, [_p, _p, _p, _p, c_int32, c_int32, c_int32, c_int32, c_int64, c_int64, c_int64, _p]),
     "dx_mha_f32": (
         c_int,
         [_p, _p, _p, _p, _p, c_int32, c_int32, c_int32, c_int32, c_int32, c_int64, c_int64, c_int64, c_int64, _p],
@@ -110,6 +112,7 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
         [_p, _p, _p, _p, _p, _p, _p, _p, _p, c_int32, c_int32, c_int32, c_int32, c_int32, c_float, _p],
     ),
     "dx_head_combine_f32": (c_int, [_p, _p, _p, _p, _p, c_int64, c_float, c_float, _p]),
+    "dx_head_combine_scaled_f32": (c_int, [_p, _p, _p, _p, _p, _p, _p, _p, c_int64, _p]),
 }
 
 _LIB: ctypes.CDLL | None = None

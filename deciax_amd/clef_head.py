@@ -9,7 +9,6 @@ include/deciax_hip.h); torch only supplies the device buffers. Batched tensors t
 
 from __future__ import annotations
 
-import math
 from collections.abc import Mapping
 from pathlib import Path
 from typing import Any
@@ -19,7 +18,6 @@ import torch
 
 from deciax_amd import kernels as K
 
-MAX_LOGIT_SCALE = math.log(100.0)  # head.py:17
 EPS = 1e-5                         # head.py:20-21
 
 
@@ -41,10 +39,8 @@ def lexical_vectors(embedding: torch.Tensor, lexical_ids: Any, lexical_spans: An
     lexical_spans [B, O, 2] (how the reference builds `lexical`, tests/clef/test_head.py:16,
     with `means` of head.py:24-29). Returns [B, O, H] fp32."""
     ids = _dev(lexical_ids, torch.int32, embedding.device)
-    batch, seq = ids.shape
-    rows = K.gather_rows_f32(embedding, ids.reshape(1, batch * seq), batch=1)
     spans = _dev(lexical_spans, torch.int32, embedding.device)
-    return K.span_means_f32(rows, spans, batch=batch).reshape(batch, spans.shape[1], embedding.shape[1])
+    return K.span_means_gather_f32(embedding, ids, spans).reshape(ids.shape[0], spans.shape[1], embedding.shape[1])
 
 
 def forward(p: Mapping[str, torch.Tensor], hidden: Any, lexical: Any, a: Mapping[str, Any], *, heads: int,
@@ -118,12 +114,9 @@ def forward(p: Mapping[str, torch.Tensor], hidden: Any, lexical: Any, a: Mapping
         dense(ff, n + ".linear2", out=fields, accumulate=True)
 
     fields_o = K.gather_rows_f32(norm(fields, "field_norm"), owners, batch=batch)   # head.py:97-109
-    prior_scale = math.exp(min(float(p["prior_logit_scale"]), MAX_LOGIT_SCALE))
     features, prior, cosine = K.head_features_f32(fields_o, norm(options, "option_norm"), questions, global_vector,
-                                                  lex, owners, batch=batch, prior_scale=prior_scale)
+                                                  lex, owners, batch=batch, prior_scale=1.0)
     residual = dense(dense(features, "residual_scorer.0", gelu=True), "residual_scorer.3")
-    gate = 1.0 / (1.0 + math.exp(-float(p["residual_gate"])))
-    joint_scale = math.exp(min(float(p["joint_logit_scale"]), MAX_LOGIT_SCALE))
-    logits = K.head_combine_f32(prior, cosine, residual.reshape(-1), opt_mask.reshape(-1), gate=gate,
-                                joint_scale=joint_scale)
+    scalars = {n: _dev(p[n], torch.float32, dev) for n in ("prior_logit_scale", "joint_logit_scale", "residual_gate")}
+    logits = K.head_combine_scaled_f32(prior, cosine, residual.reshape(-1), opt_mask.reshape(-1), **scalars)
     return logits.reshape(batch, n_opt)

@@ -662,6 +662,18 @@ int dx_span_means_f32(const float *x, const int32_t *spans, float *out, int32_t 
                       "span_means launch");
 }
 
+int dx_span_means_gather_f32(const float *x, const int32_t *index, const int32_t *spans, float *out, int32_t batch,
+                             int32_t rows, int32_t seq, int32_t spans_per_row, int64_t d, int64_t ldx, int64_t ld_out,
+                             void *stream) {
+  REQUIRE(x && index && spans && out, "span_means_gather: null pointer argument");
+  REQUIRE(batch >= 0 && rows > 0 && seq > 0 && spans_per_row >= 0 && d > 0 && ldx >= d && ld_out >= d,
+          "span_means_gather: bad sizes");
+  if (batch == 0 || spans_per_row == 0) return DX_OK;
+  return check_launch(dx_span_means_gather_f32_launch(x, index, spans, out, batch, rows, seq, spans_per_row, (int)d, ldx,
+                                                      ld_out, as_stream(stream)),
+                      "span_means_gather launch");
+}
+
 int dx_mha_f32(const float *q, const float *k, const float *v, const uint8_t *key_mask, float *out, int32_t batch,
                int32_t num_queries, int32_t num_keys, int32_t heads, int32_t head_dim, int64_t ldq, int64_t ldk,
                int64_t ldv, int64_t ld_out, void *stream) {
@@ -733,5 +745,18 @@ int dx_head_combine_f32(const float *prior, const float *cosine, const float *re
   return check_launch(dx_combine_f32_launch(prior, cosine, residual, option_mask, logits, n, gate, joint_scale,
                                             as_stream(stream)),
                       "head_combine launch");
+}
+
+int dx_head_combine_scaled_f32(const float *prior, const float *cosine, const float *residual,
+                               const uint8_t *option_mask, const float *prior_logit_scale,
+                               const float *joint_logit_scale, const float *residual_gate, float *logits, int64_t n,
+                               void *stream) {
+  REQUIRE(prior && cosine && residual && option_mask && prior_logit_scale && joint_logit_scale && residual_gate && logits,
+          "head_combine_scaled: null pointer argument");
+  REQUIRE(n >= 0, "head_combine_scaled: bad size");
+  if (n == 0) return DX_OK;
+  return check_launch(dx_combine_scaled_f32_launch(prior, cosine, residual, option_mask, prior_logit_scale,
+                                                   joint_logit_scale, residual_gate, logits, n, as_stream(stream)),
+                      "head_combine_scaled launch");
 }
 

@@ -434,27 +434,33 @@ linear_split_kernel(const float *__restrict__ x, const float *__restrict__ w, co
 
 // out[b * O + o, :] = mean of x[b * S + s, :] over s in [spans[b, o, 0], spans[b, o, 1]) (within
 // [0, S)); an empty span gives 0 (head.py:28 divides by max(count, 1)). One workgroup per span and 256 columns.
+// With `index`, row s of batch row b is x[index[b * S + s]] of a table of R rows: 48653 ids over 4096 spans, width
+// 4096, take one pass over the rows they name (a gathered copy first: 346 us for it and 120 for its means).
+template <bool GATHER>
 __global__ void __launch_bounds__(THREADS)
-span_means_f32_kernel(const float *__restrict__ x, const int32_t *__restrict__ spans, float *__restrict__ out, int S,
-                      int O, int d, long ldx, long ldo) {
+span_means_f32_kernel(const float *__restrict__ x, const int32_t *__restrict__ index, const int32_t *__restrict__ spans,
+                      float *__restrict__ out, int R, int S, int O, int d, long ldx, long ldo) {
   const int bo = blockIdx.x, b = bo / O, i = blockIdx.y * THREADS + threadIdx.x;
   const int lo = max(spans[2 * bo], 0), hi = min(spans[2 * bo + 1], S);
   if (i >= d) return;
   const float inv = 1.0f / (float)max(hi - lo, 1);
-  const float *p = x + ((long)b * S + lo) * ldx + i;
+  auto row = [&](int s) __attribute__((always_inline)) {
+    if constexpr (GATHER) return (long)min(max(index[(long)b * S + s], 0), R - 1);
+    else return (long)b * S + s;
+  };
   float s = 0.f;
   int t = lo;
-  for (; t + 8 <= hi; t += 8, p += 8 * ldx) {  // eight rows in flight, added in order
+  for (; t + 8 <= hi; t += 8) {  // eight rows in flight, added in order
     float v[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = p[e * ldx];
+    for (int e = 0; e < 8; ++e) v[e] = x[row(t + e) * ldx + i];
 #pragma unroll
     for (int e = 0; e < 8; ++e) s += v[e];
   }
   if (t < hi) {
     float v[7];
 #pragma unroll
-    for (int e = 0; e < 7; ++e) v[e] = p[min(e, hi - 1 - t) * ldx];
+    for (int e = 0; e < 7; ++e) v[e] = x[row(min(t + e, hi - 1)) * ldx + i];
 #pragma unroll
     for (int e = 0; e < 7; ++e)
       if (t + e < hi) s += v[e];
@@ -825,6 +831,25 @@ combine_f32_kernel(const float *__restrict__ prior, const float *__restrict__ co
   out[i] = option_mask[i] ? prior[i] + gate * (joint_scale * cosine[i] + residual[i]) : -1e9f;
 }
 
+// The same with the learned scalars still on the device: out = prior_scale prior + gate (joint_scale cosine +
+// residual), scales exp(min(s, ln 100)) and gate sigmoid(g), each rounded once from double. Asking the host for them
+// stalled the forward three times.
+__global__ void __launch_bounds__(THREADS)
+combine_scaled_f32_kernel(const float *__restrict__ prior, const float *__restrict__ cosine,
+                          const float *__restrict__ residual, const uint8_t *__restrict__ option_mask,
+                          const float *__restrict__ prior_logit_scale, const float *__restrict__ joint_logit_scale,
+                          const float *__restrict__ residual_gate, float *__restrict__ out, long n) {
+  const long i = (long)blockIdx.x * THREADS + threadIdx.x;
+  if (i >= n) return;
+  auto scale = [](float v) {
+    const double most = 4.605170185988092;  // ln 100
+    return (float)exp((double)v > most ? most : (double)v);
+  };
+  const float ps = scale(*prior_logit_scale), js = scale(*joint_logit_scale);
+  const float gate = (float)(1.0 / (1.0 + exp(-(double)*residual_gate)));
+  out[i] = option_mask[i] ? ps * prior[i] + gate * (js * cosine[i] + residual[i]) : -1e9f;
+}
+
 unsigned blocks(long n, int per) { return (unsigned)((n + per - 1) / per); }
 
 }  // namespace
@@ -911,8 +936,15 @@ hipError_t dx_linear_f32_launch(const float *x, const float *w, const float *bia
 
 hipError_t dx_span_means_f32_launch(const float *x, const int32_t *spans, float *out, int B, int S, int O, int d,
                                     long ldx, long ldo, hipStream_t s) {
-  span_means_f32_kernel<<<dim3((unsigned)(B * O), blocks(d, THREADS)), THREADS, 0, s>>>(x, spans, out, S, O, d, ldx,
-                                                                                      ldo);
+  span_means_f32_kernel<false><<<dim3((unsigned)(B * O), blocks(d, THREADS)), THREADS, 0, s>>>(x, nullptr, spans, out, 0,
+                                                                                             S, O, d, ldx, ldo);
+  return hipGetLastError();
+}
+
+hipError_t dx_span_means_gather_f32_launch(const float *x, const int32_t *index, const int32_t *spans, float *out, int B,
+                                           int R, int S, int O, int d, long ldx, long ldo, hipStream_t s) {
+  span_means_f32_kernel<true><<<dim3((unsigned)(B * O), blocks(d, THREADS)), THREADS, 0, s>>>(x, index, spans, out, R, S,
+                                                                                            O, d, ldx, ldo);
   return hipGetLastError();
 }
 
@@ -993,5 +1025,15 @@ hipError_t dx_combine_f32_launch(const float *prior, const float *cosine, const 
                                  hipStream_t s) {
   combine_f32_kernel<<<blocks(n, THREADS), THREADS, 0, s>>>(prior, cosine, residual, option_mask, out, n, gate,
                                                             joint_scale);
+  return hipGetLastError();
+}
+
+hipError_t dx_combine_scaled_f32_launch(const float *prior, const float *cosine, const float *residual,
+                                        const uint8_t *option_mask, const float *prior_logit_scale,
+                                        const float *joint_logit_scale, const float *residual_gate, float *out, long n,
+                                        hipStream_t s) {
+  combine_scaled_f32_kernel<<<blocks(n, THREADS), THREADS, 0, s>>>(prior, cosine, residual, option_mask,
+                                                                  prior_logit_scale, joint_logit_scale, residual_gate,
+                                                                  out, n);
   return hipGetLastError();
 }

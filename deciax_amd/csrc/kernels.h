@@ -102,6 +102,8 @@ hipError_t dx_linear_f32_launch(const float *x, const float *w, const float *bia
                                 long ldx, long ldw, long ldy, int act, int acc, hipStream_t s);
 hipError_t dx_span_means_f32_launch(const float *x, const int32_t *spans, float *out, int B, int S, int O, int d,
                                     long ldx, long ldo, hipStream_t s);
+hipError_t dx_span_means_gather_f32_launch(const float *x, const int32_t *index, const int32_t *spans, float *out, int B,
+                                           int R, int S, int O, int d, long ldx, long ldo, hipStream_t s);
 hipError_t dx_mha_f32_launch(const float *q, const float *k, const float *v, const uint8_t *key_mask, float *out,
                              int B, int Q, int K, int H, int dh, long ldq, long ldk, long ldv, long ldo, hipStream_t s);
 hipError_t dx_gather_rows_f32_launch(const float *x, const int32_t *idx, float *y, int B, int R, int I, int d,
@@ -119,3 +121,7 @@ hipError_t dx_features_f32_launch(const float *fields, const float *opts, const 
 hipError_t dx_combine_f32_launch(const float *prior, const float *cosine, const float *residual,
                                  const uint8_t *option_mask, float *out, long n, float gate, float joint_scale,
                                  hipStream_t s);
+hipError_t dx_combine_scaled_f32_launch(const float *prior, const float *cosine, const float *residual,
+                                        const uint8_t *option_mask, const float *prior_logit_scale,
+                                        const float *joint_logit_scale, const float *residual_gate, float *out, long n,
+                                        hipStream_t s);

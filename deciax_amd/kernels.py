@@ -709,6 +709,21 @@ def span_means_f32(x: torch.Tensor, spans: torch.Tensor, *, batch: int) -> torch
     return out
 
 
+def span_means_gather_f32(table: torch.Tensor, index: torch.Tensor, spans: torch.Tensor) -> torch.Tensor:
+    """table [rows, d], index [batch, S], spans [batch, n, 2] -> [batch * n, d]: `span_means_f32` of the rows that
+    `gather_rows_f32` would copy."""
+    _f32(table, "table")
+    _need(index, "index", torch.int32, 2)
+    _need(spans, "spans", torch.int32, 3)
+    batch, n = index.shape[0], spans.shape[1]
+    if spans.shape[0] < batch or spans.shape[2] != 2:
+        raise ValueError("span_means_gather_f32: index must be [batch, S] and spans [batch, n, 2]")
+    out = torch.empty((batch * n, table.shape[1]), dtype=F32, device=table.device)
+    call("dx_span_means_gather_f32", _ptr(table), _ptr(index.contiguous()), _ptr(spans.contiguous()), _ptr(out), batch,
+         table.shape[0], index.shape[1], n, table.shape[1], _rows(table, "table"), _rows(out, "out"), _stream())
+    return out
+
+
 def mha_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, key_mask: torch.Tensor, *, batch: int,
             heads: int) -> torch.Tensor:
     """Masked multi-head attention core over [batch * n, heads * dh] rows (head.py:41-51)."""
@@ -808,6 +823,26 @@ def head_combine_f32(prior: torch.Tensor, cosine: torch.Tensor, residual: torch.
     out = torch.empty_like(prior)
     call("dx_head_combine_f32", _ptr(prior), _ptr(cosine), _ptr(residual), _ptr(option_mask), _ptr(out),
          prior.numel(), float(gate), float(joint_scale), _stream())
+    return out
+
+
+def head_combine_scaled_f32(prior: torch.Tensor, cosine: torch.Tensor, residual: torch.Tensor,
+                            option_mask: torch.Tensor, *, prior_logit_scale: torch.Tensor,
+                            joint_logit_scale: torch.Tensor, residual_gate: torch.Tensor) -> torch.Tensor:
+    """`head_combine_f32` of the unscaled prior, with the learned scalars (one fp32 element each) on the device."""
+    for t, n in ((prior, "prior"), (cosine, "cosine"), (residual, "residual")):
+        _need(t, n, F32, 1)
+    _need(option_mask, "option_mask", torch.uint8, 1)
+    if not prior.numel() == cosine.numel() == residual.numel() == option_mask.numel():
+        raise ValueError("head_combine_scaled_f32: one prior, cosine, residual and mask entry per option")
+    for t, n in ((prior_logit_scale, "prior_logit_scale"), (joint_logit_scale, "joint_logit_scale"),
+                 (residual_gate, "residual_gate")):
+        _need(t, n, F32)
+        if t.numel() != 1:
+            raise ValueError(f"head_combine_scaled_f32: {n} must hold one element, got shape {tuple(t.shape)}")
+    out = torch.empty_like(prior)
+    call("dx_head_combine_scaled_f32", _ptr(prior), _ptr(cosine), _ptr(residual), _ptr(option_mask),
+         _ptr(prior_logit_scale), _ptr(joint_logit_scale), _ptr(residual_gate), _ptr(out), prior.numel(), _stream())
     return out
 
 

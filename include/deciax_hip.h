@@ -410,6 +410,14 @@ int dx_span_means_f32(const float *x, const int32_t *spans, float *out,
                       int32_t batch, int32_t seq, int32_t spans_per_row,
                       int64_t d, int64_t ldx, int64_t ld_out, void *stream);
 
+/* The same over rows of a table: position s of batch row b is
+ * x[index[b * seq + s]], indices clamped to [0, rows). */
+int dx_span_means_gather_f32(const float *x, const int32_t *index,
+                             const int32_t *spans, float *out, int32_t batch,
+                             int32_t rows, int32_t seq, int32_t spans_per_row,
+                             int64_t d, int64_t ldx, int64_t ld_out,
+                             void *stream);
+
 /* Per batch row b, query i, head h: softmax over keys j (masked where
  * key_mask[b, j] == 0, at MASK_FILL) of q_i . k_j / sqrt(head_dim), times v.
  * The attention core of `mha`, src/deciax/models/clef/head.py:41-51, with the
@@ -467,6 +475,17 @@ int dx_head_combine_f32(const float *prior, const float *cosine,
                         const float *residual, const uint8_t *option_mask,
                         float *logits, int64_t n, float gate,
                         float joint_scale, void *stream);
+
+/* The same with the learned scalars read on the device (one float each):
+ * prior times exp(min(prior_logit_scale, ln 100)), gate and joint_scale from
+ * residual_gate and joint_logit_scale as above. */
+int dx_head_combine_scaled_f32(const float *prior, const float *cosine,
+                               const float *residual,
+                               const uint8_t *option_mask,
+                               const float *prior_logit_scale,
+                               const float *joint_logit_scale,
+                               const float *residual_gate, float *logits,
+                               int64_t n, void *stream);
 
 #ifdef __cplusplus
 }

@@ -245,6 +245,52 @@ def test_linear_f32_split_not_finite() -> None:
     assert ((got - want).abs() <= bound)[live].all() and (got.sign() == want.sign())[want.isinf()].all()
 
 
+@pytest.mark.parametrize("batch,rows,seq,n,d", [(1, 1, 1, 1, 1), (2, 50, 31, 7, 257), (3, 1000, 40, 20, 512)])
+def test_span_means_gather_f32(batch: int, rows: int, seq: int, n: int, d: int) -> None:
+    """Bit for bit the means of the gathered rows: empty and clipped spans, indices outside the table (clamped), rows
+    in blocks of eight and the rest."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    say(f"span_means_gather {batch} x {seq} of {rows} rows, {n} spans, width {d}")
+    r = rng(rows + d)
+    table = torch.as_tensor(r.normal(size=(rows, d)).astype(np.float32)).cuda()
+    ids = torch.as_tensor(r.integers(-2, rows + 2, (batch, seq)).astype(np.int32)).cuda()
+    lo = r.integers(-1, seq + 1, (batch, n))
+    spans = torch.as_tensor(np.stack([lo, lo + r.integers(-1, 19, (batch, n))], -1).astype(np.int32)).cuda()
+    copied = K.gather_rows_f32(table, ids.reshape(1, batch * seq), batch=1)
+    got = K.span_means_gather_f32(table, ids, spans)
+    assert torch.equal(got, K.span_means_f32(copied, spans, batch=batch))
+
+
+def test_head_combine_scaled_f32() -> None:
+    """The learned scalars on the device against the host's doubles, rounded once: capped and uncapped scales, both
+    signs of the gate. Three products and two sums of fp32: 4 2^-24 of the terms' size."""
+    import math
+
+    import torch
+
+    from deciax_amd import kernels as K
+
+    say("head_combine_scaled")
+    r = rng(3)
+    n = 300
+    prior, cosine, residual = (torch.as_tensor(r.normal(size=n).astype(np.float32)).cuda() for _ in range(3))
+    mask = torch.as_tensor((r.random(n) < 0.8).astype(np.uint8)).cuda()
+    for a, b, g in ((2.0, 2.5, 0.3), (4.605170, 7.0, -3.0), (80.0, -2.0, 40.0)):
+        ps, js = (np.float32(math.exp(min(float(np.float32(v)), math.log(100.0)))) for v in (a, b))
+        gate = np.float32(1.0 / (1.0 + math.exp(-float(np.float32(g)))))
+        t = [torch.tensor(v, device="cuda") for v in (a, b, g)]
+        got = K.head_combine_scaled_f32(prior, cosine, residual, mask, prior_logit_scale=t[0], joint_logit_scale=t[1],
+                                        residual_gate=t[2]).double().cpu().numpy()
+        p, c, x = (v.double().cpu().numpy() for v in (prior, cosine, residual))
+        want = float(ps) * p + float(gate) * (float(js) * c + x)
+        size = float(ps) * abs(p) + float(gate) * (float(js) * abs(c) + abs(x))
+        live = mask.cpu().numpy().astype(bool)
+        assert (abs(got - want) <= 4 * 2.0 ** -24 * size)[live].all() and (got[~live] == -1e9).all()
+
+
 @pytest.mark.parametrize("batch,nq,nk,heads,dh", [
     (1, 1, 1, 1, 16), (2, 17, 65, 3, 32), (1, 6, 600, 16, 64), (2, 33, 130, 2, 48), (1, 5, 70, 2, 80), (1, 40, 64, 2, 96),
     (2, 20, 31, 2, 112), (1, 50, 515, 4, 128), (8, 40, 127, 40, 64), (1, 9, 40, 2, 24),
