@@ -596,8 +596,12 @@ _OFFSETS: dict[int, tuple[weakref.ref, tuple[int, ...]]] = {}
 
 def offsets_tensor(values: Sequence[int], device: torch.device | str) -> torch.Tensor:
     """An int32 device copy of question offsets, remembered together with its host values."""
+    return remember_offsets(torch.as_tensor([int(v) for v in values], dtype=torch.int32).to(device), values)
+
+
+def remember_offsets(t: torch.Tensor, values: Sequence[int]) -> torch.Tensor:
+    """`t`, known from here on to hold the host values `values`."""
     host = tuple(int(v) for v in values)
-    t = torch.as_tensor(host, dtype=torch.int32).to(device)
     key = id(t)
     _OFFSETS[key] = (weakref.ref(t), host)
     weakref.finalize(t, _OFFSETS.pop, key, None)
