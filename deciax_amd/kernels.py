@@ -9,7 +9,6 @@ asynchronously on `torch.cuda.current_stream()`.
 
 from __future__ import annotations
 
-import ctypes
 import weakref
 from collections.abc import Sequence
 
@@ -23,18 +22,20 @@ F32 = torch.float32
 ACTIVATIONS = {"gelu_tanh": DX_ACT_GELU_TANH, "gelu_pytorch_tanh": DX_ACT_GELU_TANH, "silu": DX_ACT_SILU}
 
 
-def _ptr(t: torch.Tensor | None) -> ctypes.c_void_p | None:
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+def _ptr(t: torch.Tensor | None) -> int | None:
+    return None if t is None else t.data_ptr()
 
 
-def _stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+def _stream() -> int:
+    # the current device's current stream as a handle; torch.cuda.current_stream() builds a Stream object around it,
+    # which was a third of a launch's host time
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _need(t: torch.Tensor, name: str, dtype: torch.dtype, ndim: int | None = None) -> None:
     if not isinstance(t, torch.Tensor):
         raise ValueError(f"{name} must be a torch.Tensor")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{name} must be a device (HIP) tensor, got {t.device}")
     if t.dtype != dtype:
         raise ValueError(f"{name} must be {dtype}, got {t.dtype}")
