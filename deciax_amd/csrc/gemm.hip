@@ -6,11 +6,11 @@
 // wave owns a BM/2 x 128 quadrant in 32x32x16 MFMA blocks with fp32
 // accumulators (a single wave saturates the matrix core with this shape).
 //
-// Two kernels: gemm_nt_kernel, described here (256 x 256 tiles, which large M takes, and the 128-row tiles of the
-// residual-norm epilogue), and gemm_ring_kernel further down (smaller tiles, for launches that 256 x 256 tiles would
+// Two kernels: gemm_nt_kernel, described here (256 x 256 tiles, which large M takes, 192 x 256 ones where those fill
+// the CUs better, and the 128-row tiles of the residual-norm epilogue), and gemm_ring_kernel further down (smaller tiles, for launches that 256 x 256 tiles would
 // leave short of workgroups). dispatch() chooses by the tiles' rounds over the chip.
 //
-// Two data paths (256-row tiles, and 128-row tiles with K <= 8192, take the second):
+// Two data paths (256- and 192-row tiles, and 128-row tiles with K <= 8192, take the second):
 //
 // Register-staged. Per thread and K tile: 16-byte chunks arrive through buffer loads
 // (the resource is based at the tile origin, so rows past M read as zero and
@@ -176,12 +176,12 @@ gemm_nt_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, v
   constexpr int AC = BM * BK / 8 / THREADS, BC = BN * BK / 8 / THREADS;  // 16-byte chunks per thread
   constexpr int NC = AC + BC;
   constexpr int RATIO = NC / AC;  // chunk j is an A chunk iff j % RATIO == 0
-  static_assert(NC % 4 == 0 && NC % AC == 0, "chunk schedule");
+  static_assert(DTL || (NC % 4 == 0 && NC % AC == 0), "chunk schedule");
   constexpr int OUT_W = EPI == EPI_GATED ? BN / 2 : BN;
   constexpr int OUT_PITCH = OUT_W + 8;
-  // 256-row direct-to-LDS tiles use a ring of 3 A and 2 B stages (5 x 32 KB = the whole 160 KB)
-  constexpr bool RING = DTL && BM == 256;
-  constexpr int OPERANDS = RING ? 5 * BM * BK : 2 * STAGE;
+  // 256- and 192-row direct-to-LDS tiles use a ring of 3 A and 2 B stages (at 256 rows the whole 160 KB)
+  constexpr bool RING = DTL && BM >= 192;
+  constexpr int OPERANDS = RING ? (3 * BM + 2 * BN) * BK : 2 * STAGE;
   constexpr int SMEM = (OPERANDS > BM * OUT_PITCH) ? OPERANDS : BM * OUT_PITCH;
   // q|k|v epilogue: each tile row's clamped RoPE position and V^T column (2 BM int32) sit in LDS above
   // the staged tile (row-major BM x OUT_PITCH, or transposed BN x (BM + 8) for a V^T tile)
@@ -305,8 +305,9 @@ gemm_nt_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, v
     // With EB, B's second 4 loads all go in k-step 0 and A's 8 in k-steps 1 / 2 (4 / 4). The counter
     // drains in issue order, so the wait that makes B of tile T + 1 visible then leaves all 8 A loads
     // in flight, instead of waiting for A's first 4 as well: B gets about a k-step more to land.
-    static_assert(AI == 8 && BI == 8, "ring schedule: 8 A and 8 B instructions per wave");
-    constexpr int RS = BM * BK;  // elements per stage (A or B)
+    // 192-row tiles have 6 A loads: the third k-step then carries 2 (EB: the second and third 3 each).
+    static_assert((AI == 8 || AI == 6) && BI == 8, "ring schedule: 8 or 6 A and 8 B instructions per wave");
+    constexpr int RS = BM * BK, RSB = BN * BK;  // elements per stage of A, of B
     auto la = [&](int kt, int sa, int j0, int j1) __attribute__((always_inline)) {
 #pragma unroll
       for (int j = j0; j < j1; ++j) lds_load16(ra, smem + sa * RS + (wave * AI + j) * 512, aoff[j], kt * BK * 2);
@@ -314,11 +315,11 @@ gemm_nt_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, v
     auto lb = [&](int kt, int sb, int j0, int j1) __attribute__((always_inline)) {
 #pragma unroll
       for (int j = j0; j < j1; ++j)
-        lds_load16(rb, smem + (3 + sb) * RS + (wave * BI + j) * 512, boff[j], kt * BK * 2);
+        lds_load16(rb, smem + 3 * RS + sb * RSB + (wave * BI + j) * 512, boff[j], kt * BK * 2);
     };
     auto rdr = [&](bf16x8 *fa, bf16x8 *fb, int sa, int sb, int ks) __attribute__((always_inline)) {
       const uint16_t *pa = smem + sa * RS;
-      const uint16_t *pb = smem + (3 + sb) * RS;
+      const uint16_t *pb = smem + 3 * RS + sb * RSB;
       const int c = ks * 2 + lhalf;
 #pragma unroll
       for (int i = 0; i < TM; ++i)
@@ -327,23 +328,23 @@ gemm_nt_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, v
       for (int j = 0; j < TN; ++j)
         fb[j] = as_bf16x8(*reinterpret_cast<const u32x4 *>(pb + swz(wn * (BN / 2) + j * 32 + lrow, c)));
     };
-    constexpr int DR0 = 6;  // fragment reads in MFMA slots 6..13
+    constexpr int DR0 = BM == 256 ? 6 : 5;  // fragment reads in MFMA slots 6..13 (192 rows: 5..11)
     static_assert(DR0 + NR <= NM, "ring region schedule");
 #define DX_RREGION()                                                                               \
   do {                                                                                             \
     _Pragma("unroll") for (int t = 0; t < NM; ++t) {                                               \
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                           \
-      if (t % 4 == 0) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                           \
+      if (t % (NM / 4) == 0) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                    \
       if (t >= DR0 && t - DR0 < NR) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);             \
     }                                                                                              \
   } while (0)
     auto cl = [&](int t) { return min(t, KT - 1); };  // past the end: reload the last tile into a freed stage
     // tiles 0 and 1 of A, tile 0 of B and the loads of B tile 1 that precede iteration 0
-    la(0, 0, 0, 8);
+    la(0, 0, 0, AI);
     lb(0, 0, 0, 8);
-    la(cl(1), 1, 0, 8);
+    la(cl(1), 1, 0, AI);
     lb(cl(1), 1, 0, 4);
-    asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AI + 4) : "memory");
     __syncthreads();
     rdr(fa0, fb0, 0, 0, 0);
     // Iteration kt (q = kt % 6 at compile time, so every stage is an immediate).
@@ -362,7 +363,7 @@ gemm_nt_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, v
       DX_RREGION();
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (EB) {
-        la(cl(kt + 2), sa2, 0, 4);
+        la(cl(kt + 2), sa2, 0, AI / 2);
       } else {
         lb(cl(kt + 1), sb1, 6, 8);
         la(cl(kt + 2), sa2, 2, 4);
@@ -371,15 +372,14 @@ gemm_nt_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, v
       mm(fa1, fb1);
       DX_RREGION();
       __builtin_amdgcn_sched_barrier(0);
-      la(cl(kt + 2), sa2, 4, 8);
+      la(cl(kt + 2), sa2, EB ? AI / 2 : 4, AI);
       rdr(fa1, fb1, sa, sb, 3);
       mm(fa0, fb0);
       DX_RREGION();
       __builtin_amdgcn_sched_barrier(0);
-      // A and B of tile kt + 1 have landed (younger loads: this k-step's 4, or with EB the 8 of A's tile
+      // A and B of tile kt + 1 have landed (younger loads: this k-step's, or with EB all of A's tile
       // kt + 2), and every wave is done with tile kt, whose stages the next loads refill
-      if constexpr (EB) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(EB ? AI : AI - 4) : "memory");
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
       lb(cl(kt + 2), sb, 0, 4);
@@ -948,17 +948,17 @@ hipError_t launch(const uint16_t *A, const uint16_t *B, void *C, long M, long N,
                   long ldc, int act, const QkvEpilogue &qe, const NormEpilogue &ne, hipStream_t s) {
   const long num_m = (M + BM - 1) / BM, num_n = N / BN_NT;
   const bool weight_cached = N * K * 2 <= (256L << 20);  // the weight fits the 256 MB Infinity Cache
-  // 256-row tiles always take the direct-to-LDS ring: its A stages give long-K shapes the latency slack
+  // 256- and 192-row tiles always take the direct-to-LDS ring: its A stages give long-K shapes the latency slack
   // (against the register-staged path: down K 14336 +3-8 % alone and -0.8 % step time in the 9B
   // forward, K 36864 +4.5 %, 1344- and 448-tile down shapes +2.5 % / +1 %). 128-row tiles (the
   // residual-norm epilogue up to 1024 rows) have two stages only, so long K keeps the register-staged path and its two tiles of slack there.
   auto kern = gemm_nt_kernel<BM, EPI, true>;
-  if constexpr (BM != 256)
+  if constexpr (BM < 192)
     if (K > 8192) kern = gemm_nt_kernel<BM, EPI, false>;
   // The early-B order of the ring gains where the weight fits the 256 MB Infinity Cache (9B forward: gate|up
   // +2.8%, down +1.9%, q|k|v +1.2%, step -1.7%) and loses where it does not (27B gate|up and down, 680 and
   // 340 MB: -3% each); bit-identical either way.
-  if constexpr (BM == 256)
+  if constexpr (BM >= 192)
     if (weight_cached) kern = gemm_nt_kernel<BM, EPI, true, true>;
   // Tile rows walked together per XCD. Long K: an A row tile is megabytes, and groups of 8 re-read it
   // once per 4 column tiles. So 1 row when the weight fits the Infinity Cache, where the weight's
@@ -995,6 +995,9 @@ hipError_t launch_ring(const uint16_t *A, const uint16_t *B, void *C, long M, lo
 //   3584 x 14336:  M 64 156 -> 38   M 200 156 -> 52   M 517 182 -> 89    M 1300 232 -> 149   M 3300 276 (unchanged)
 //   28672 x 3584:  M 64  75 -> 40   M 200  75 -> 57   M 517 182 -> 128   M 1000 254 -> 162
 //   8192 x 3584:   M 64  47 -> 17   M 200  68 -> 24   M 517  66 -> 41    M 1000  64 -> 55
+// 192 x 256 (plain epilogues; a quarter fewer rows a tile where 256 x 256 leaves part of a round idle), us:
+//   3584 x 14336:  M 5000 550 -> 479, M 3000 260 -> 253     4608 x 4096: M 2000 80 -> 74, M 4000 167 -> 146
+//   4608 x 36864:  M 4096 1561 -> 1449, M 2000 708 -> 694
 struct TileForm {
   int bm, bn;
 };
@@ -1015,12 +1018,12 @@ hipError_t dispatch(const uint16_t *A, const uint16_t *B, void *C, long M, long 
     constexpr bool PAIRED = EPI == EPI_GATED || EPI == EPI_QKV;
     // 256 x 256 first, then the ring forms of this epilogue (paired ones need an even TN, so they lack the
     // narrowest); q|k|v tiles must not straddle the end of the q|k columns
-    static const TileForm forms[] = {{256, 256}, {256, 128}, {192, 128}, {128, 128}, {96, 128}, {64, 128},
-                                     {128, 64},  {64, 64},   {192, 64},  {96, 64},   {64, 32},  {32, PAIRED ? 64 : 32}};
+    static const TileForm forms[] = {{256, 256}, {256, 128}, {192, 128}, {128, 128}, {96, 128}, {64, 128}, {128, 64},
+                                     {64, 64},   {192, 64},  {96, 64},   {64, 32},   {32, PAIRED ? 64 : 32}, {192, 256}};
     int best = 0;
     double least = tile_cost(forms[0], M, N);
-    for (int i = 1; i < 12; ++i) {
-      if (PAIRED && i >= 8 && i <= 10) continue;
+    for (int i = 1; i < 13; ++i) {
+      if (PAIRED && ((i >= 8 && i <= 10) || i == 12)) continue;
       if (EPI == EPI_QKV && qe.qk_cols % forms[i].bn) continue;
       const double c = tile_cost(forms[i], M, N);
       if (c < least) {
@@ -1046,6 +1049,7 @@ hipError_t dispatch(const uint16_t *A, const uint16_t *B, void *C, long M, long 
         case 9: DX_RING(3, 1, 1, 2, 7);
         case 10: DX_RING(1, 1, 2, 1, 6);
         case 11: DX_RING(1, 1, 1, 1, 8);
+        case 12: return launch<192, EPI>(A, B, C, M, N, K, lda, ldb, ldc, act, qe, ne, s);
       }
     }
 #undef DX_RING

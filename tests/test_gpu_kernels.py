@@ -1060,6 +1060,23 @@ def test_gemm_tile_forms_agree(k: int) -> None:
                 assert torch.equal(K.gated_linear(a[:m], w, act), y[:m]), f"gated M={m} N={n} K={k} {act}"
 
 
+def test_gemm_192_row_tiles_large_weight() -> None:
+    """192 x 256 tiles over a weight beyond the last-level cache (its own order of loads) give each row what smaller
+    launches, in other forms, give it."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    m, n, k = 2050, 4608, 29184  # 272 MB of weight; 456 64-deep tiles, a whole number of the loop's six
+    say(f"GEMM 192-row tiles, large weight: {m} x {n} x {k}")
+    g = torch.Generator(device="cuda").manual_seed(1)
+    a, w = (torch.empty((rows, k), dtype=torch.bfloat16, device="cuda").normal_(0, 0.1, generator=g) for rows in (m, n))
+    for kk in (k, k - 64):
+        got = K.linear(a[:, :kk], w[:, :kk])
+        assert torch.equal(got[:1000], K.linear(a[:1000, :kk], w[:, :kk]))
+        assert torch.equal(got[1050:], K.linear(a[1050:, :kk], w[:, :kk]))
+
+
 @pytest.mark.parametrize("hq,hkv,d", [(16, 8, 256), (32, 16, 128), (2, 1, 64), (6, 3, 64)])
 def test_qkv_rope_tile_forms_agree(hq: int, hkv: int, d: int) -> None:
     """Every tile form of the q|k|v projection equals linear -> rope -> transpose_v bit for bit (head counts whose
