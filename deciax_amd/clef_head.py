@@ -93,8 +93,12 @@ def forward(p: Mapping[str, torch.Tensor], hidden: Any, lexical: Any, a: Mapping
         """out += mha(query, memory) (head.py:41-51): in_proj split in q | k | v rows."""
         w, b = p[name + ".in_proj_weight"], p[name + ".in_proj_bias"]
         width = query.shape[1]
-        q = K.linear_f32(query, w[:width], b[:width])
-        kv = K.linear_f32(memory, w[width:], b[width:])
+        if query is memory:  # self-attention: one projection
+            qkv = K.linear_f32(query, w, b)
+            q, kv = qkv[:, :width], qkv[:, width:]
+        else:
+            q = K.linear_f32(query, w[:width], b[:width])
+            kv = K.linear_f32(memory, w[width:], b[width:])
         att = K.mha_f32(q, kv[:, :width], kv[:, width:], key_mask, batch=batch, heads=heads)
         return dense(att, name + ".out_proj", out=out, accumulate=True)
 

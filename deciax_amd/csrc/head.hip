@@ -41,6 +41,21 @@ DX_DEVICE float block_sum(float v, float *red) {
   __syncthreads();
   return red[0] + red[1] + red[2] + red[3];
 }
+// Several sums at once: two barriers for all of them.
+template <int N>
+DX_DEVICE void block_sums(float (&v)[N], float (*red)[THREADS / 64]) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = wave_reduce_sum(v[i]);
+  __syncthreads();
+  if (lane == 0) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) red[i][w] = v[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = red[i][0] + red[i][1] + red[i][2] + red[i][3];
+}
 DX_DEVICE float block_max(float v, float *red) {
   v = wave_reduce_max(v);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -783,38 +798,44 @@ features_f32_kernel(const float *__restrict__ fields, const float *__restrict__ 
                     const float *__restrict__ glob, const float *__restrict__ lexical, const int32_t *__restrict__ owner,
                     float *__restrict__ features, float *__restrict__ prior, float *__restrict__ cosine, int O, int NQ,
                     int W, int Hd, float prior_scale) {
-  __shared__ float red[4];
+  __shared__ float red[4][THREADS / 64];
   const int bo = blockIdx.x, b = bo / O;
   const int qi = min(max(owner[bo], 0), NQ - 1);
   const float *qr = questions + ((long)b * NQ + qi) * Hd, *gr = glob + (long)b * Hd, *lr = lexical + (long)bo * Hd;
-  float sa = 0.f, sl = 0.f;
-  for (int i = threadIdx.x; i < Hd; i += THREADS) {
-    const float a = qr[i] + gr[i];
-    sa += a * a;
-    sl += lr[i] * lr[i];
-  }
-  const float ia = inv_length(block_sum(sa, red), 1e-12f), il = inv_length(block_sum(sl, red), 1e-12f);
-  float dp = 0.f;
-  for (int i = threadIdx.x; i < Hd; i += THREADS) dp += (lr[i] * il) * ((qr[i] + gr[i]) * ia);
-  dp = block_sum(dp, red);
   const float *fr = fields + (long)bo * W, *orow = opts + (long)bo * W;
-  float sf = 0.f, so = 0.f;
-  for (int i = threadIdx.x; i < W; i += THREADS) {
-    sf += fr[i] * fr[i];
-    so += orow[i] * orow[i];
+  // Two passes with one reduction each (one value at a time they took six, 11.6 us for 23 options): the lengths, then
+  // the two products with the features.
+  float len[4] = {0.f, 0.f, 0.f, 0.f};  // of the anchor, the label vector, the field and the option
+#pragma unroll 4
+  for (int i = threadIdx.x; i < Hd; i += THREADS) {
+    const float a = qr[i] + gr[i], l = lr[i];
+    len[0] += a * a;
+    len[1] += l * l;
   }
-  const float jf = inv_length(block_sum(sf, red), 1e-8f), jo = inv_length(block_sum(so, red), 1e-8f);
-  float cs = 0.f;
-  float *ft = features + (long)bo * 4 * W;
+#pragma unroll 4
   for (int i = threadIdx.x; i < W; i += THREADS) {
     const float f = fr[i], o = orow[i];
-    cs += (f * jf) * (o * jo);
+    len[2] += f * f;
+    len[3] += o * o;
+  }
+  block_sums(len, red);
+  const float ia = inv_length(len[0], 1e-12f), il = inv_length(len[1], 1e-12f);
+  const float jf = inv_length(len[2], 1e-8f), jo = inv_length(len[3], 1e-8f);
+  float dots[2] = {0.f, 0.f};
+#pragma unroll 4
+  for (int i = threadIdx.x; i < Hd; i += THREADS) dots[0] += (lr[i] * il) * ((qr[i] + gr[i]) * ia);
+  float *ft = features + (long)bo * 4 * W;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < W; i += THREADS) {
+    const float f = fr[i], o = orow[i];
+    dots[1] += (f * jf) * (o * jo);
     ft[i] = f;
     ft[W + i] = o;
     ft[2 * W + i] = f * o;
     ft[3 * W + i] = fabsf(f - o);
   }
-  cs = block_sum(cs, red);
+  block_sums(dots, red);
+  const float dp = dots[0], cs = dots[1];
   if (threadIdx.x == 0) {
     prior[bo] = dp * prior_scale;
     cosine[bo] = cs;
