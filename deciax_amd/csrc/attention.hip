@@ -48,7 +48,7 @@ constexpr int BKV = 64;     // V^T block alignment of dx_transpose_v
 // Head_dim 128 takes the short form when a query row sees 2048 keys or fewer on average (window <= 2048,
 // or causal sequences up to 4096): 27B heads, 8 x 2048 -4%, window 512 -12 to -15%, window 1024 -5 to
 // -10%, 16 x 3400 -2%; on longer spans it measured +0.2 to +1.1% (4 x 16384). Head_dim 64 takes it up to 4096
-// keys: its 32 KB ring puts two workgroups on a CU too, and half the query rows spread small launches further
+// keys: its 32 KB ring puts three workgroups on a CU, and half the query rows spread small launches further
 // (12 heads: 2 x 1021 35 -> 30 us, 4 x 2048 83 -> 72, 1 x 2048 42 -> 32, 8 x 1021 49 -> 47; 4 x 8192 +2.8%).
 // Head_dim 256: the short form measured 6-11% slower. Where the long one has at most a workgroup per CU, four waves
 // over the same 4-stage ring (one per SIMD) halve what the longest workgroup has to do: 16/8 heads, 1 x 736 40 -> 31
@@ -139,8 +139,17 @@ struct Flag {
 // KM: a per-key mask (key_bits, key_words 32-bit words per sequence; bit j of word w of sequence b is key
 // 32 w + j) hides keys beyond the causal / window rule. Tiles that hold a masked key take the masked body,
 // and a query row that sees no key is written as zeros.
+// Waves per SIMD that the registers are kept for: what the ring lets a CU hold. Head_dim 64's short form (32 KB) runs
+// three, 136 registers a lane for 169: its loop waits on exponentials and LDS more than on the matrix core. 12 heads,
+// 8 x 1021 68 -> 59 us; 16 heads, 12 x 2048 312 -> 289, window 64 94 -> 80; four measured like three.
+constexpr int waves_least(int d, int waves, int stages) {
+  return waves * stages == 16 ? 1 : d == 64 && waves == 4 ? 3 : 2;
+}
+constexpr int waves_most(int d, int waves, int stages) { return d == 64 && waves == 4 && stages == 2 ? 3 : 2; }
+
 template <int D, int G, int MODE, bool KM, int WAVES, int NSTAGE>
-__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES * NSTAGE == 16 ? 1 : 2, 2)))
+__global__ void __launch_bounds__(64 * WAVES)
+__attribute__((amdgpu_waves_per_eu(waves_least(D, WAVES, NSTAGE), waves_most(D, WAVES, NSTAGE))))
 attn_bf16_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ Vt,
                  uint16_t *__restrict__ O, const int32_t *__restrict__ seq_start,
                  const int32_t *__restrict__ seq_len, const int32_t *__restrict__ vt_start, long vt_seq_stride,
