@@ -282,8 +282,6 @@ attn_bf16_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
 
   const float c2inv = 1.f / (-2.f * LOG2E * softcap);
   const float c3 = 0.5f * LOG2E * softcap;
-  // running-max form: scores (soft-capped ones carry the scale already) to log2 units
-  const float to_log2 = MODE == MODE_CAP ? LOG2E : scale * LOG2E;
 
   // Which 32-key blocks this wave's rows see: active = some key visible, masked = some key hidden.
   auto block_state = [&](const int kbase, bool &need_mask) {
@@ -307,20 +305,6 @@ attn_bf16_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
     vhi = window > 0 ? min(qi + window, len - 1) : len - 1;
     vlo = window > 0 ? qi - window : 0;
   }
-
-  // Running-max form: the row's maximum (its 32-key halves sit in lanes l and l ^ 32) joins mrun, and O follows.
-  auto raise_max = [&](const float tmax) __attribute__((always_inline)) {
-    const float mnew = fmaxf(mrun, fmaxf(tmax, __shfl_xor(tmax, 32, 64)));
-    if (__builtin_amdgcn_ballot_w64(mnew != mrun)) {
-      const float alpha = fast_exp2(mrun - mnew);
-      mrun = mnew;
-      lsum *= alpha;
-#pragma unroll
-      for (int i = 0; i < NDB; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
-    }
-  };
 
   // One 32-key block kb of the tile in stage sk (K, then V^T at sk + KST): S^T = K Q^T, softmax,
   // O^T += V^T P^T. MASKED evaluates the causal / window / length mask and skips blocks no row sees.
@@ -363,24 +347,39 @@ attn_bf16_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
         lsum += p;
       }
     } else {
-      if constexpr (MODE == MODE_CAP) {
+      // The maximum is raised once per 32-key block and P rounded against it, so outputs depend on that step (64 keys
+      // under one maximum: 4 x 2048 172 us for 183, outputs moved by 1e-3 of their size). What rounds where is spelled
+      // out, so that no change of the code around it moves them: interior blocks round the exponent once, in the fma,
+      // masked ones after each operation, which changes a P in some 1e5 by its last bit.
+#pragma clang fp contract(off)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = softcap * tanhf(s[r] * scale / softcap);
+      for (int r = 0; r < 16; ++r) {
+        s[r] *= scale;
+        if constexpr (MODE == MODE_CAP) s[r] = softcap * tanhf(s[r] / softcap);
       }
-      float smax = NEG_BIG;
+      float smax = -INFINITY;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         if constexpr (M) smax = keep(r) ? fmaxf(smax, s[r]) : smax;
         else smax = fmaxf(smax, s[r]);
       }
-      const float tmax = fmaxf(smax * to_log2, NEG_BIG);
-      raise_max(tmax);
+      const float tmax = fmaxf(smax * LOG2E, NEG_BIG);
+      const float mnew = fmaxf(mrun, fmaxf(tmax, __shfl_xor(tmax, 32, 64)));
+      const float alpha = fast_exp2(mrun - mnew);
+      if (__builtin_amdgcn_ballot_w64(mnew != mrun)) {  // else alpha is 1 for all 32 rows
+#pragma unroll
+        for (int i = 0; i < NDB; ++i)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
+      }
+      mrun = mnew;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        float p = fast_exp2(__builtin_fmaf(s[r], to_log2, -mrun));
-        if constexpr (M) p = keep(r) ? p : 0.f;
+        float p;
+        if constexpr (M) p = keep(r) ? fast_exp2(s[r] * LOG2E - mnew) : 0.f;
+        else p = fast_exp2(__builtin_fmaf(s[r], LOG2E, -mnew));
         s[r] = p;
-        lsum += p;
+        lsum = r == 0 ? __builtin_fmaf(lsum, alpha, p) : lsum + p;
       }
     }
     bf16x8 pf[2];
@@ -403,65 +402,13 @@ attn_bf16_kernel(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
     stream_sched<2 * NDB>();
   };
 
-  // Both blocks of a 64-key tile without masked keys, running-max form: one maximum and one pass over O for the
-  // tile. The softmax's vector instructions bound this form, and that pass was a third of them (head_dim 128).
-  auto tile64 = [&](const uint16_t *sk) __attribute__((always_inline)) {
-    floatx16 s[2];
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[kb][r] = 0.f;
-      const int krow = kb * 32 + kperm(lrow);
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) {
-        const int lo = ((ks * 2 + lhalf) ^ k_swz<D>(krow)) << 3;
-        s[kb] = mfma32(as_bf16x8(*reinterpret_cast<const u32x4 *>(sk + krow * D + lo)), qf[ks], s[kb]);
-      }
-    }
-    stream_sched<2 * NKS>();
-    float smax = NEG_BIG;
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) smax = fmaxf(smax, s[kb][r]);
-    raise_max(fmaxf(smax * to_log2, NEG_BIG));
-    bf16x8 pf[4];
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        s[kb][r] = fast_exp2(__builtin_fmaf(s[kb][r], to_log2, -mrun));
-        lsum += s[kb][r];
-      }
-#pragma unroll
-      for (int h2 = 0; h2 < 2; ++h2) {
-        u32x4 w;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) w[i] = pack_bf2(s[kb][8 * h2 + 2 * i], s[kb][8 * h2 + 2 * i + 1]);
-        pf[2 * kb + h2] = as_bf16x8(w);
-      }
-    }
-    const uint16_t *sv = sk + KST;
-#pragma unroll
-    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-      for (int h2 = 0; h2 < 4; ++h2)
-        o[db] = mfma32(as_bf16x8(*reinterpret_cast<const u32x4 *>(sv + vt_off<TK>(db * 32 + lrow, 2 * h2 + lhalf))),
-                       pf[h2], o[db]);
-    stream_sched<4 * NDB>();
-  };
-
   // Ring of NSTAGE tiles: tile kt sits in stage (kt - kt0) % NSTAGE, and tile kt + NSTAGE - 1 is
   // fetched while tile kt is multiplied (clamped: the last tiles reload themselves harmlessly).
   auto tile = [&](const int kt, auto masked) {
     issue(min(kt + NSTAGE - 1, kt1 - 1), (kt - kt0 + NSTAGE - 1) % NSTAGE);
     const uint16_t *sk = smem + ((kt - kt0) % NSTAGE) * STAGE;
-    if constexpr (MODE == MODE_ONLINE && TK == 64 && !decltype(masked)::value) {
-      tile64(sk);
-    } else {
 #pragma unroll
-      for (int kb = 0; kb < TK / 32; ++kb) block(sk, kt * TK + kb * 32, kb, masked);
-    }
+    for (int kb = 0; kb < TK / 32; ++kb) block(sk, kt * TK + kb * 32, kb, masked);
     // tile kt + 1 has landed in every wave's share (the NSTAGE - 2 younger tiles may stay in flight)
     // and every wave is done reading tile kt, whose stage the next iteration refills. A plain s_barrier:
     // __syncthreads would also wait for the younger tiles' loads (its fence waits for all LDS writes).

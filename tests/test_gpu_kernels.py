@@ -424,6 +424,57 @@ def test_attention_fp32_config1() -> None:
     np.testing.assert_allclose(got[0], want, rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("d,hq,hkv,causal,softcap", [(64, 4, 4, False, 0.0), (128, 4, 2, True, 0.0), (128, 2, 1, False, 80.0),
+                                                    (256, 2, 1, False, 0.0)])
+def test_attention_running_max_per_32_keys(d: int, hq: int, hkv: int, causal: bool, softcap: float) -> None:
+    """P is rounded to bf16 against the row's maximum over the 32-key blocks so far, in every tile alike: the same
+    steps in float64 with those roundings, and the same rows within a longer padded batch. Scores differ from the
+    kernel's by their fp32 summation order (some 1e-6), which moves one P or output in 2^-8 / 1e-6 = 4000 to the next
+    bf16, 2^-8 of its size: sqrt(1 / 4000) 2^-9 is 3e-5 of the 2-norm, bounded by 2e-4. One maximum per 64 keys
+    instead differs by 1e-3."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    n = 700
+    say(f"attention running max d={d} hq={hq} hkv={hkv} causal={causal} softcap={softcap}")
+    r = rng(d + hq)
+    q, k, v = (to_dev(bf16_np(r.normal(size=(1, n, h, d)).astype(np.float32) * a)) for h, a in ((hq, 2.0), (hkv, 1.0), (hkv, 1.0)))
+    mask = torch.ones((1, n), dtype=torch.bool, device="cuda")
+    got = K.attention(q, k, v, mask, causal=causal, softcap=softcap)
+
+    log2e = 1.4426950408889634
+    rep = hq // hkv
+    kk, vv = (t[0].double().repeat_interleave(rep, 1).transpose(0, 1) for t in (k, v))
+    z = q[0].double().transpose(0, 1) @ kk.transpose(1, 2).contiguous() * d ** -0.5
+    if softcap:
+        z = softcap * torch.tanh(z / softcap)
+    i = torch.arange(n, device="cuda")
+    keep = (i[None, :] <= i[:, None]) if causal else torch.ones((n, n), dtype=torch.bool, device="cuda")
+    z = (z * log2e).masked_fill(~keep, -1e30)
+    m = torch.full((hq, n, 1), -1e30, dtype=torch.float64, device="cuda")
+    total, acc = torch.zeros_like(m), torch.zeros((hq, n, d), dtype=torch.float64, device="cuda")
+    for j in range(0, n, 32):
+        part = z[:, :, j:j + 32]
+        mn = torch.maximum(m, part.amax(-1, keepdim=True))
+        p = torch.exp2(part - mn) * keep[:, j:j + 32]
+        total = total * torch.exp2(m - mn) + p.sum(-1, keepdim=True)
+        acc = acc * torch.exp2(m - mn) + p.to(torch.bfloat16).double() @ vv[:, j:j + 32]
+        m = mn
+    want = (acc / total).transpose(0, 1)[None]
+    rel = lambda a, b: float((a.double() - b.double()).norm() / b.double().norm())  # noqa: E731
+    err = rel(got, want.to(torch.bfloat16))
+    say(f"  against the same steps in float64: {err:.2e}")
+    assert err < 2e-4
+    # the last rows of a sequence, whose wave holds rows past its end, and the same rows inside a longer batch
+    short = [t[:, :100].contiguous() for t in (q, k, v)]
+    alone = K.attention(*short, mask[:, :100], causal=causal, softcap=softcap)
+    padded = K.attention(*(torch.nn.functional.pad(t, (0, 0, 0, 0, 0, 100)) for t in short),
+                         torch.arange(200, device="cuda")[None] < 100, causal=causal, softcap=softcap)[:, :100]
+    say(f"  alone and padded: {rel(alone, padded):.2e}")
+    assert rel(alone, padded) < 2e-4
+
+
 # (lengths, hq, hkv, d, window, softcap, causal): tiles of 16 (head_dim 256, fewer than 256 tiles of 32) and of 32
 # queries, 16-key blocks split over 4 (head_dim 256) or 8 waves; ends of tiles, fewer blocks than waves, empty
 # sequences, one launch at and one below the switch of the tile height
