@@ -539,6 +539,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, key_mask: torch
         vp = torch.zeros_like(kp)
         mp = torch.zeros((b, length), dtype=torch.bool, device=q.device)
         qp[:, :nq], kp[:, :nk], vp[:, :nk], mp[:, :nk] = q, k, v, mask
+    for t, n in ((qp, "q"), (kp, "k"), (vp, "v")):
+        _need(t, n, q.dtype)
     # The key-mask kernel always: tiles whose keys the mask keeps run its unmasked body, so a full mask costs about
     # what the maskless kernel does. Rows that see no key are found and filled on the device. Nothing here asks the
     # device for a value, which would stall the stream for a host round trip.

@@ -83,6 +83,27 @@ def test_product_package_never_touches_the_oracle() -> None:
             assert not any(n.split(".")[0] == "oracle" for n in names), f"{path} imports the oracle"
 
 
+@pytest.mark.parametrize("host,nq", [("q", 64), ("k", 64), ("v", 64), ("all", 64), ("all", 40)])
+def test_attention_refuses_host_tensors(monkeypatch: pytest.MonkeyPatch, host: str, nq: int) -> None:
+    """`attention` and `flash_attention` raise for a tensor in host memory, and no library call sees its address.
+    (A tensor on the meta device stands for one on the GPU: its kind is all that the check may look at.)"""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    calls: list[str] = []
+    monkeypatch.setattr(K, "call", lambda name, *args: calls.append(name))
+    monkeypatch.setattr(K, "_stream", lambda: 0)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda t: t.device.type == "meta"))
+    t = {n: torch.zeros((1, length, 2, 64), device="cpu" if host in (n, "all") else "meta")
+         for n, length in (("q", nq), ("k", 64), ("v", 64))}
+    with pytest.raises(ValueError, match="device"):
+        K.attention(t["q"], t["k"], t["v"], torch.ones((1, 64), dtype=torch.bool))
+    with pytest.raises(ValueError, match="device"):
+        K.flash_attention(torch.zeros((1, 64, 3 * 128), dtype=torch.bfloat16), torch.ones((1, 64), dtype=torch.bool), heads=2)
+    assert not calls
+
+
 def test_missing_library_fails_loudly(monkeypatch: pytest.MonkeyPatch, tmp_path: Any) -> None:
     from deciax_amd import _lib
 
