@@ -51,6 +51,7 @@
 // attention kernel stages (one column per token: vt_col[row]).
 #include "common.h"
 #include "kernels.h"
+#include "loads.h"
 #include "rownorm.h"
 
 namespace {
@@ -768,14 +769,14 @@ gemm_ring_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
   const int bbytes = (int)((long)brows * ldb * 2);
   const int KT = K / BK;
   auto issue = [&](int t, int stage) __attribute__((always_inline)) {
-    // past the last tile: empty resources, so the loads count but touch no memory
-    const __amdgpu_buffer_rsrc_t ra = make_rsrc(A + (long)m0 * lda, t < KT ? abytes : 0);
-    const __amdgpu_buffer_rsrc_t rb = make_rsrc(B + (long)row0 * ldb, t < KT ? bbytes : 0);
+    const LoadRange la = tile_range(t, KT, abytes, BK * 2), lb = tile_range(t, KT, bbytes, BK * 2);
+    const __amdgpu_buffer_rsrc_t ra = make_rsrc(A + (long)m0 * lda, la.bytes);
+    const __amdgpu_buffer_rsrc_t rb = make_rsrc(B + (long)row0 * ldb, lb.bytes);
     uint16_t *base = smem + stage * STAGE;
 #pragma unroll
-    for (int j = 0; j < AI; ++j) lds_load16(ra, base + (wave * AI + j) * 512, aoff[j], t * BK * 2);
+    for (int j = 0; j < AI; ++j) lds_load16(ra, base + (wave * AI + j) * 512, aoff[j], la.at);
 #pragma unroll
-    for (int j = 0; j < BI; ++j) lds_load16(rb, base + BM * BK + (wave * BI + j) * 512, boff[j], t * BK * 2);
+    for (int j = 0; j < BI; ++j) lds_load16(rb, base + BM * BK + (wave * BI + j) * 512, boff[j], lb.at);
   };
   floatx16 acc[TM][TN];
 #pragma unroll
