@@ -14,6 +14,7 @@
 // the latency of some sixty small launches.
 #include "common.h"
 #include "kernels.h"
+#include "loads.h"
 
 namespace {
 
@@ -318,23 +319,20 @@ linear_split_kernel(const float *__restrict__ x, const float *__restrict__ w, co
   const int xstep = (int)(RPP * ldx * 4), wstep = (int)(RPP * ldw * 4);
   floatx4 st[AP + BP];
   auto load = [&](int kk) __attribute__((always_inline)) {
+    const int at = column_offset(kk + 4 * pc, k, kk * 4);  // chunks at k or past it read as zeros
 #pragma unroll
     for (int j = 0; j < AP; ++j)
-      st[j] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rx, xoff + j * xstep, kk * 4, 0));
+      st[j] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rx, xoff + j * xstep + at, 0, 0));
 #pragma unroll
     for (int j = 0; j < BP; ++j)
-      st[AP + j] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rw, woff + j * wstep, kk * 4, 0));
+      st[AP + j] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rw, woff + j * wstep + at, 0, 0));
   };
   const int dst = pc / 2 * HALF + prow * 8 + pc % 2 * 4;
-  // chunks at k or past it (the next row's values) count as zeros: w's are cleared
-  auto put = [&](int stage, int kk) __attribute__((always_inline)) {
-    const bool live = kk + 4 * pc < k;
+  auto put = [&](int stage) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < AP + BP; ++j) {
-      floatx4 v = st[j];
-      if (j >= AP) v = live ? v : floatx4{0.f, 0.f, 0.f, 0.f};
       u32x2 p[3];
-      split3(v, p);
+      split3(st[j], p);
       uint16_t *d = smem + stage * STAGE + dst + (j < AP ? j * RPP : BM + (j - AP) * RPP) * 8;
 #pragma unroll
       for (int t = 0; t < 3; ++t) *reinterpret_cast<u32x2 *>(d + t * PLANE) = p[t];
@@ -371,12 +369,12 @@ linear_split_kernel(const float *__restrict__ x, const float *__restrict__ w, co
   };
   const int steps = (k + BK - 1) / BK;
   load(0);
-  put(0, 0);
+  put(0);
   load(min(BK, (steps - 1) * BK));
   __syncthreads();
   for (int t = 0; t < steps; ++t) {
     mma(t & 1);
-    put((t + 1) & 1, (t + 1) * BK);  // past the end: zeros or old chunks that nothing reads
+    put((t + 1) & 1);  // past the end: old chunks that nothing reads
     load(min(t + 2, steps - 1) * BK);
     __syncthreads();
   }

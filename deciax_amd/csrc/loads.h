@@ -14,3 +14,7 @@ struct LoadRange {
 constexpr LoadRange tile_range(int t, int tiles, int bytes, int step) {
   return t < tiles ? LoadRange{bytes, t * step} : LoadRange{0, 0};
 }
+
+// What a load of column `col` (of `cols`) adds to its row's offset: `bytes`, or past every operand whose rows span less
+// than 2^30 bytes (row offsets stay below that too, so the sum fits 31 bits).
+constexpr int column_offset(int col, int cols, int bytes) { return col < cols ? bytes : 1 << 30; }

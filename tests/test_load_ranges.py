@@ -49,9 +49,32 @@ int main() {
 }
 """
 
+SPLIT = r"""
+int main() {
+  // fp32 rows of ld elements in 16-byte chunks, 16 columns a step, up to 128 rows a tile: linear_split_kernel's loads,
+  // of an operand that ends with column k of its last row
+  for (int k : {64, 68, 100, 1024, 1028})
+    for (int64_t pad : {(int64_t)0, (int64_t)4, (int64_t)(1 << 20) - k})
+      for (int rows : {1, 7, 127, 128}) {
+        const int64_t ld = k + pad;
+        const int bytes = (int)(((rows - 1) * ld + k) * 4);
+        for (int kk = 0; kk < k; kk += 16)
+          for (int64_t row = 0; row < 128; ++row)
+            for (int c = 0; c < 4; ++c) {
+              const int64_t v = (row * ld + 4 * c) * 4 + column_offset(kk + 4 * c, k, kk * 4);
+              CHECK(v < ((int64_t)1 << 31));
+              CHECK(safe((uint32_t)v, 0, bytes, bytes));
+              if (row >= rows || kk + 4 * c >= k) CHECK(blocked((uint32_t)v, 0, bytes));
+              else CHECK(v + 16 <= bytes);
+            }
+      }
+  return 0;
+}
+"""
+
 
 @pytest.mark.skipif(GXX is None, reason="no g++")
-@pytest.mark.parametrize("name,body", [pytest.param("ring", RING, id="ring")])
+@pytest.mark.parametrize("name,body", [pytest.param("ring", RING, id="ring"), pytest.param("split", SPLIT, id="split")])
 def test_loads_stay_inside_their_operand(tmp_path: Path, name: str, body: str) -> None:
     src, exe = tmp_path / f"{name}.cpp", tmp_path / name
     src.write_text(PRELUDE + body)
