@@ -687,6 +687,16 @@ attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, const 
           l[u] += p;
         }
     }
+    if (k0 + KB > len) {  // rows past the sequence count as zeros (their weight is 0, the last row's value may be infinite)
+#pragma unroll
+      for (int s = 0; s < SUB; ++s)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          if (k0 + 16 * s + 4 * g + t >= len) {
+#pragma unroll
+            for (int a = 0; a < A; ++a) vf[s][t][a] = floatx4{0.f, 0.f, 0.f, 0.f};
+          }
+    }
 #pragma unroll
     for (int s = 0; s < SUB; ++s)
 #pragma unroll

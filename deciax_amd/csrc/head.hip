@@ -650,6 +650,16 @@ mha_f32_mfma_kernel(const float *__restrict__ q, const float *__restrict__ k, co
           l[u] += p;
         }
     }
+    if (k0 + KB > K) {  // keys past K count as zeros (their weight is 0, the last key's value may be infinite)
+#pragma unroll
+      for (int s = 0; s < SUB; ++s)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          if (k0 + 16 * s + 4 * g + t >= K) {
+#pragma unroll
+            for (int c = 0; c < N; ++c) vf[s][t][c] = 0.f;
+          }
+    }
 #pragma unroll
     for (int s = 0; s < SUB; ++s)
 #pragma unroll

@@ -318,3 +318,23 @@ def test_mha_f32_forms(batch: int, nq: int, nk: int, heads: int, dh: int) -> Non
     # scores of dh products: relative 2^-24 (dh + 4) of sum |q k|, a few units; the weights inherit it
     err = (got - want).abs().max().item()
     assert err < 4 * 2.0 ** -24 * (dh + 16) * float((split(q).abs() @ split(k).abs().transpose(-1, -2)).max()) / dh ** 0.5, err
+
+
+@pytest.mark.parametrize("nq,dh", [(3, 16), (40, 64), (5, 128), (700, 64)])
+@pytest.mark.parametrize("nk", [1, 65, 127])
+def test_mha_f32_infinite_last_value(nq: int, dh: int, nk: int) -> None:
+    """An infinite value of the last key comes out infinite, in both workgroup forms: keys past the last add nothing."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    say(f"mha_f32, infinite last value, {nq} x {nk} x {dh}")
+    r = rng(nq + nk + dh)
+    heads = 16
+    q, k, v = (torch.as_tensor(r.normal(size=(t, heads * dh)).astype(np.float32)).cuda() for t in (nq, nk, nk))
+    mask = torch.ones((1, nk), dtype=torch.uint8, device="cuda")
+    want = K.mha_f32(q, k, v, mask, batch=1, heads=heads)
+    v[nk - 1, 5], v[nk - 1, heads * dh - 1] = np.inf, -np.inf
+    got = K.mha_f32(q, k, v, mask, batch=1, heads=heads)
+    want[:, 5], want[:, -1] = np.inf, -np.inf
+    assert torch.equal(got, want)

@@ -509,6 +509,26 @@ def test_attention_fp32_tiles(lengths, hq, hkv, d, window, softcap, causal) -> N
     np.testing.assert_allclose(to_np(out).reshape(want.shape), want, rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("n", [17, 33, 127])
+def test_attention_fp32_infinite_last_value(d: int, n: int) -> None:
+    """An infinite value in a sequence's last row, which every row sees, comes out infinite: rows that a block reads
+    past the end add nothing to it."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    say(f"attention fp32, infinite last value, d={d} n={n}")
+    r = rng(d + n)
+    q, k, v = (to_dev(r.normal(size=(1, n, 2, d)).astype(np.float32), "f32") for _ in range(3))
+    want = K.attention(q, k, v, torch.ones((1, n), dtype=torch.bool))
+    v[0, n - 1, 1, 3], v[0, n - 1, 0, d - 1] = np.inf, -np.inf
+    got = K.attention(q, k, v, torch.ones((1, n), dtype=torch.bool))
+    assert (got[0, :, 1, 3] == np.inf).all() and (got[0, :, 0, d - 1] == -np.inf).all()
+    want[0, :, 1, 3], want[0, :, 0, d - 1] = np.inf, -np.inf
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("window", [0, 64])
 def test_attention_fp32_window_softcap(window: int) -> None:
     from deciax_amd import kernels as K
