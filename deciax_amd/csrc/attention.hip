@@ -544,7 +544,7 @@ attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, const 
                     float scale, float softcap, int window, int causal, const uint8_t *__restrict__ key_mask) {
   constexpr int C = D / 16, A = D / 64, KB = 16 * SUB, BQ = 16 * QB, OP = D + 4;
   constexpr int NC = D / 32;  // partial sums per score
-  static_assert(D % 64 == 0 && KB <= 64, "tile shape");
+  static_assert(D % 64 == 0 && KB <= 64 && (WAVES & (WAVES - 1)) == 0, "tile shape");
   __shared__ __attribute__((aligned(16))) float os[WAVES * BQ * OP];
   __shared__ float ms[WAVES][BQ], ls[WAVES][BQ];
 
@@ -595,7 +595,10 @@ attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, const 
 #pragma unroll
     for (int c = 0; c < C; ++c) o[u][c] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
-  int k0 = klo / KB * KB + wave * KB;
+  // key block j goes to wave j % WAVES, counted from key 0: a row's sums then do not depend on the tile it is in, whose
+  // height follows the size of the launch
+  const int first = klo / KB;
+  int k0 = (first + ((wave - first) & (WAVES - 1))) * KB;
   if (k0 < khi) load_k(k0);
   for (; k0 < khi; k0 += WAVES * KB) {
     floatx4 vf[SUB][4][A];

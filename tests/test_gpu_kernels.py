@@ -509,6 +509,32 @@ def test_attention_fp32_tiles(lengths, hq, hkv, d, window, softcap, causal) -> N
     np.testing.assert_allclose(to_np(out).reshape(want.shape), want, rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("d,window,causal", [(256, 100, True), (256, 37, False), (256, 0, True), (128, 70, True), (64, 21, False)])
+def test_attention_fp32_rows_do_not_depend_on_the_launch(d: int, window: int, causal: bool) -> None:
+    """A sequence alone and as one of six, padded and packed: the same bits, whichever tile height the launch takes
+    (head_dim 256: 16 query rows below 256 tiles of 32)."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    lengths = [517, 600, 1, 333, 700, 690]
+    hq, hkv = 8, 4
+    say(f"attention fp32, one sequence alone and in a batch, d={d} window={window} causal={causal}")
+    r = rng(d + window)
+    q, k, v, starts = _packed_case(d + window, lengths, hq, hkv, d, dtype="f32", scale=1.0)
+    dev = [to_dev(a.reshape(a.shape[0], -1), "f32") for a in (q, k, v)]
+    kw = dict(num_q_heads=hq, num_kv_heads=hkv, head_dim=d, scale=d ** -0.5, window=window, causal=causal)
+    packed = K.attention_varlen(*dev, i32(starts), i32(lengths), max(lengths), **kw)
+    x = [torch.as_tensor(r.normal(size=(6, 700, h, d)).astype(np.float32)).cuda() for h in (hq, hkv, hkv)]
+    mask = torch.arange(700, device="cuda")[None] < torch.tensor(lengths, device="cuda")[:, None]
+    padded = K.attention(*x, mask, causal=causal, window=window)
+    for b, (s, n) in enumerate(zip(starts, lengths)):
+        alone = K.attention_varlen(*(t[s:s + n] for t in dev), i32([0]), i32([n]), n, **kw)
+        assert torch.equal(alone, packed[s:s + n]), f"packed sequence {b}"
+        alone = K.attention(*(t[b:b + 1, :n] for t in x), mask[b:b + 1, :n], causal=causal, window=window)
+        assert torch.equal(alone[0], padded[b, :n]), f"padded sequence {b}"
+
+
 @pytest.mark.parametrize("d", [64, 128, 256])
 @pytest.mark.parametrize("n", [17, 33, 127])
 def test_attention_fp32_infinite_last_value(d: int, n: int) -> None:
