@@ -980,15 +980,17 @@ hipError_t dx_span_means_gather_f32_launch(const float *x, const int32_t *index,
 template <int N>
 static void mha_run(const float *q, const float *k, const float *v, const uint8_t *key_mask, float *out, int B, int Q,
                     int K, int H, long ldq, long ldk, long ldv, long ldo, hipStream_t s) {
-  // keys per block: as many as leave registers for two waves per SIMD (the softmax of one beside the products of
-  // the other)
-  constexpr int SUB = N <= 4 ? 4 : 2, SUB2 = N <= 2 ? 4 : N <= 5 ? 2 : 1;
+  // Eight waves and SUB blocks of 16 keys a step (as many as leave registers for two waves per SIMD, the softmax of one
+  // beside the products of the other) at every size, so that a row's sums do not depend on the launch; its size picks
+  // 16 or 32 queries alone. us, 4 waves -> 8, 16 heads x 64: 1 x 23 x 600 11.9 -> 11.8, 8 x 64 x 4096 169 -> 164,
+  // 8 x 512 x 4096 657 -> 677; 8 heads x 128, 2 x 100 x 1500 48 -> 47. SUB 4 at head_dim 64: 14, 163 and 860.
+  constexpr int SUB = N <= 2 ? 4 : N <= 5 ? 2 : 1;
   if ((long)B * H * ((Q + 31) / 32) >= 512)
-    mha_f32_mfma_kernel<N, 2, 4, SUB2><<<dim3((Q + 31) / 32, H, B), 256, 0, s>>>(q, k, v, key_mask, out, Q, K, ldq, ldk,
-                                                                              ldv, ldo);
+    mha_f32_mfma_kernel<N, 2, 8, SUB><<<dim3((Q + 31) / 32, H, B), 512, 0, s>>>(q, k, v, key_mask, out, Q, K, ldq, ldk,
+                                                                             ldv, ldo);
   else
     mha_f32_mfma_kernel<N, 1, 8, SUB><<<dim3((Q + 15) / 16, H, B), 512, 0, s>>>(q, k, v, key_mask, out, Q, K, ldq, ldk,
-                                                                              ldv, ldo);
+                                                                             ldv, ldo);
 }
 
 hipError_t dx_mha_f32_launch(const float *q, const float *k, const float *v, const uint8_t *key_mask, float *out,

@@ -338,3 +338,24 @@ def test_mha_f32_infinite_last_value(nq: int, dh: int, nk: int) -> None:
     got = K.mha_f32(q, k, v, mask, batch=1, heads=heads)
     want[:, 5], want[:, -1] = np.inf, -np.inf
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("heads,dh", [(16, 32), (16, 64), (8, 80), (8, 128)])
+def test_mha_f32_rows_do_not_depend_on_the_launch(heads: int, dh: int) -> None:
+    """A batch row alone and among eight, with its own keys and padded by masked ones: the same bits, in both workgroup
+    forms."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    say(f"mha_f32, one batch row alone and among eight, {heads} heads x {dh}")
+    r = rng(heads + dh)
+    nq, nk, w, lens = 130, 300, heads * dh, [300, 17, 64, 250, 299, 1, 128, 200]
+    q, k, v = (torch.as_tensor(r.normal(size=(8, t, w)).astype(np.float32)).cuda() for t in (nq, nk, nk))
+    mask = (torch.arange(nk, device="cuda")[None] < torch.tensor(lens, device="cuda")[:, None]).to(torch.uint8)
+    flat = lambda t: t.reshape(-1, w).contiguous()  # noqa: E731
+    got = K.mha_f32(flat(q), flat(k), flat(v), mask, batch=8, heads=heads).view(8, nq, w)
+    for b, n in enumerate(lens):
+        for few in (nq, 5):
+            alone = K.mha_f32(flat(q[b, :few]), flat(k[b, :n]), flat(v[b, :n]), mask[b:b + 1, :n].contiguous(), batch=1, heads=heads)
+            assert torch.equal(alone, got[b, :few]), f"batch row {b}, {few} queries"
