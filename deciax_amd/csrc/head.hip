@@ -20,7 +20,6 @@ namespace {
 
 constexpr int THREADS = 256;
 constexpr float MASK_FILL = -1e30f;  // src/deciax/kernels/attention/reference.py:8
-constexpr float LOG2E = 1.4426950408889634f;
 
 DX_DEVICE float wave_reduce_sum(float v) {
 #pragma unroll
@@ -634,7 +633,7 @@ mha_f32_mfma_kernel(const float *__restrict__ q, const float *__restrict__ k, co
       mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
       const float mn = fmaxf(mr[u], mx);
-      const float alpha = fast_exp2((mr[u] - mn) * LOG2E);
+      const float alpha = expf(mr[u] - mn);
       mr[u] = mn;
       l[u] *= alpha;
       if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {
@@ -645,7 +644,7 @@ mha_f32_mfma_kernel(const float *__restrict__ q, const float *__restrict__ k, co
       for (int s = 0; s < SUB; ++s)
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-          const float p = fast_exp2((sc[u][s][t] - mn) * LOG2E);
+          const float p = expf(sc[u][s][t] - mn);
           sc[u][s][t] = p;
           l[u] += p;
         }
@@ -693,7 +692,7 @@ mha_f32_mfma_kernel(const float *__restrict__ q, const float *__restrict__ k, co
     float num = 0.f, den = 0.f;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
-      const float f = fast_exp2((ms[w][qi] - mx) * LOG2E);
+      const float f = expf(ms[w][qi] - mx);
       num += os[w][qi][d] * f;
       den += ls[w][qi] * f;
     }

@@ -359,3 +359,30 @@ def test_mha_f32_rows_do_not_depend_on_the_launch(heads: int, dh: int) -> None:
         for few in (nq, 5):
             alone = K.mha_f32(flat(q[b, :few]), flat(k[b, :n]), flat(v[b, :n]), mask[b:b + 1, :n].contiguous(), batch=1, heads=heads)
             assert torch.equal(alone, got[b, :few]), f"batch row {b}, {few} queries"
+
+
+@pytest.mark.parametrize("nq", [3, 600])
+def test_mha_f32_weights_keep_fp32_precision(nq: int) -> None:
+    """Scores that are exact (multiples of 1/8) from 0 to -70, one-hot values: each weight within 6 units in the last place
+    of e^s / sum (a 2-ulp exponential, a sum of 64 positive terms in parts of a few, one quotient, the merge's factor).
+    Rounding s log2(e) first would miss by |s| 2^-24: 35 units at -70."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    say(f"mha_f32 weights, {nq} queries")
+    heads, dh, nk = 16, 64, 64
+    r = rng(nq)
+    s = -np.sort(r.integers(0, 560, (nk,)) / 8.0)[::-1]
+    s[-1] = 0.0
+    q = torch.zeros((nq, heads, dh), device="cuda")
+    k = torch.zeros((nk, heads, dh), device="cuda")
+    q[:, :, 0] = 8.0
+    k[:, :, 0] = torch.as_tensor(s.copy(), dtype=torch.float32, device="cuda")[:, None]
+    v = torch.eye(64, device="cuda")[:, None, :].expand(nk, heads, dh)
+    mask = torch.ones((1, nk), dtype=torch.uint8, device="cuda")
+    got = K.mha_f32(*(t.reshape(-1, heads * dh).contiguous() for t in (q, k, v)), mask, batch=1, heads=heads)
+    e = np.exp(s)
+    want = torch.as_tensor(e / e.sum(), device="cuda")
+    rel = ((got.view(nq, heads, dh).double() - want) / want).abs()
+    assert rel.max() < 6 * 2.0 ** -23, float(rel.max())
