@@ -136,21 +136,22 @@ layer_norm_f32_row_kernel(const float *__restrict__ x, const float *__restrict__
 DX_DEVICE floatx4 mfma16_f32(float a, float b, floatx4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 // y[m, n] = (acc ? y[m, n] : 0) + act(x[m, :] . w[n, :] + bias[n]); act: 0 identity, 1 exact GELU.
-// A wave computes 16 TM x 16 TN outputs over its share of k: KW waves of the workgroup split k in runs of 16 KC
-// (interleaved, so together they read whole cache lines) and add their sums through LDS; WM x WN such groups
-// stand side by side. A wave's lane (l % 16, l / 16) holds k values k0 + 16 c + 4 (l / 16) .. + 3 of its row, for
-// chunks c < KC, loaded one step ahead into the other half of its registers. Rows past m and n read the last
-// row (not stored). VEC: rows are 16-byte aligned, else elements are read one at a time.
-template <int TM, int TN, int KW, int WM, int WN, int KC, bool VEC>
-__global__ void __launch_bounds__(64 * KW * WM * WN)
+// Rows that are not whole 16-byte chunks, and short ones (the others take the split products below). A workgroup
+// computes 16 TM x 16 TN outputs; its KW waves split k in runs of 32 (interleaved, so together they read whole cache
+// lines) and add their sums through LDS, in the same order for every tile shape, so that a row does not depend on m.
+// A wave's lane (l % 16, l / 16) holds k values k0 + 16 c + 4 (l / 16) .. + 3 of its row, for chunks c < KC, loaded one
+// step ahead into the other half of its registers. Rows past m and n read the last row (not stored). VEC: rows are
+// 16-byte aligned, else elements are read one at a time.
+template <int TM, int TN, bool VEC>
+__global__ void __launch_bounds__(256)
 linear_f32_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
                   float *__restrict__ y, long m, int n, int k, long ldx, long ldw, long ldy, int act, int acc) {
-  constexpr int STEP = 16 * KC;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int kw = wave % KW, wn = wave / KW % WN, wm = wave / (KW * WN);
+  constexpr int KW = 4, KC = 2, STEP = 16 * KC;
+  const int tid = threadIdx.x, lane = tid & 63, kw = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lk = lane >> 4;
-  const long m0 = ((long)blockIdx.y * WM + wm) * (16 * TM);
-  const int n0 = ((int)blockIdx.x * WN + wn) * (16 * TN);
+  const unsigned num_n = (n + 16 * TN - 1) / (16 * TN);
+  const long m0 = (long)(blockIdx.x / num_n) * (16 * TM);
+  const int n0 = (int)(blockIdx.x % num_n) * (16 * TN);
   const float *xp[TM], *wp[TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i) xp[i] = x + min(m0 + 16 * i + lr, m - 1) * ldx + 4 * lk;
@@ -231,45 +232,35 @@ linear_f32_kernel(const float *__restrict__ x, const float *__restrict__ w, cons
     float *dst = y + gm * ldy + gn;
     *dst = acc ? *dst + v : v;
   };
-  if constexpr (KW == 1) {
+  constexpr int TILE = 256 * TM * TN;
+  __shared__ float part[KW * TILE];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
+    for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) store(m0 + 16 * i + 4 * lk + r, n0 + 16 * j + lr, c[i][j][r]);
-  } else {
-    static_assert(WM == 1 && WN == 1, "k-split workgroups hold one tile");
-    constexpr int TILE = 256 * TM * TN;
-    __shared__ float part[KW * TILE];
+      for (int r = 0; r < 4; ++r)
+        part[kw * TILE + (16 * i + 4 * lk + r) * (16 * TN) + 16 * j + lr] = c[i][j][r];
+  __syncthreads();
+  for (int idx = tid; idx < TILE; idx += 256) {
+    float v = 0.f;
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          part[kw * TILE + (16 * i + 4 * lk + r) * (16 * TN) + 16 * j + lr] = c[i][j][r];
-    __syncthreads();
-    for (int idx = tid; idx < TILE; idx += 64 * KW) {
-      float v = 0.f;
-#pragma unroll
-      for (int q = 0; q < KW; ++q) v += part[q * TILE + idx];
-      store(m0 + idx / (16 * TN), n0 + idx % (16 * TN), v);
-    }
+    for (int q = 0; q < KW; ++q) v += part[q * TILE + idx];
+    store(m0 + idx / (16 * TN), n0 + idx % (16 * TN), v);
   }
 }
 
-// Large products: fp32 operands as sums of three bf16 (x = h + m + l, each the bf16 nearest to what is left: 24 bits
-// or more), multiplied by six bf16 MFMAs: h h into one fp32 accumulator, l h, h l, m m, m h, h m into another, 2^-8
-// of its size, so that one rounding per 16 k counts. What is left out (m l, l m, l l) is below 2^-25 of |x w|, less
-// than the rounding of an fp32 product. Error against 64 bits at k = 1024 / 4096: 1.3e-7 / 2.9e-7 (fp32 MFMAs in one
-// chain 4.0e-7 / 8.2e-7; both accumulators in one 3.4e-7 / 7.2e-7, 4% faster).
-// Tile (64 TM) x (64 TN) of 2 x 2 waves, 16 k per step. A step's fp32 chunks arrive in registers one step ahead, are
-// split once per workgroup and go to the other half of the LDS. What bounds it: the bf16 MFMAs, 6 / 16 of the cycles
-// of fp32 ones, at the rate the large bf16 GEMMs reach (1.2 PFLOP/s of them). Two register sets, or the split spread
-// between the MFMAs, measured the same or slower; 32 k per step 20% slower.
+// fp32 operands as sums of three bf16 (x = h + m + l, each the bf16 nearest to what is left: 24 bits or more),
+// multiplied by six bf16 MFMAs: h h into one fp32 accumulator, l h, h l, m m, m h, h m into another, 2^-8 of its size,
+// so that one rounding per 16 k counts. What is left out (m l, l m, l l) is below 2^-24 of |x w| (m below 2^-8 |x|, l
+// below 2^-17 |x|, so 2^-25 for each of the first two): the rounding of an fp32 product at most. The pair of accumulators
+// joins the sum after every PART k. Error against 64 bits at k = 1024 / 4096: 1.0e-7 / 1.2e-7 (over all of k 1.9e-7 /
+// 4.0e-7; both accumulators in one 3.4e-7 / 7.2e-7; fp32 MFMAs in one chain 4.0e-7 / 8.2e-7, in four 2.9e-7 / 5.7e-7).
+// Two kernels, the same chain of MFMAs and sums for an output in both, so that a row does not depend on m.
 // An infinity, a NaN or a value past the largest bf16 leaves its row or column of the accumulators not finite (inf -
-// inf): a wave that finds one multiplies its part again with fp32 MFMAs.
+// inf): those outputs, and no others, are multiplied again with fp32 MFMAs.
+constexpr int PART = 256;
+
 DX_DEVICE void split3(const floatx4 &v, u32x2 (&p)[3]) {
   float a[4] = {v[0], v[1], v[2], v[3]};
 #pragma unroll
@@ -286,6 +277,252 @@ DX_DEVICE void split3(const floatx4 &v, u32x2 (&p)[3]) {
   }
 }
 
+// One lane's outputs of a 32 x 32 block, from the rows of x and w that the lane feeds (whole 16-byte chunks). Rare, so
+// a plain loop.
+DX_DEVICE floatx16 product32_f32(const float *xr, const float *wr, int k, int lhalf) {
+  floatx16 c;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) c[r] = 0.f;
+  for (int k0 = 4 * lhalf; k0 < k + 4 * lhalf; k0 += 8) {  // both lane halves take as many steps
+    floatx4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
+    if (k0 < k) {
+      a = *reinterpret_cast<const floatx4 *>(xr + k0);
+      b = *reinterpret_cast<const floatx4 *>(wr + k0);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_32x32x2f32(b[e], a[e], c, 0, 0, 0);
+  }
+  return c;
+}
+
+// Four sums of a row, columns col..col + 3 at dst: bias, act and accumulation as linear_f32_kernel.
+DX_DEVICE void store_quad(floatx4 v, float *dst, const float *__restrict__ bias, int col, int n, int act, int acc_y,
+                          int vec_y) {
+  if (vec_y && col + 4 <= n) {
+    if (bias) v += *reinterpret_cast<const floatx4 *>(bias + col);
+    if (act == 1) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = gelu_erf(v[e]);
+    }
+    if (acc_y) v += *reinterpret_cast<const floatx4 *>(dst);
+    *reinterpret_cast<floatx4 *>(dst) = v;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (col + e >= n) continue;
+      float s = v[e] + (bias ? bias[col + e] : 0.f);
+      if (act == 1) s = gelu_erf(s);
+      dst[e] = acc_y ? dst[e] + s : s;
+    }
+  }
+}
+
+// 16 bytes per lane from a buffer resource into LDS at lds + 16 * lane. The builtin is compiled in the device pass only:
+// this clang drops a kernel's host-side symbols when the host pass sees it.
+typedef __attribute__((address_space(3))) void lds_void;
+DX_DEVICE void lds_load16(__amdgpu_buffer_rsrc_t rsrc, float *lds, int voffset) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void *)lds, 16, voffset, 0, 0, 0);
+#endif
+}
+
+// Few rows, or few columns: tiles of 32 x 32, a part of k per wave (parts w, w + WAVES, .. for wave w). A wave streams
+// SK columns of its 64 rows at a time through a ring of its own in LDS (loads to LDS, no barrier: a load straight into
+// the MFMA layout would take four rows per quad of lanes and four times the address cycles; 11 us for 8 at 23 x 1024 x
+// 1024, 35 for 22 at k = 4096), reads them in the MFMA layout (lane (l % 32, l / 32): k 8 (l / 32) .. + 7 of row l % 32)
+// and splits them itself. The parts' sums meet in LDS. What bounds it: some 110 vector instructions a wave and 16 k.
+template <int WAVES, int SK, int RING>
+__global__ void __launch_bounds__(64 * WAVES)
+linear_split_small_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
+                          float *__restrict__ y, long m, int n, int k, long ldx, long ldw, long ldy, int act, int acc_y,
+                          int vec_y) {
+  constexpr int STAGES = PART / SK, SUB = SK / 16;      // stages of a part; 16 k of a stage
+  constexpr int CPR = SK / 4, RPI = 64 / CPR, NI = 32 / RPI;  // 16-byte chunks per row; rows and instructions per load
+  constexpr int SLOT = 64 * SK;                         // floats: x's 32 rows, then w's
+  static_assert((SK == 16 || SK == 32) && STAGES % 2 == 0 && WAVES >= 4 && (RING - 1) * 2 * NI <= 63, "wave schedule");
+  // the rings, then the waves' sums; a flag over the first ring at the end. One array: with several the compiler waits for
+  // every load to LDS before each read of the ring.
+  __shared__ __attribute__((aligned(1024))) float smem[WAVES * RING * SLOT + WAVES * 1024];
+  floatx4(*const sums)[4][64] = reinterpret_cast<floatx4(*)[4][64]>(smem + WAVES * RING * SLOT);  // [register / 4][lane]
+  int *const bad = reinterpret_cast<int *>(smem);
+  const int num_n = (n + 31) / 32;
+  const long m0 = (long)(blockIdx.x / num_n) * 32;
+  const int n0 = (int)(blockIdx.x % num_n) * 32;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lrow = lane & 31, lhalf = lane >> 5;
+  const int arows = (int)min(32L, m - m0), brows = min(32, n - n0);
+  // rows past m and n, and columns past k, read as zeros
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)(x + m0 * ldx), (short)0, (int)(((long)(arows - 1) * ldx + k) * 4), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)(w + (long)n0 * ldw), (short)0, (int)(((long)(brows - 1) * ldw + k) * 4), 0x00020000);
+  const int parts = (k + PART - 1) / PART, rounds = (parts + WAVES - 1) / WAVES;
+  // Row r's chunk c lies in slot c ^ swz(r): 16 rows' reads of one chunk fall on all banks
+  auto swz = [](int r) { return SK == 32 ? (r >> 1) & 7 : (r >> 2) & 3; };
+  float *const mine = smem + wave * RING * SLOT;
+  int col[NI], xoff[NI], woff[NI];  // of the lane's 16 bytes in each instruction
+#pragma unroll
+  for (int j = 0; j < NI; ++j) {
+    const int row = j * RPI + lane / CPR;
+    col[j] = 4 * ((lane % CPR) ^ swz(row));
+    xoff[j] = (int)(row * ldx * 4);
+    woff[j] = (int)(row * ldw * 4);
+  }
+  auto load = [&](int u) __attribute__((always_inline)) {  // the wave's stage u
+    const int c0 = ((u / STAGES) * WAVES + wave) * PART + u % STAGES * SK;
+    float *to = mine + u % RING * SLOT;
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      const int at = column_offset(c0 + col[j], k, (c0 + col[j]) * 4);
+      lds_load16(rx, to + j * 256, xoff[j] + at);
+      lds_load16(rw, to + 32 * SK + j * 256, woff[j] + at);
+    }
+  };
+  auto read = [&](floatx4 (&v)[SUB][4], int u) __attribute__((always_inline)) {
+    const float *from = mine + u % RING * SLOT + lrow * SK;
+#pragma unroll
+    for (int i = 0; i < SUB; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int at = ((4 * i + 2 * lhalf + j) ^ swz(lrow)) * 4;
+        v[i][j] = *reinterpret_cast<const floatx4 *>(from + at);
+        v[i][2 + j] = *reinterpret_cast<const floatx4 *>(from + 32 * SK + at);
+      }
+  };
+  auto planes = [&](const floatx4 &lo, const floatx4 &hi, bf16x8 (&f)[3]) __attribute__((always_inline)) {
+    u32x2 p[3], q[3];
+    split3(lo, p);
+    split3(hi, q);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) f[t] = as_bf16x8(u32x4{p[t][0], p[t][1], q[t][0], q[t][1]});
+  };
+  floatx16 c, small;
+  struct Planes {
+    bf16x8 a[3], b[3];
+  };
+  // multiplies 16 k while the next 16 are split, the vector instructions spread over the MFMAs
+  auto step = [&](const Planes &p, const floatx4 (&next)[4], Planes &q) __attribute__((always_inline)) {
+    small = mfma32(p.b[0], p.a[2], small);
+    c = mfma32(p.b[0], p.a[0], c);
+    small = mfma32(p.b[2], p.a[0], small);
+    small = mfma32(p.b[1], p.a[1], small);
+    small = mfma32(p.b[0], p.a[1], small);
+    small = mfma32(p.b[1], p.a[0], small);
+    planes(next[0], next[1], q.a);
+    planes(next[2], next[3], q.b);
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // stage u has landed once the RING - 1 younger ones are all that is in flight
+  auto landed = [&]() __attribute__((always_inline)) {
+    constexpr int VM = (RING - 1) * 2 * NI;
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((VM & 15) | (VM >> 4) << 14 | 7 << 4 | 15 << 8);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto refill = [&](int u) __attribute__((always_inline)) {  // stage u's slot, read by now, takes stage u + RING
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(15 | 3 << 14 | 7 << 4);
+    __builtin_amdgcn_sched_barrier(0);
+    load(u + RING);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  floatx4 total = {0.f, 0.f, 0.f, 0.f};  // of the first four waves: registers 4 wave .. + 3 of lane
+  // Stage u + 1 (SK 32) or u + 2 (SK 16) is read while stage u is multiplied.
+  floatx4 v0[SUB][4], v1[SUB][4];
+  Planes p0, p1;
+  if (wave < parts) {
+#pragma unroll
+    for (int i = 0; i < RING; ++i) load(i);
+    landed();
+    read(v0, 0);
+    refill(0);
+    planes(v0[0][0], v0[0][1], p0.a);
+    planes(v0[0][2], v0[0][3], p0.b);
+    if constexpr (SUB == 1) {
+      landed();
+      read(v1, 1);
+      refill(1);
+    }
+  }
+  for (int r = 0; r < rounds; ++r) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) c[e] = small[e] = 0.f;
+    if (r * WAVES + wave < parts) {
+      for (int t = 0; t < STAGES; t += 2) {
+        const int u = r * STAGES + t;
+        if constexpr (SUB == 1) {
+          landed();
+          read(v0, u + 2);
+          __builtin_amdgcn_sched_barrier(0);
+          step(p0, v1[0], p1);
+          refill(u + 2);
+          landed();
+          read(v1, u + 3);
+          __builtin_amdgcn_sched_barrier(0);
+          step(p1, v0[0], p0);
+          refill(u + 3);
+        } else {
+          landed();
+          read(v1, u + 1);
+          __builtin_amdgcn_sched_barrier(0);
+          step(p0, v0[SUB - 1], p1);
+          refill(u + 1);
+          step(p1, v1[0], p0);
+          landed();
+          read(v0, u + 2);
+          __builtin_amdgcn_sched_barrier(0);
+          step(p0, v1[SUB - 1], p1);
+          refill(u + 2);
+          step(p1, v0[0], p0);
+        }
+      }
+    }
+    if (r > 0) __syncthreads();  // the last round's sums are read
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      sums[wave][q][lane] = floatx4{c[4 * q] + small[4 * q], c[4 * q + 1] + small[4 * q + 1], c[4 * q + 2] + small[4 * q + 2],
+                                    c[4 * q + 3] + small[4 * q + 3]};
+    __syncthreads();
+    if (wave < 4)
+      for (int q = 0; q < min(WAVES, parts - r * WAVES); ++q) total += sums[q][wave][lane];
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // loads to LDS past the last part
+  if (tid == 0) *bad = 0;
+  __syncthreads();
+  if (wave < 4)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (!(fabsf(total[e]) < INFINITY)) *bad = 1;
+  __syncthreads();
+  const long row = m0 + lrow;
+  if (*bad) {
+    if (wave == 0) {
+      const floatx16 f = product32_f32(x + min(row, m - 1) * ldx, w + (long)min(n0 + lrow, n - 1) * ldw, k, lhalf);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sums[0][q][lane] = floatx4{f[4 * q], f[4 * q + 1], f[4 * q + 2], f[4 * q + 3]};
+    }
+    __syncthreads();
+    if (wave < 4) {
+      const floatx4 f = sums[0][wave][lane];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) total[e] = fabsf(total[e]) < INFINITY ? total[e] : f[e];
+    }
+  }
+  if (wave < 4 && row < m) {
+    const int col = n0 + 8 * wave + 4 * lhalf;
+    store_quad(total, y + row * ldy + col, bias, col, n, act, acc_y, vec_y);
+  }
+}
+
+// Many rows: tile (64 TM) x (64 TN) of 2 x 2 waves, 16 k per step. A step's fp32 chunks arrive in registers one step
+// ahead, are split once per workgroup and go to the other half of the LDS. What bounds it: the bf16 MFMAs, 6 / 16 of
+// the cycles of fp32 ones, at the rate the large bf16 GEMMs reach (1.2 PFLOP/s of them). Two register sets, or the
+// split spread between the MFMAs, measured the same or slower; 32 k per step 20% slower.
 template <int TM, int TN>
 __global__ void __launch_bounds__(256, 2)
 linear_split_kernel(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
@@ -337,13 +574,24 @@ linear_split_kernel(const float *__restrict__ x, const float *__restrict__ w, co
       for (int t = 0; t < 3; ++t) *reinterpret_cast<u32x2 *>(d + t * PLANE) = p[t];
     }
   };
-  floatx16 c[TM][TN], small[TM][TN];
+  floatx16 c[TM][TN], small[TM][TN], total[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) c[i][j][r] = small[i][j][r] = 0.f;
+      for (int r = 0; r < 16; ++r) c[i][j][r] = small[i][j][r] = total[i][j][r] = 0.f;
+  auto fold = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          total[i][j][r] += c[i][j][r] + small[i][j][r];
+          c[i][j][r] = small[i][j][r] = 0.f;
+        }
+  };
   auto mma = [&](int stage) __attribute__((always_inline)) {
     const uint16_t *pa = smem + stage * STAGE + lhalf * HALF + (wm * 32 * TM + lrow) * 8;
     const uint16_t *pb = smem + stage * STAGE + lhalf * HALF + (BM + wn * 32 * TN + lrow) * 8;
@@ -373,9 +621,15 @@ linear_split_kernel(const float *__restrict__ x, const float *__restrict__ w, co
   __syncthreads();
   for (int t = 0; t < steps; ++t) {
     mma(t & 1);
+    // (where the fold stands decides the registers: here 128 x 128 tiles keep two workgroups a CU, and after the barrier
+    // 128 x 64 tiles let the split run beside the MFMAs, 33 us for 39 at k = 1024)
+    if constexpr (TN == 2)
+      if ((t + 1) % (PART / BK) == 0 || t + 1 == steps) fold();
     put((t + 1) & 1);  // past the end: old chunks that nothing reads
     load(min(t + 2, steps - 1) * BK);
     __syncthreads();
+    if constexpr (TN == 1)
+      if ((t + 1) % (PART / BK) == 0 || t + 1 == steps) fold();
   }
 
   bool bad = false;
@@ -385,62 +639,33 @@ linear_split_kernel(const float *__restrict__ x, const float *__restrict__ w, co
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        c[i][j][r] += small[i][j][r];
-        bad = bad || !(fabsf(c[i][j][r]) < INFINITY);
+        bad = bad || !(fabsf(total[i][j][r]) < INFINITY);
       }
   if (__builtin_amdgcn_ballot_w64(bad)) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
+      for (int j = 0; j < TN; ++j) {
+        const floatx16 f = product32_f32(x + min(m0 + wm * 32 * TM + 32 * i + lrow, m - 1) * ldx,
+                                         w + (long)min(n0 + wn * 32 * TN + 32 * j + lrow, n - 1) * ldw, k, lhalf);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) c[i][j][r] = 0.f;
-    for (int k0 = 0; k0 < k; k0 += 2) {
-      const int kk = k0 + lhalf;
-      float a[TM], b[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-        a[i] = kk < k ? x[min(m0 + wm * 32 * TM + 32 * i + lrow, m - 1) * ldx + kk] : 0.f;
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-        b[j] = kk < k ? w[(long)min(n0 + wn * 32 * TN + 32 * j + lrow, n - 1) * ldw + kk] : 0.f;
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) c[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[j], a[i], c[i][j], 0, 0, 0);
-    }
+        for (int r = 0; r < 16; ++r) total[i][j][r] = fabsf(total[i][j][r]) < INFINITY ? total[i][j][r] : f[r];
+      }
   }
-
-  // lane (lrow, lhalf) holds row 32 i + lrow, columns 32 j + 8 q + 4 lhalf + 0..3 in registers 4 q .. 4 q + 3
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const long row = m0 + wm * 32 * TM + 32 * i + lrow;
     if (row >= m) continue;
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+    for (int j = 0; j < TN; ++j) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int col = n0 + wn * 32 * TN + 32 * j + 8 * q + 4 * lhalf;
-        float *out = y + row * ldy + col;
-        floatx4 v = {c[i][j][4 * q], c[i][j][4 * q + 1], c[i][j][4 * q + 2], c[i][j][4 * q + 3]};
-        if (vec_y && col + 4 <= n) {
-          if (bias) v += *reinterpret_cast<const floatx4 *>(bias + col);
-          if (act == 1) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = gelu_erf(v[e]);
-          }
-          if (acc_y) v += *reinterpret_cast<const floatx4 *>(out);
-          *reinterpret_cast<floatx4 *>(out) = v;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            if (col + e >= n) continue;
-            float s = v[e] + (bias ? bias[col + e] : 0.f);
-            if (act == 1) s = gelu_erf(s);
-            out[e] = acc_y ? out[e] + s : s;
-          }
-        }
+        const floatx16 &v = total[i][j];
+        store_quad(floatx4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]}, y + row * ldy + col, bias, col, n, act, acc_y,
+                   vec_y);
       }
+    }
   }
 }
 
@@ -896,69 +1121,57 @@ hipError_t dx_layer_norm_f32_launch(const float *x, const float *w, const float 
   return hipGetLastError();
 }
 
-template <int TM, int TN, int KW, int WM, int WN, int KC>
+template <int TM, int TN>
 static void linear_run(const float *x, const float *w, const float *bias, float *y, long m, int n, int k, long ldx,
                        long ldw, long ldy, int act, int acc, hipStream_t s) {
   const bool vec = ((ldx | ldw) & 3) == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
-  const dim3 grid(blocks(n, 16 * TN * WN), blocks(m, 16 * TM * WM));
-  auto kern = vec ? linear_f32_kernel<TM, TN, KW, WM, WN, KC, true> : linear_f32_kernel<TM, TN, KW, WM, WN, KC, false>;
-  kern<<<grid, 64 * KW * WM * WN, 0, s>>>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc);
-}
-
-template <int TM, int TN>
-static void split_run(const float *x, const float *w, const float *bias, float *y, long m, int n, int k, long ldx,
-                      long ldw, long ldy, int act, int acc, hipStream_t s) {
-  const int vec_y = (ldy & 3) == 0 && ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(bias)) & 15) == 0;
-  linear_split_kernel<TM, TN><<<blocks(n, 64 * TN) * blocks(m, 64 * TM), 256, 0, s>>>(x, w, bias, y, m, n, k, ldx, ldw,
-                                                                                     ldy, act, acc, vec_y);
+  auto kern = vec ? linear_f32_kernel<TM, TN, true> : linear_f32_kernel<TM, TN, false>;
+  kern<<<blocks(n, 16 * TN) * blocks(m, 16 * TM), 256, 0, s>>>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc);
 }
 
 hipError_t dx_linear_f32_launch(const float *x, const float *w, const float *bias, float *y, long m, int n, int k,
                                 long ldx, long ldw, long ldy, int act, int acc, hipStream_t s) {
-  // Each form's time is its rounds of waves over the 1024 SIMDs times a wave's share of one 64 x 64 x k product,
-  // and the smaller tiles re-read their operands more often: a 64 x 32, 32 x 32 or 16 x 16 wave runs at 0.7, 0.55
-  // or 0.22 of the 64 x 64 wave's rate (measured; us, 64 x 64 with k whole / split 2 / 4, 64 x 32, 32 x 32, 16 x 16):
-  //   23 x 1024 x 4096: 249 / 126 / 67, 35, 28, 20     200 x 1024 x 1024: 72 / 38 / 24, 16, 11, 18
-  //   512 x 1024 x 1024: 71 / 38 / 25, 17, 20, 36      600 x 2048 x 1024: 72 / 41 / 47, 48, 44, 80
-  //   1200 x 2048 x 1024: 74 / 80 / 71, 84, 84, 156    2000 x 1024 x 4096: 264 / 137 / 151, 225, 237, 566
-  //   32768 x 2048 x 1024: 1143 / 1327 / 1443, 1700, 2015, -
+  // n, k, strides and alignment choose between the split products and the fp32 ones (another order of the sums); m, by
+  // the rounds of tiles over the chip, only a tile shape.
   auto tiles = [&](int tm, int tn) { return (m + tm - 1) / tm * ((n + tn - 1) / tn); };
-  auto rounds = [](long waves) { return (double)((waves + 1023) / 1024); };
-  const long t64 = tiles(64, 64);
-  const double cost[6] = {rounds(t64),
-                          rounds(2 * t64) / 2,
-                          rounds(4 * t64) / 4,
-                          rounds(4 * tiles(64, 32)) / 8 * 1.45,
-                          rounds(4 * tiles(32, 32)) / 16 * 1.8,
-                          rounds(16 * tiles(16, 16)) / 256 * 4.5};
-  int best = 0;
-  for (int i = 1; i < 6; ++i)
-    if (cost[i] < cost[best]) best = i;
-  // In the same unit (71 us at k = 1024), the split forms: 128 x 128 tiles 46 us a round of 256 workgroups, 128 x 64
-  // tiles 27 us and 4 (us, the best of the above -> 128 x 128, 128 x 64):
-  //   600 x 2048 x 1024: 42 -> 47, 32      1200 x 2048 x 1024: 70 -> 50, 47    2000 x 1024 x 4096: 141 -> 162, 119
-  //   4096 x 1024 x 1024: 86 -> 57, 57     4096 x 2048 x 4096: 535 -> 350, 402 32768 x 1024 x 4096: 2093 -> 1375, 1584
-  //   512 x 2048 x 1024: 27 -> 47, 32      600 x 1024 x 4096: 70 -> 162, 105
-  // They read whole 16-byte chunks of a row through 32-bit offsets.
+  // the split kernels read whole 16-byte chunks of a row through 32-bit offsets
   const bool chunks = k >= 64 && ((k | ldx | ldw) & 3) == 0 && ldx <= (1 << 20) && ldw <= (1 << 20) &&
                       ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
   if (chunks) {
-    const long wide = (tiles(128, 128) + 255) / 256, slim = (tiles(128, 64) + 255) / 256;
-    const double wide_cost = wide * (46 / 71.), slim_cost = (27 * slim + 4) / 71.;
-    if (fmin(wide_cost, slim_cost) < cost[best]) {
-      if (wide_cost <= slim_cost) split_run<2, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s);
-      else split_run<2, 1>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s);
-      return hipGetLastError();
+    const int vec_y = (ldy & 3) == 0 && ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(bias)) & 15) == 0;
+    // us per 1024 k: 128 x 128 tiles 46 a round of 256 workgroups and 10, 128 x 64 tiles 28 and 6, 32 x 32 tiles 7 for
+    // one round, then 2 and 0.0215 a tile. Measured us, 32 x 32 / 128 x 64 / 128 x 128 (fp32 or split products chosen by
+    // m, before):
+    //   23 x 1024 x 1024: 8 / 33 / 56 (6)       23 x 1024 x 4096: 22 / 126 / 210 (20)     200 x 1024 x 4096: 24 / 137 / 212 (34)
+    //   600 x 1024 x 4096: 67 / 139 / 214 (73)  600 x 2048 x 1024: 29 / 38 / 59 (35)      2000 x 1024 x 1024: 45 / 42 / 61 (38)
+    //   4096 x 1024 x 4096: 339 / 229 / 231 (197)   4096 x 2048 x 4096: 689 / 453 / 374 (357)
+    //   32768 x 1024 x 4096: 2812 / 1619 / 1395 (1296)
+    const long wide = tiles(128, 128), slim = tiles(128, 64), few = tiles(32, 32);
+    const double wide_us = 46. * ((wide + 255) / 256) + 10, slim_us = 28. * ((slim + 255) / 256) + 6;
+    const double few_us = few <= 256 ? 7 : 0.0215 * few + 2;
+    if (few_us <= fmin(wide_us, slim_us)) {
+      // eight parts of k at once, or four in rings of 32 columns
+      if (k <= 4 * PART)
+        linear_split_small_kernel<4, 32, 2><<<(unsigned)few, 256, 0, s>>>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc,
+                                                                         vec_y);
+      else
+        linear_split_small_kernel<8, 16, 2><<<(unsigned)few, 512, 0, s>>>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc,
+                                                                         vec_y);
+    } else if (wide_us <= slim_us) {
+      linear_split_kernel<2, 2><<<(unsigned)wide, 256, 0, s>>>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, vec_y);
+    } else {
+      linear_split_kernel<2, 1><<<(unsigned)slim, 256, 0, s>>>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, vec_y);
     }
+    return hipGetLastError();
   }
-  switch (best) {
-    case 0: linear_run<4, 4, 1, 4, 1, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s); break;
-    case 1: linear_run<4, 4, 2, 1, 1, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s); break;
-    case 2: linear_run<4, 4, 4, 1, 1, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s); break;
-    case 3: linear_run<4, 2, 4, 1, 1, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s); break;
-    case 4: linear_run<2, 2, 4, 1, 1, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s); break;
-    default: linear_run<1, 1, 16, 1, 1, 4>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s); break;
-  }
+  // A tile's time is its rounds of waves over the 1024 SIMDs times a wave's share of one 64 x 64 x k product; a 64 x 32
+  // or 32 x 32 wave, which re-reads its operands more often, runs at 0.7 or 0.55 of the 64 x 64 wave's rate.
+  auto rounds = [](long waves) { return (double)((waves + 1023) / 1024); };
+  const double cost[3] = {rounds(4 * tiles(64, 64)) / 4, rounds(4 * tiles(64, 32)) / 8 * 1.45,
+                          rounds(4 * tiles(32, 32)) / 16 * 1.8};
+  if (cost[0] <= fmin(cost[1], cost[2])) linear_run<4, 4>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s);
+  else if (cost[1] <= cost[2]) linear_run<4, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s);
+  else linear_run<2, 2>(x, w, bias, y, m, n, k, ldx, ldw, ldy, act, acc, s);
   return hipGetLastError();
 }
 

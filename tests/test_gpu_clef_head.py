@@ -164,9 +164,9 @@ def test_encoded_requests_through_head() -> None:
 
 
 @pytest.mark.parametrize("m,n,k,pad", [
-    (1, 1, 1, 0), (3, 17, 31, 0), (16, 16, 64, 0), (17, 1000, 1029, 3),   # 16 x 16 tiles, k over 16 waves
-    (200, 1030, 95, 1), (300, 1000, 96, 0), (513, 515, 100, 1),           # 32 x 32 and 64 x 32 tiles, k over 4 waves
-    (601, 2047, 70, 0), (20000, 200, 36, 0), (4097, 1025, 130, 4),        # 64 x 64 tiles, k over 2, 4 and 1 waves
+    (1, 1, 1, 0), (3, 17, 31, 0), (17, 1000, 1029, 3), (200, 1030, 95, 1), (513, 515, 100, 1),  # fp32 products, 32 x 32
+    (601, 2047, 70, 0), (4097, 1025, 130, 4), (20000, 200, 36, 0),                              # and 64 x 32, 64 x 64 tiles
+    (16, 16, 64, 0), (300, 1000, 96, 0),                                                        # split products
 ])
 def test_linear_f32_tiles(m: int, n: int, k: int, pad: int) -> None:
     """Every tile shape at its edges, rows with and without 16-byte alignment, bias, GELU and accumulation, against
@@ -191,14 +191,16 @@ def test_linear_f32_tiles(m: int, n: int, k: int, pad: int) -> None:
 
 
 @pytest.mark.parametrize("m,n,k,pad,scale", [
-    (1300, 2000, 100, 4, 1.0), (4097, 1025, 132, 0, 1.0), (1281, 2050, 64, 8, 1e-30),   # 128 x 128 tiles
-    (600, 2048, 68, 0, 1.0), (577, 2049, 80, 4, 1e30), (641, 2047, 1028, 0, 1.0),       # 128 x 64 tiles
+    (1300, 2000, 100, 4, 1.0), (4097, 1025, 132, 0, 1.0), (1281, 2050, 64, 8, 1e-30),   # 128 x 64 tiles
+    (4097, 2050, 100, 4, 1.0), (8200, 1025, 264, 0, 1.0),                               # 128 x 128 tiles
+    (600, 2048, 68, 0, 1.0), (577, 2049, 80, 4, 1e30), (641, 2047, 1028, 0, 1.0),       # 32 x 32 tiles
+    (1, 1, 64, 0, 1.0), (33, 31, 260, 4, 1.0), (65, 70, 2052, 0, 1.0), (5, 40, 6000, 8, 1.0),
 ])
 def test_linear_f32_split_tiles(m: int, n: int, k: int, pad: int, scale: float) -> None:
     """The three-bf16 products at the edges of their tiles and of a 16-wide step, with bias, GELU and accumulation and
-    rows that hold NaN past k, against 64 bits. The six products leave out 2^-25 |x w|, and the two accumulators take
-    k / 16 and 5 k / 16 roundings, the second of terms 2^-8 the size: within the bound k 2^-24 sum |x w| of an fp32
-    sum, and its 2-norm within that of torch's fp32 product."""
+    rows that hold NaN past k, against 64 bits. The six products leave out up to 2^-24 |x w|, and the two accumulators
+    take k / 16 and 5 k / 16 roundings, the second of terms 2^-8 the size: within the bound (k + 2) 2^-24 sum |x w| of an
+    fp32 sum, and its 2-norm within that of torch's fp32 product."""
     import torch
 
     from deciax_amd import kernels as K
@@ -386,3 +388,53 @@ def test_mha_f32_weights_keep_fp32_precision(nq: int) -> None:
     want = torch.as_tensor(e / e.sum(), device="cuda")
     rel = ((got.view(nq, heads, dh).double() - want) / want).abs()
     assert rel.max() < 6 * 2.0 ** -23, float(rel.max())
+
+
+@pytest.mark.parametrize("n,k,pad", [(1024, 1024, 0), (2047, 4096, 4), (1, 2048, 0), (96, 100, 0), (1030, 257, 0), (70, 63, 1)])
+def test_linear_f32_rows_do_not_depend_on_m(n: int, k: int, pad: int) -> None:
+    """A row has the same bits in every launch that holds it, whichever tiles its size takes: split products (rows of
+    whole 16-byte chunks) and fp32 ones, with bias, GELU and accumulation. Values of other rows that are not finite change
+    nothing either."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    say(f"linear_f32 rows, {n} x {k}, row padding {pad}")
+    r = rng(n + k)
+    big = 9000
+    x = torch.as_tensor(r.normal(size=(big, k + pad)).astype(np.float32)).cuda()[:, :k]
+    w = torch.as_tensor(r.normal(size=(n, k + pad)).astype(np.float32)).cuda()[:, :k]
+    b = torch.as_tensor(r.normal(size=n).astype(np.float32)).cuda()
+    base = torch.as_tensor(r.normal(size=(big, n)).astype(np.float32)).cuda()
+    run = lambda rows, xx=x: K.linear_f32(xx[rows], w, b, gelu=True, out=base[rows].clone(), accumulate=True)  # noqa: E731
+    want = run(slice(0, big))
+    for m in (1, 5, 33, 130, 600, 1300, 2100, 4200, 6500):
+        assert torch.equal(run(slice(0, m)), want[:m]), f"first {m} rows"
+        assert torch.equal(run(slice(big - m, big)), want[big - m:]), f"last {m} rows"
+    dirty = x.clone()
+    dirty[1::64, 0], dirty[2::64, k - 1], dirty[3::64, k // 2] = np.nan, np.inf, 3.395e38
+    clean = torch.ones(big, dtype=torch.bool, device="cuda")
+    for i in (1, 2, 3):
+        clean[i::64] = False
+    for m in (600, 2100, big):
+        assert torch.equal(run(slice(0, m), dirty)[clean[:m]], want[:m][clean[:m]]), f"{m} rows beside others not finite"
+
+
+def test_head_results_do_not_depend_on_the_batch() -> None:
+    """Requests alone and in one padded batch (other lengths, option and field counts): the same logits, bit for bit."""
+    import torch
+
+    from deciax_amd import clef_head
+
+    say("joint head, requests alone and in a batch")
+    p, a, hidden, lexical = _random_case(3, batch=5, seq=700, hidden=1024, width=512, ff=1024, nq=20, no=90, ntypes=3,
+                                         routing_layers=2, layers=2)
+    params = {n: v * 0.2 if v.ndim == 2 else v for n, v in _dev_params(p).items()}
+    kw = dict(heads=8, routing_layers=2, layers=2)
+    want = clef_head.forward(params, hidden, lexical, a, **kw)
+    for i in range(5):
+        size = {"mask": int(a["mask"][i].sum()), "question": int(a["question_mask"][i].sum()),
+                "types": int(a["question_mask"][i].sum()), "option": int(a["option_mask"][i].sum())}
+        own = {n: v[i:i + 1, :size[n.split("_")[0]]] for n, v in a.items()}
+        got = clef_head.forward(params, hidden[i:i + 1, :size["mask"]], lexical[i:i + 1, :size["option"]], own, **kw)
+        assert got.isfinite().all() and torch.equal(got[0], want[i, :size["option"]]), f"request {i}"
