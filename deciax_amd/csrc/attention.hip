@@ -847,7 +847,7 @@ hipError_t launch_bf16_dgw(const AttnArgs &a, hipStream_t s) {
                                            : attn_bf16_kernel<D, G, MODE_ONLINE, true, W, NS>)
                          : (fixed_shift(a) ? attn_bf16_kernel<D, G, MODE_FIXED, false, W, NS>
                                            : attn_bf16_kernel<D, G, MODE_ONLINE, false, W, NS>);
-  if constexpr (W == 8)
+  if constexpr (W == 8 || D == 128)
     if (a.softcap > 0.f && !fixed_shift(a))
       kern = a.key_bits ? attn_bf16_kernel<D, G, MODE_CAP, true, W, NS> : attn_bf16_kernel<D, G, MODE_CAP, false, W, NS>;
   kern<<<grid, dim3(64 * W), 0, s>>>(
@@ -868,7 +868,8 @@ inline long mean_key_span(const AttnArgs &a) {
 
 template <int D, int G>
 hipError_t launch_bf16_dg(const AttnArgs &a, hipStream_t s) {
-  if (a.softcap > 0.f && !fixed_shift(a)) return launch_bf16_dgw<D, G, 8, 4>(a, s);  // the one form built with MODE_CAP
+  // MODE_CAP is built for the long form and the short one at head_dim 128
+  if (D != 128 && a.softcap > 0.f && !fixed_shift(a)) return launch_bf16_dgw<D, G, 8, 4>(a, s);
   if constexpr (D <= 128)
     if (mean_key_span(a) <= (D == 64 ? 4096 : 2048)) return launch_bf16_dgw<D, G, 4, 2>(a, s);
   if constexpr (D == 256) {

@@ -291,6 +291,8 @@ def test_attention_head_dim_128_short_and_long_forms_agree(hq: int, hkv: int) ->
     (4, 4, 256, 0, 0.0, False, 16384),
     (12, 12, 64, 0, 0.0, False, 8192),      # 4096 keys or fewer a row: 4 waves over two stages
     (8, 2, 64, 0, 50.0, True, 16384),
+    (8, 4, 128, 0, 80.0, True, 16384),      # caps beyond the fixed shift: 2048 keys or fewer a row 4 waves, else 8
+    (8, 4, 128, 0, 80.0, False, 16384),
 ])
 def test_attention_forms_agree(hq: int, hkv: int, d: int, window: int, softcap: float, causal: bool,
                                longer: int) -> None:
