@@ -691,6 +691,8 @@ UNSEEN_CASES = [
     (1, 65, 2, 2, 64, True, 0, "bf16"),
     (200, 129, 4, 2, 128, True, 70, "f32"),
     (129, 200, 2, 2, 256, False, 3, "f32"),
+    (90, 700, 4, 2, 64, False, 0, "bf16"),   # more keys than a pass of the mean takes
+    (70, 300, 4, 1, 256, True, 9, "f32"),
 ]
 
 
