@@ -86,6 +86,9 @@ int validate_attn_v(int32_t head_dim, int32_t num_kv_heads, int64_t k_row_stride
   return DX_OK;
 }
 
+// A window as long as the longest sequence hides nothing; the kernels add it to row indices in 32 bits.
+int32_t in_range(int32_t window, int32_t max_seq_len) { return window < max_seq_len ? window : max_seq_len; }
+
 // The bf16 kernel reads one sequence's K rows and one KV head's V^T block through buffer resources whose
 // byte ranges and per-lane offsets are 32-bit: len * k_stride * 2 bytes of K, and
 // ((D - 1) * vt_ld + len rounded up to 64) * 2 bytes of V^T. Larger spans would wrap.
@@ -194,7 +197,8 @@ int attn_prefill(const void *q, const void *k, const void *v, const uint8_t *key
   if (st) return st;
   if (num_seqs == 0 || max_seq_len == 0) return DX_OK;
   AttnArgs a{q, k, v, out, seq_start, seq_len, nullptr, num_seqs, max_seq_len, num_q_heads, num_kv_heads, head_dim,
-             q_row_stride, k_row_stride, v_row_stride, out_row_stride, 0, scale, softcap, window, causal ? 1 : 0};
+             q_row_stride, k_row_stride, v_row_stride, out_row_stride, 0, scale, softcap,
+             in_range(window, max_seq_len), causal ? 1 : 0};
   a.key_mask = key_mask;
   if (dtype == DX_F32) return check_launch(dx_attn_f32(a, as_stream(stream)), "attention fp32 launch");
 
@@ -299,7 +303,7 @@ int dx_attn_padded(const void *q, const void *k, const void *v, const uint8_t *k
   if (batch == 0 || num_q == 0) return DX_OK;
   hipStream_t s = as_stream(stream);
   AttnArgs a{q, k, v, out, nullptr, nullptr, nullptr, batch, len, num_q_heads, num_kv_heads, head_dim,
-             q_row_stride, k_row_stride, v_row_stride, out_row_stride, 0, scale, softcap, window, causal ? 1 : 0};
+             q_row_stride, k_row_stride, v_row_stride, out_row_stride, 0, scale, softcap, in_range(window, len), causal ? 1 : 0};
   AttnArgs rows = a;  // token-major values, for the rows that see no key
   hipError_t e;
   if (dtype == DX_F32) {
@@ -347,7 +351,8 @@ int dx_attn_prefill_vt(const void *q, const void *k, const void *vt, void *out, 
   if (st) return st;
   if (num_seqs == 0 || max_seq_len == 0) return DX_OK;
   AttnArgs a{q, k, vt, out, seq_start, seq_len, vt_start, num_seqs, max_seq_len, num_q_heads, num_kv_heads,
-             head_dim, q_row_stride, k_row_stride, vt_ld, out_row_stride, 0, scale, softcap, window, causal ? 1 : 0};
+             head_dim, q_row_stride, k_row_stride, vt_ld, out_row_stride, 0, scale, softcap,
+             in_range(window, max_seq_len), causal ? 1 : 0};
   return check_launch(dx_attn_bf16(a, as_stream(stream)), "attention bf16 launch");
 }
 

@@ -724,6 +724,23 @@ def test_attention_rows_that_see_no_key(nq, nk, hq, hkv, d, causal, window, dtyp
             np.testing.assert_allclose(got[bi], want, rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("causal", [False, True])
+def test_attention_window_beyond_every_row(dtype: str, causal: bool) -> None:
+    """The largest window is none, bit for bit (index sums with it stay in 32 bits)."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    say(f"attention, largest window, {dtype} causal={causal}")
+    r = rng(5)
+    q, k, v = (to_dev(bf16_np(r.normal(size=(2, 150, h, 64)).astype(np.float32)), dtype) for h in (4, 2, 2))
+    mask = torch.arange(150, device="cuda")[None] < torch.tensor([[150], [77]], device="cuda")
+    want = K.attention(q, k, v, mask, causal=causal)
+    for window in (150, 2 ** 31 - 1):
+        assert torch.equal(K.attention(q, k, v, mask, causal=causal, window=window), want), window
+
+
 @pytest.mark.parametrize("b,s,heads,window,dtype", [(2, 200, 4, 0, "bf16"), (2, 257, 3, 32, "bf16"),
                                                      (1, 96, 2, 8, "f32")])
 def test_flash_attention_packed_interface(b: int, s: int, heads: int, window: int, dtype: str) -> None:
