@@ -7,8 +7,9 @@
 // accumulators (a single wave saturates the matrix core with this shape).
 //
 // Two kernels: gemm_nt_kernel, described here (256 x 256 tiles, which large M takes, 192 x 256 ones where those fill
-// the CUs better, and the 128-row tiles of the residual-norm epilogue), and gemm_ring_kernel further down (smaller tiles, for launches that 256 x 256 tiles would
-// leave short of workgroups). dispatch() chooses by the tiles' rounds over the chip.
+// the CUs better, and the 128-row tiles of the residual-norm epilogue), and gemm_ring_kernel further down (smaller
+// tiles, for launches that 256 x 256 tiles would leave short of workgroups). dispatch() chooses by the tiles' rounds over
+// the chip.
 //
 // Two data paths (256- and 192-row tiles, and 128-row tiles with K <= 8192, take the second):
 //
@@ -993,7 +994,7 @@ hipError_t launch_ring(const uint16_t *A, const uint16_t *B, void *C, long M, lo
 // the smallest tile that still fits one round wins. Past two rounds the tiles drift apart and half of the last
 // round overlaps. Over 54 shapes (N x K of the 9B projections, M from 8 to 3300) the choice is within 0.8% of the
 // best measured form on average. us before (64 x 128, 128 x 256 or 256 x 256 tiles) -> now:
-//   3584 x 14336:  M 64 156 -> 38   M 200 156 -> 52   M 517 182 -> 89    M 1300 232 -> 149   M 3300 276 (unchanged)
+//   3584 x 14336:  M 64 156 -> 38   M 200 156 -> 52   M 517 182 -> 89    M 1300 232 -> 149   M 3300 276 -> 263
 //   28672 x 3584:  M 64  75 -> 40   M 200  75 -> 57   M 517 182 -> 128   M 1000 254 -> 162
 //   8192 x 3584:   M 64  47 -> 17   M 200  68 -> 24   M 517  66 -> 41    M 1000  64 -> 55
 // 192 x 256 (plain epilogues; a quarter fewer rows a tile where 256 x 256 leaves part of a round idle), us:
@@ -1020,11 +1021,12 @@ hipError_t dispatch(const uint16_t *A, const uint16_t *B, void *C, long M, long 
     // 256 x 256 first, then the ring forms of this epilogue (paired ones need an even TN, so they lack the
     // narrowest); q|k|v tiles must not straddle the end of the q|k columns
     static const TileForm forms[] = {{256, 256}, {256, 128}, {192, 128}, {128, 128}, {96, 128}, {64, 128}, {128, 64},
-                                     {64, 64},   {192, 64},  {96, 64},   {64, 32},   {32, PAIRED ? 64 : 32}, {192, 256}};
+                                     {64, 64},   {96, 64},   {64, 32},   {32, PAIRED ? 64 : 32}, {192, 256}};
+    constexpr int FORMS = sizeof(forms) / sizeof(forms[0]);
     int best = 0;
     double least = tile_cost(forms[0], M, N);
-    for (int i = 1; i < 13; ++i) {
-      if (PAIRED && ((i >= 8 && i <= 10) || i == 12)) continue;
+    for (int i = 1; i < FORMS; ++i) {
+      if (PAIRED && (i == 8 || i == 9 || i == 11)) continue;
       if (EPI == EPI_QKV && qe.qk_cols % forms[i].bn) continue;
       const double c = tile_cost(forms[i], M, N);
       if (c < least) {
@@ -1043,14 +1045,13 @@ hipError_t dispatch(const uint16_t *A, const uint16_t *B, void *C, long M, long 
       case 7: DX_RING(1, 2, 2, 1, 5);
     }
     if constexpr (PAIRED) {
-      if (best == 11) DX_RING(1, 2, 1, 1, 5);
+      if (best == 10) DX_RING(1, 2, 1, 1, 5);
     } else {
       switch (best) {
-        case 8: DX_RING(3, 1, 2, 2, 5);
-        case 9: DX_RING(3, 1, 1, 2, 7);
-        case 10: DX_RING(1, 1, 2, 1, 6);
-        case 11: DX_RING(1, 1, 1, 1, 8);
-        case 12: return launch<192, EPI>(A, B, C, M, N, K, lda, ldb, ldc, act, qe, ne, s);
+        case 8: DX_RING(3, 1, 1, 2, 7);
+        case 9: DX_RING(1, 1, 2, 1, 6);
+        case 10: DX_RING(1, 1, 1, 1, 8);
+        case 11: return launch<192, EPI>(A, B, C, M, N, K, lda, ldb, ldc, act, qe, ne, s);
       }
     }
 #undef DX_RING

@@ -1146,9 +1146,10 @@ def test_fused_residual_norm_forward_bit_identical() -> None:
     assert np.array_equal(out[True][1], out[False][1])
 
 
-# Rows whose choice of GEMM tile covers every form at N = 3584 (32 x 32, 64 x 32, 64 x 64, 96 x 64, 128 x 64, 96 x 128,
-# 128 x 128, 192 x 128, 256 x 128 and 256 x 256 tiles; 192 x 64 and 64 x 128 at the widths below), one row either side
-# of a tile edge among them; K of one and of five 64-deep tiles, fewer than the ring's stages.
+# Rows whose choice of GEMM tile covers every form at N = 3584: 32 x 32, 64 x 32, 64 x 64, 96 x 64, 128 x 64, 64 x 128,
+# 96 x 128, 128 x 128, 192 x 128, 256 x 128 and 192 x 256 tiles (gated ones the same but 64 x 32, 96 x 64 and 192 x 256,
+# 32 x 64 for 32 x 32, 256 x 256 last), one row either side of a tile edge among them; K of one and of five 64-deep
+# tiles, fewer than the ring's stages.
 FORM_ROWS = (1, 32, 33, 65, 100, 129, 200, 300, 400, 513, 600, 769, 1000, 1300, 1537, 2100, 3300)
 
 
@@ -1162,7 +1163,7 @@ def test_gemm_tile_forms_agree(k: int) -> None:
 
     say(f"GEMM tile forms, K={k}")
     r = rng(k)
-    big = 8192
+    big = 10240  # 256 x 256 tiles at each width below, plain and gated
     a = to_dev(bf16_np(r.normal(size=(big, k + 8)).astype(np.float32)))[:, :k]
     for n in (3584, 4608, 1280):
         w = to_dev(bf16_np(r.normal(size=(n, k)).astype(np.float32) * 0.1))
