@@ -947,7 +947,7 @@ routing_f32_kernel(const float *__restrict__ options, const float *__restrict__ 
                    const uint8_t *__restrict__ option_mask, float *__restrict__ summary, int O, int NQ, int W) {
   extern __shared__ __attribute__((aligned(16))) float p[];  // [O][FG] routing weights
   constexpr int WAVES = THREADS / 64;
-  const int b = blockIdx.z, f0 = blockIdx.y * FG, nf = min(FG, NQ - f0);
+  const int groups = (NQ + FG - 1) / FG, b = blockIdx.x / groups, f0 = blockIdx.x % groups * FG, nf = min(FG, NQ - f0);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const float *ob = options + (long)b * O * W;
   const float inv = 1.0f / sqrtf((float)W);
@@ -984,7 +984,7 @@ routing_f32_kernel(const float *__restrict__ options, const float *__restrict__ 
     for (int o = lane; o < O; o += 64) p[o * FG + f] /= sum;
   }
   __syncthreads();
-  const int i = blockIdx.x * THREADS + threadIdx.x;
+  const int i = blockIdx.y * THREADS + threadIdx.x;
   if (i >= W) return;
   float s[FG] = {};
   int o = 0;
@@ -1238,10 +1238,10 @@ hipError_t dx_routing_f32_launch(const float *options, const float *base, const 
   // eight questions per workgroup where that still fills the chip and their weights fit 64 KB of LDS
   const unsigned cols = blocks(W, THREADS);
   if (O <= 2048 && (long)B * blocks(NQ, 8) * cols >= 128)
-    routing_f32_kernel<8><<<dim3(cols, blocks(NQ, 8), B), THREADS, (size_t)O * 8 * sizeof(float), s>>>(
+    routing_f32_kernel<8><<<dim3(B * blocks(NQ, 8), cols), THREADS, (size_t)O * 8 * sizeof(float), s>>>(
         options, base, owner, option_mask, summary, O, NQ, W);
   else
-    routing_f32_kernel<1><<<dim3(cols, NQ, B), THREADS, (size_t)O * sizeof(float), s>>>(options, base, owner,
+    routing_f32_kernel<1><<<dim3((unsigned)(B * NQ), cols), THREADS, (size_t)O * sizeof(float), s>>>(options, base, owner,
                                                                                       option_mask, summary, O, NQ, W);
   return hipGetLastError();
 }

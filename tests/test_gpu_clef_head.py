@@ -438,3 +438,22 @@ def test_head_results_do_not_depend_on_the_batch() -> None:
         own = {n: v[i:i + 1, :size[n.split("_")[0]]] for n, v in a.items()}
         got = clef_head.forward(params, hidden[i:i + 1, :size["mask"]], lexical[i:i + 1, :size["option"]], own, **kw)
         assert got.isfinite().all() and torch.equal(got[0], want[i, :size["option"]]), f"request {i}"
+
+
+@pytest.mark.parametrize("batch,fields", [(70000, 1), (1, 70000)])
+def test_head_routing_beyond_a_grid_dimension(batch: int, fields: int) -> None:
+    """More batch rows or fields than a launch's y or z dimension holds: a field that owns one option gets that option."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    say(f"head routing, {batch} x {fields} fields")
+    g = torch.Generator(device="cuda").manual_seed(1)
+    options = torch.empty((batch * 2, 16), device="cuda").normal_(generator=g)
+    base = torch.empty((batch * fields, 16), device="cuda").normal_(generator=g)
+    owner = torch.tensor([[0, fields]], dtype=torch.int32, device="cuda").repeat(batch, 1)  # the second: no field's
+    mask = torch.ones((batch, 2), dtype=torch.uint8, device="cuda")
+    got = K.head_routing_f32(options, base, owner, mask, batch=batch)
+    assert torch.equal(got[::fields], options[::2])
+    if fields > 1:  # the others own none: the mean of all options
+        torch.testing.assert_close(got[1:], options.mean(0).expand(fields - 1, 16), rtol=1e-6, atol=1e-6)
