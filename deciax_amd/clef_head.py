@@ -9,6 +9,7 @@ include/deciax_hip.h); torch only supplies the device buffers. Batched tensors t
 
 from __future__ import annotations
 
+import math
 from collections.abc import Mapping
 from pathlib import Path
 from typing import Any
@@ -18,6 +19,7 @@ import torch
 
 from deciax_amd import kernels as K
 
+MAX_LOGIT_SCALE = math.log(100.0)  # head.py:17
 EPS = 1e-5                         # head.py:20-21
 
 
@@ -134,9 +136,20 @@ def forward(p: Mapping[str, torch.Tensor], hidden: Any, lexical: Any, a: Mapping
         dense(ff, n + ".linear2", out=fields, accumulate=True)
 
     fields_o = K.gather_rows_f32(norm(fields, "field_norm"), owners, batch=batch)   # head.py:97-109
+    scalars = {n: p[n] for n in ("prior_logit_scale", "joint_logit_scale", "residual_gate")}
+    # Learned scalars on the device stay there (reading them would wait for the stream). Those in host memory, or in 64
+    # bits, which the device form does not take, are read here.
+    on_device = all(isinstance(t, torch.Tensor) and t.device == dev and t.dtype != torch.float64 for t in scalars.values())
+    host = {} if on_device else {n: float(t) for n, t in scalars.items()}
+    prior_scale = 1.0 if on_device else math.exp(min(host["prior_logit_scale"], MAX_LOGIT_SCALE))
     features, prior, cosine = K.head_features_f32(fields_o, norm(options, "option_norm"), questions, global_vector,
-                                                  lex, owners, batch=batch, prior_scale=1.0)
-    residual = dense(dense(features, "residual_scorer.0", gelu=True), "residual_scorer.3")
-    scalars = {n: _dev(p[n], torch.float32, dev) for n in ("prior_logit_scale", "joint_logit_scale", "residual_gate")}
-    logits = K.head_combine_scaled_f32(prior, cosine, residual.reshape(-1), opt_mask.reshape(-1), **scalars)
+                                                  lex, owners, batch=batch, prior_scale=prior_scale)
+    residual = dense(dense(features, "residual_scorer.0", gelu=True), "residual_scorer.3").reshape(-1)
+    if on_device:
+        logits = K.head_combine_scaled_f32(prior, cosine, residual, opt_mask.reshape(-1),
+                                           **{n: t.to(torch.float32) for n, t in scalars.items()})
+    else:
+        logits = K.head_combine_f32(prior, cosine, residual, opt_mask.reshape(-1),
+                                    gate=1.0 / (1.0 + math.exp(-host["residual_gate"])),
+                                    joint_scale=math.exp(min(host["joint_logit_scale"], MAX_LOGIT_SCALE)))
     return logits.reshape(batch, n_opt)

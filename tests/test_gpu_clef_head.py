@@ -293,6 +293,46 @@ def test_head_combine_scaled_f32() -> None:
         assert (abs(got - want) <= 4 * 2.0 ** -24 * size)[live].all() and (got[~live] == -1e9).all()
 
 
+@pytest.mark.parametrize("kind", ["python", "host64", "device64", "device32", "device16"])
+def test_head_scalars_keep_their_precision(kind: str, monkeypatch: pytest.MonkeyPatch) -> None:
+    """Learned scalars in 64 bits are exponentiated in 64 bits wherever they are; those of fewer bits on the device are
+    not read back. The two ways of combining agree to the roundings of their products and sums."""
+    import math
+
+    import torch
+
+    from deciax_amd import clef_head
+    from deciax_amd import kernels as K
+
+    say(f"clef head, learned scalars: {kind}")
+    p, a, hidden, lexical = _random_case(4, batch=2, seq=90, hidden=64, width=32, ff=48, nq=3, no=9, ntypes=3,
+                                         routing_layers=1, layers=1)
+    values = {"prior_logit_scale": 2.1, "joint_logit_scale": 4.3, "residual_gate": 0.7}  # none of them an fp32 number
+    make = {"python": float, "host64": lambda v: torch.tensor(v, dtype=torch.float64),
+            "device64": lambda v: torch.tensor(v, dtype=torch.float64, device="cuda"),
+            "device32": lambda v: torch.tensor(v, device="cuda"),
+            "device16": lambda v: torch.tensor(v, dtype=torch.bfloat16, device="cuda")}[kind]
+    params = _dev_params(p)
+    seen = {}
+    features, combine = K.head_features_f32, K.head_combine_f32
+    monkeypatch.setattr(K, "head_features_f32",
+                        lambda *t, prior_scale, **kw: (seen.update(prior=prior_scale), features(*t, prior_scale=prior_scale, **kw))[1])
+    monkeypatch.setattr(K, "head_combine_f32", lambda *t, **kw: (seen.update(kw), combine(*t, **kw))[1])
+    got = clef_head.forward(params | {n: make(v) for n, v in values.items()}, hidden, lexical, a, heads=4, routing_layers=1,
+                            layers=1)
+    if kind.startswith("device") and kind != "device64":
+        assert seen == {"prior": 1.0}
+    else:
+        assert seen == {"prior": math.exp(2.1), "joint_scale": math.exp(4.3), "gate": 1.0 / (1.0 + math.exp(-0.7))}
+    if kind != "device16":
+        want = clef_head.forward(params | {n: torch.tensor(v, device="cuda") for n, v in values.items()}, hidden, lexical, a,
+                                 heads=4, routing_layers=1, layers=1)
+        live = torch.as_tensor(a["option_mask"]).cuda()
+        # scales of up to e^4.3 from scalars 2^-24 apart, times values of order one, and the roundings after them
+        assert (got - want)[live].abs().max() <= 16 * 2.0 ** -24 * 4.3 * math.exp(4.3)
+        assert torch.equal(got[~live], want[~live])
+
+
 @pytest.mark.parametrize("batch,nq,nk,heads,dh", [
     (1, 1, 1, 1, 16), (2, 17, 65, 3, 32), (1, 6, 600, 16, 64), (2, 33, 130, 2, 48), (1, 5, 70, 2, 80), (1, 40, 64, 2, 96),
     (2, 20, 31, 2, 112), (1, 50, 515, 4, 128), (8, 40, 127, 40, 64), (1, 9, 40, 2, 24),
