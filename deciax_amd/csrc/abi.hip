@@ -78,7 +78,7 @@ int validate_attn_v(int32_t head_dim, int32_t num_kv_heads, int64_t k_row_stride
   const int64_t vec = dtype == DX_BF16 ? 8 : 4;
   REQUIRE(v_row_stride % vec == 0 && v_row_stride >= (int64_t)num_kv_heads * head_dim,
           "attention: bad v row stride %ld", (long)v_row_stride);
-  // row strides whose 32-key block would not fit 32-bit byte offsets: never taken at head_dim 64 and 128
+  // a limit of the interface: no kernel needs it any more, but what was refused stays so
   if (dtype == DX_F32)
     SUPPORTED(head_dim > 128 || (k_row_stride < (INT64_C(1) << 24) && v_row_stride < (INT64_C(1) << 24)),
               "attention: fp32 k / v row strides of 2^24 elements or more are not supported at head_dim %d",

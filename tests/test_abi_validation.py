@@ -63,6 +63,16 @@ def test_head_op_validation() -> None:
     check("dx_gather_rows_f32", _lib.DX_ERR_INVALID, P, P, P, 2, 0, 3, 16, 16, 16, 0, NUL)
     check("dx_head_routing_f32", _lib.DX_ERR_UNSUPPORTED, P, P, P, P, P, 1, 20000, 4, 16, NUL)
     check("dx_head_combine_f32", _lib.DX_OK, P, P, P, P, P, 0, ctypes.c_float(0.5), ctypes.c_float(2.0), NUL)
+    check("dx_span_means_gather_f32", _lib.DX_ERR_INVALID, P, NUL, P, P, 2, 9, 8, 3, 16, 16, 16, NUL)
+    check("dx_span_means_gather_f32", _lib.DX_ERR_INVALID, P, P, P, P, 2, 0, 8, 3, 16, 16, 16, NUL)   # no table rows
+    check("dx_span_means_gather_f32", _lib.DX_ERR_INVALID, P, P, P, P, 2, 9, 0, 3, 16, 16, 16, NUL)   # no positions
+    check("dx_span_means_gather_f32", _lib.DX_ERR_INVALID, P, P, P, P, 2, 9, 8, 3, 16, 8, 16, NUL)    # ldx below d
+    check("dx_span_means_gather_f32", _lib.DX_OK, P, P, P, P, 2, 9, 8, 0, 16, 16, 16, NUL)
+    for hole in range(8):
+        pointers = [NUL if i == hole else P for i in range(8)]
+        check("dx_head_combine_scaled_f32", _lib.DX_ERR_INVALID, *pointers, 4, NUL)
+    check("dx_head_combine_scaled_f32", _lib.DX_ERR_INVALID, P, P, P, P, P, P, P, P, -1, NUL)
+    check("dx_head_combine_scaled_f32", _lib.DX_OK, P, P, P, P, P, P, P, P, 0, NUL)
 
 
 @pytest.mark.parametrize("name", sorted(_lib.SIGNATURES))
@@ -88,6 +98,33 @@ def test_attention_grid_limits() -> None:
     check("dx_transpose_v", _lib.DX_OK, P, P, P, P, P, 0, 64, 2, 128, 256, 4096, NUL)
 
 
+def test_padded_attention_validation() -> None:
+    f = ctypes.c_float
+
+    def padded(q=P, mask=P, batch=2, length=64, nq=64, nk=64, hq=4, hkv=2, d=128, qs=512, ks=256, vs=256, scale=0.1,
+               window=0, dtype=_lib.DX_BF16, ws=P, ws_bytes=1 << 30):
+        return ("dx_attn_padded", q, P, P, mask, P, batch, length, nq, nk, hq, hkv, d, qs, ks, vs, 512, f(scale), f(0.0),
+                window, 1, dtype, ws, ws_bytes, NUL)
+
+    name = "dx_attn_padded"
+    for bad in (dict(q=NUL), dict(mask=NUL), dict(nq=65), dict(nk=65), dict(nk=0), dict(nq=-1), dict(batch=-1),
+                dict(qs=256), dict(ks=128), dict(vs=128), dict(vs=260), dict(scale=0.0), dict(window=-1), dict(dtype=7),
+                dict(q=ctypes.c_void_p(0x10008)), dict(ws=NUL), dict(ws=ctypes.c_void_p(0x10004)),
+                dict(batch=60000, length=60000, nq=60000, nk=60000),
+                dict(ws_bytes=lib().dx_attn_padded_workspace(2, 64, 2, 128, _lib.DX_BF16) - 1)):
+        assert status(*padded(**bad)) == _lib.DX_ERR_INVALID, (bad, lib().dx_last_error())
+        assert b"attention" in lib().dx_last_error()
+    for unsupported in (dict(d=96, qs=384, ks=192, vs=192), dict(hq=16, qs=2048), dict(batch=70000, length=8, nq=8, nk=8),
+                        dict(ks=1 << 26, vs=256, length=64),
+                        dict(dtype=_lib.DX_F32, ks=1 << 24)):
+        assert status(*padded(**unsupported)) == _lib.DX_ERR_UNSUPPORTED, (unsupported, lib().dx_last_error())
+    check(name, _lib.DX_OK, *padded(batch=0)[1:])
+    check(name, _lib.DX_OK, *padded(nq=0)[1:])
+    assert lib().dx_attn_padded_workspace(2, 64, 2, 128, _lib.DX_F32) == 0
+    masked = lib().dx_attn_prefill_masked_workspace(3, 100, 2, 64, _lib.DX_BF16)
+    assert lib().dx_attn_padded_workspace(3, 100, 2, 64, _lib.DX_BF16) == (masked + 255) // 256 * 256 + 24
+
+
 def test_attention_32bit_ranges_refused() -> None:
     """The bf16 kernel's K and V^T buffer ranges are 32-bit: spans of 2 GiB or more are refused
     before any launch instead of wrapping."""
@@ -110,12 +147,12 @@ def test_attention_32bit_ranges_refused() -> None:
     assert packed(2048, 4096) == _lib.DX_ERR_UNSUPPORTED
     assert b"2 GiB" in lib().dx_last_error()
 
-    # fp32: a 32-key block of K or V is read through 32-bit byte offsets, so row strides stop at 2^24
+    # fp32 at head_dim 64 and 128: row strides stop at 2^24, a limit of the interface
     fp32 = status("dx_attn_prefill", P, P, P, P, P, P, 1, 64, 8, 4, 128, 1024, 1 << 24, 512, 1024,
                   f(0.088), f(0.0), 0, 1, _lib.DX_F32, NUL, 0, NUL)
     assert fp32 == _lib.DX_ERR_UNSUPPORTED and b"2^24" in lib().dx_last_error()
-    # the limit is checked before an empty call returns, and only at head_dim 64 / 128: the head_dim 256
-    # kernel addresses with 64-bit pointers, so the same strides pass (empty calls, no launch)
+    # the limit is checked before an empty call returns, and only at head_dim 64 / 128: at head_dim 256 the same strides
+    # pass (empty calls, no launch)
     def fp32_empty(d):
         return status("dx_attn_prefill", P, P, P, P, P, P, 0, 64, 8, 4, d, 8 * d, 1 << 24, 1 << 24, 8 * d,
                       f(0.0625), f(0.0), 0, 1, _lib.DX_F32, NUL, 0, NUL)
