@@ -46,14 +46,14 @@ constexpr int BKV = 64;     // V^T block alignment of dx_transpose_v
 // ring (64 KB), runs two workgroups per CU that fall out of step with each other, so one's prologue,
 // epilogue and barrier waits overlap the other's key loop; it halves the query rows per staged K/V tile.
 // Head_dim 128 takes the short form when a query row sees 2048 keys or fewer on average (window <= 2048,
-// or causal sequences up to 4096): 27B heads, 8 x 2048 -4%, window 512 -12 to -15%, window 1024 -5 to
-// -10%, 16 x 3400 -2%; on longer spans it measured +0.2 to +1.1% (4 x 16384). Head_dim 64 takes it up to 4096
-// keys: its 32 KB ring puts three workgroups on a CU, and half the query rows spread small launches further
-// (12 heads: 2 x 1021 35 -> 30 us, 4 x 2048 83 -> 72, 1 x 2048 42 -> 32, 8 x 1021 49 -> 47; 4 x 8192 +2.8%).
-// Head_dim 256: the short form measured 6-11% slower. Where the long one has at most a workgroup per CU, four waves
-// over the same 4-stage ring (one per SIMD) halve what the longest workgroup has to do: 16/8 heads, 1 x 736 40 -> 31
-// us, 1 x 2000 102 -> 84, 1 x 3300 161 -> 133 (208 workgroups of 8 waves), 4 x 1000 63 -> 59 (256); 1 x 4500 (288)
-// is even, 8 x 1000 (512) 84 -> 114. Two waves measured like four. All forms give the same bits.
+// or causal sequences up to 4096): 27B heads, 8 x 2048 -4%, window 512 -12 to -15%, window 1024 -5 to -10%, 16 x 3400
+// -2%; on longer spans it measured +0.2 to +1.1% (4 x 16384). Head_dim 64 takes it up to 4096 keys: its 32 KB ring puts
+// three workgroups on a CU, and half the query rows spread small launches further (us of the kernel alone, 12 heads, no
+// soft-cap, long -> short: 2 x 1021 37 -> 31, 4 x 2048 105 -> 79, 1 x 2048 49 -> 38, 8 x 1021 57 -> 47, 4 x 8192 causal
+// 605 -> 554). Head_dim 256: the short form measured 6-11% slower. Where the long one has at most a workgroup per CU, four
+// waves over the same 4-stage ring (one per SIMD) halve what the longest workgroup has to do: kernel alone, 16/8 heads,
+// soft-capped, 1 x 736 40 -> 32 us, 1 x 2000 103 -> 87, 1 x 3300 162 -> 137 (208 workgroups of 8 waves), 4 x 1000 61 -> 58
+// (256); 1 x 4500 (288) is even, 8 x 1000 (512) 84 -> 114. Two waves measured like four. All forms give the same bits.
 // bf16 grid order switch (see attn_bf16_kernel). Whole units per XCD measured 3-9% faster at 3257-4096
 // tokens (16 sequences, 9B and 27B heads), 2% slower at 8 x 3072 and 15% slower at 8 x 2048.
 constexpr int SHORT_SEQ = 3072;
@@ -140,8 +140,8 @@ struct Flag {
 // 32 w + j) hides keys beyond the causal / window rule. Tiles that hold a masked key take the masked body,
 // and a query row that sees no key is written as zeros.
 // Waves per SIMD that the registers are kept for: what the ring lets a CU hold. Head_dim 64's short form (32 KB) runs
-// three, 136 registers a lane for 169: its loop waits on exponentials and LDS more than on the matrix core. 12 heads,
-// 8 x 1021 68 -> 59 us; 16 heads, 12 x 2048 312 -> 289, window 64 94 -> 80; four measured like three.
+// three: its loop waits on exponentials and LDS more than on the matrix core. Kernel alone, two -> three, us: 12 heads, 8 x
+// 1021 58 -> 47, 4 x 2048 87 -> 79; 16 heads, 12 x 2048 284 -> 269, window 64 64 -> 53; four measured like three.
 constexpr int waves_least(int d, int waves, int stages) {
   return waves * stages == 16 ? 1 : d == 64 && waves == 4 ? 3 : 2;
 }
@@ -536,8 +536,9 @@ DX_DEVICE floatx4 mfma16_f32(float a, float b, floatx4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
+// Registers for two workgroups a CU at head_dim 64 (4 x 1024, 32/8 heads 275 -> 219 us), one above.
 template <int D, int QB, int WAVES, int SUB>
-__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(1, 1)))
+__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 1, D == 64 ? 4 : 1)))
 attn_f32_kernel(const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V,
                     float *__restrict__ O, const int32_t *__restrict__ seq_start, const int32_t *__restrict__ seq_len,
                     int max_seq_len, int hq, int hkv, long q_stride, long k_stride, long v_stride, long o_stride,
