@@ -256,12 +256,14 @@ linear_f32_kernel(const float *__restrict__ x, const float *__restrict__ w, cons
 // below 2^-17 |x|, so 2^-25 for each of the first two): the rounding of an fp32 product at most. The pair of accumulators
 // joins the sum after every PART k. Error against 64 bits at k = 1024 / 4096: 1.0e-7 / 1.2e-7 (over all of k 1.9e-7 /
 // 4.0e-7; both accumulators in one 3.4e-7 / 7.2e-7; fp32 MFMAs in one chain 4.0e-7 / 8.2e-7, in four 2.9e-7 / 5.7e-7).
-// bf16 has fp32's exponents, so l of an operand below 2^-109 (1.5e-33) falls under the smallest bf16: rows that hold no
-// larger value lose bits of it (error 2.7e-6 at 1e-35, 2.7e-4 at 1e-37).
 // Two kernels, the same chain of MFMAs and sums for an output in both, so that a row does not depend on m.
-// An infinity, a NaN or a value past the largest bf16 leaves its row or column of the accumulators not finite (inf -
-// inf): those outputs, and no others, are multiplied again with fp32 MFMAs.
+// Some outputs, and no others, are multiplied again with fp32 MFMAs: those that are not finite (an infinity, a NaN or a
+// value past the largest bf16 leaves its row or column so, inf - inf), and those below 2^-84. bf16 has fp32's exponents, so
+// an operand below 2^-109 loses bits of l (error 2.7e-6 at 1e-35, 2.7e-4 at 1e-37), and its row's outputs are that small
+// unless the other operand is past 2^24 / k.
 constexpr int PART = 256;
+
+DX_DEVICE bool outside_split(float v) { return !(fabsf(v) < INFINITY) || (fabsf(v) < 0x1p-84f && v != 0.f); }
 
 DX_DEVICE void split3(const floatx4 &v, u32x2 (&p)[3]) {
   float a[4] = {v[0], v[1], v[2], v[3]};
@@ -499,7 +501,7 @@ linear_split_small_kernel(const float *__restrict__ x, const float *__restrict__
   if (wave < 4)
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (!(fabsf(total[e]) < INFINITY)) *bad = 1;
+      if (outside_split(total[e])) *bad = 1;
   __syncthreads();
   const long row = m0 + lrow;
   if (*bad) {
@@ -512,7 +514,7 @@ linear_split_small_kernel(const float *__restrict__ x, const float *__restrict__
     if (wave < 4) {
       const floatx4 f = sums[0][wave][lane];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) total[e] = fabsf(total[e]) < INFINITY ? total[e] : f[e];
+      for (int e = 0; e < 4; ++e) total[e] = outside_split(total[e]) ? f[e] : total[e];
     }
   }
   if (wave < 4 && row < m) {
@@ -641,7 +643,7 @@ linear_split_kernel(const float *__restrict__ x, const float *__restrict__ w, co
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        bad = bad || !(fabsf(total[i][j][r]) < INFINITY);
+        bad = bad || outside_split(total[i][j][r]);
       }
   if (__builtin_amdgcn_ballot_w64(bad)) {
 #pragma unroll
@@ -651,7 +653,7 @@ linear_split_kernel(const float *__restrict__ x, const float *__restrict__ w, co
         const floatx16 f = product32_f32(x + min(m0 + wm * 32 * TM + 32 * i + lrow, m - 1) * ldx,
                                          w + (long)min(n0 + wn * 32 * TN + 32 * j + lrow, n - 1) * ldw, k, lhalf);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) total[i][j][r] = fabsf(total[i][j][r]) < INFINITY ? total[i][j][r] : f[r];
+        for (int r = 0; r < 16; ++r) total[i][j][r] = outside_split(total[i][j][r]) ? f[r] : total[i][j][r];
       }
   }
 #pragma unroll

@@ -225,6 +225,30 @@ def test_linear_f32_split_tiles(m: int, n: int, k: int, pad: int, scale: float) 
     assert ((got - base.double() - act).abs() <= 1.2 * bound + 2.0 ** -21 * (act.abs() + base.double().abs()) + 1e-6).all()
 
 
+@pytest.mark.parametrize("m", [20, 600, 4100])
+@pytest.mark.parametrize("scale", [1e-33, 1e-35, 1e-37])
+def test_linear_f32_split_tiny_rows(m: int, scale: float) -> None:
+    """Rows below the range in which three bf16 hold an fp32 number keep an fp32 sum's bound (k 2^-24 sum |x w|, a
+    denormal's half unit per product), in every tile, beside rows of ordinary size and of zeros."""
+    import torch
+
+    from deciax_amd import kernels as K
+
+    say(f"linear_f32 split, {m} rows, every other scaled by {scale}")
+    r = rng(m)
+    n, k = 1000, 260
+    x = torch.as_tensor(r.normal(size=(m, k)).astype(np.float32)).cuda()
+    w = torch.as_tensor(r.normal(size=(n, k)).astype(np.float32)).cuda()
+    x[::2] *= scale
+    x[5] = 0
+    want = x.double() @ w.double().t()
+    bound = (k + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) + k * 2.0 ** -150
+    got = K.linear_f32(x, w).double()
+    assert ((got - want).abs() <= bound).all() and (got[5] == 0).all()
+    ordinary = K.linear_f32(x[1::2].contiguous(), w).double()
+    assert torch.equal(got[1::2], ordinary)
+
+
 def test_linear_f32_split_not_finite() -> None:
     """Infinities, NaN and values past the largest bf16 give what fp32 products give."""
     import torch
