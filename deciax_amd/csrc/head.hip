@@ -790,6 +790,17 @@ DX_DEVICE void load_run(float (&v)[N], const float *p) {  // N consecutive float
   }
 }
 
+// e^d for d <= 0 (or NaN), within some two units in the last place: 2^n 2^f with n the integer nearest to d log2(e) and f
+// what is left, log2(e) in two parts (Cody and Waite's reduction). expf without its tests for large results: 8 vector
+// instructions for 13. Below the smallest number f, or the scaling by 2^n, ends in 0.
+DX_DEVICE float exp_below0(float d) {
+  constexpr double LOG2E = 1.4426950408889634074;
+  constexpr float HI = (float)LOG2E, LO = (float)(LOG2E - (double)HI);
+  const float n = rintf(fmaxf(d * HI, -300.f));
+  const float f = __builtin_fmaf(d, LO, __builtin_fmaf(d, HI, -n));
+  return ldexpf(fast_exp2(f), (int)n);
+}
+
 template <int N, int QB, int WAVES, int SUB>
 __global__ void __launch_bounds__(64 * WAVES)
 mha_f32_mfma_kernel(const float *__restrict__ q, const float *__restrict__ k, const float *__restrict__ v,
@@ -862,7 +873,7 @@ mha_f32_mfma_kernel(const float *__restrict__ q, const float *__restrict__ k, co
       mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
       const float mn = fmaxf(mr[u], mx);
-      const float alpha = expf(mr[u] - mn);
+      const float alpha = exp_below0(mr[u] - mn);
       mr[u] = mn;
       l[u] *= alpha;
       if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {
@@ -873,7 +884,7 @@ mha_f32_mfma_kernel(const float *__restrict__ q, const float *__restrict__ k, co
       for (int s = 0; s < SUB; ++s)
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-          const float p = expf(sc[u][s][t] - mn);
+          const float p = exp_below0(sc[u][s][t] - mn);
           sc[u][s][t] = p;
           l[u] += p;
         }
@@ -921,7 +932,7 @@ mha_f32_mfma_kernel(const float *__restrict__ q, const float *__restrict__ k, co
     float num = 0.f, den = 0.f;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
-      const float f = expf(ms[w][qi] - mx);
+      const float f = exp_below0(ms[w][qi] - mx);
       num += os[w][qi][d] * f;
       den += ls[w][qi] * f;
     }
