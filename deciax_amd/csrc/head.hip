@@ -1154,15 +1154,16 @@ hipError_t dx_linear_f32_launch(const float *x, const float *w, const float *bia
                       ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
   if (chunks) {
     const int vec_y = (ldy & 3) == 0 && ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(bias)) & 15) == 0;
-    // us per 1024 k: 128 x 128 tiles 46 a round of 256 workgroups and 10, 128 x 64 tiles 28 and 6, 32 x 32 tiles 7 for
+    // us per 1024 k: 128 x 128 tiles 46 a round of 256 workgroups and 17, 128 x 64 tiles 28 and 6, 32 x 32 tiles 7 for
     // one round, then 2 and 0.0215 a tile. Measured us, 32 x 32 / 128 x 64 / 128 x 128 (fp32 or split products chosen by
     // m, before):
     //   23 x 1024 x 1024: 8 / 33 / 56 (6)       23 x 1024 x 4096: 22 / 126 / 210 (20)     200 x 1024 x 4096: 24 / 137 / 212 (34)
     //   600 x 1024 x 4096: 67 / 139 / 214 (73)  600 x 2048 x 1024: 29 / 38 / 59 (35)      2000 x 1024 x 1024: 45 / 42 / 61 (38)
-    //   4096 x 1024 x 4096: 339 / 229 / 231 (197)   4096 x 2048 x 4096: 689 / 453 / 374 (357)
+    //   4096 x 1024 x 1024: 89 / 63 / 69 (59)   4096 x 1024 x 4096: 339 / 229 / 231 (197)
+    //   4096 x 2048 x 4096: 689 / 453 / 374 (357)
     //   32768 x 1024 x 4096: 2812 / 1619 / 1395 (1296)
     const long wide = tiles(128, 128), slim = tiles(128, 64), few = tiles(32, 32);
-    const double wide_us = 46. * ((wide + 255) / 256) + 10, slim_us = 28. * ((slim + 255) / 256) + 6;
+    const double wide_us = 46. * ((wide + 255) / 256) + 17, slim_us = 28. * ((slim + 255) / 256) + 6;
     const double few_us = few <= 256 ? 7 : 0.0215 * few + 2;
     if (few_us <= fmin(wide_us, slim_us)) {
       // eight parts of k at once, or four in rings of 32 columns
