@@ -397,7 +397,9 @@ int dx_layer_norm_f32(const float *x, const float *w, const float *b, float *y,
  * act DX_ACT_NONE or DX_ACT_GELU_ERF (exact GELU, jax.nn.gelu with
  * approximate=False). Replaces `linear` (src/deciax/nn.py:11-19) / `dense`
  * (src/deciax/models/qwen3_5/text.py:21-22) with the head's residual adds
- * (head.py:71-74,92-95) folded in. bias nullable. */
+ * (head.py:71-74,92-95) folded in. bias nullable. The order of an output's sum
+ * is set by n, k and the strides and alignment of x and w, not by m, so a row
+ * has the same bits in every launch that holds it. */
 int dx_linear_f32(const float *x, const float *w, const float *bias, float *y,
                   int64_t m, int64_t n, int64_t k, int64_t ldx, int64_t ldw,
                   int64_t ldy, int32_t activation, int32_t accumulate,

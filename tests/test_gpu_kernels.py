@@ -61,9 +61,9 @@ def test_linear_bf16(m: int, n: int, k: int) -> None:
 
 @pytest.mark.parametrize("n,k", [(3584, 4096), (3584, 14336), (1024, 2048)])
 def test_linear_rows_do_not_depend_on_m(n: int, k: int) -> None:
-    """Small M takes other tile shapes (64 x 128 below 64 standard tiles, 128 x 256 up to 1024 rows,
-    256 x 256 above), and long K another load path; every row must still equal the same row of a
-    4096-row product, bf16 and fp32 out, so a request's result does not depend on its batch."""
+    """Each M takes the tile shape that its rounds over the chip favour, from 32 x 32 to 256 x 256; every row
+    must still equal the same row of a 4096-row product, bf16 and fp32 out, so a request's result does not
+    depend on its batch."""
     import torch
 
     from deciax_amd import kernels as K
