@@ -233,9 +233,9 @@ def test_full_size_batch_order_invariance(model: str) -> None:
 @pytest.mark.parametrize("model", ["gemma2-9b", "gemma2-27b"])
 def test_request_alone_equals_request_in_batch(model: str) -> None:
     """A request's logits and probabilities are bit-identical alone and inside a larger batch, across
-    the switches between tile shapes that follow the row count (64 x 128 plain-epilogue tiles for one
-    short request, 128-row tiles up to 1024 rows, 256-row tiles above) and between the attention grid
-    orders (batches up to 4096 tokens per sequence launch tile-major): every GEMM row, norm row,
+    the switches between tile shapes that follow the row count (ring tiles of 64 to 192 rows for one
+    short request, 192- and 256-row tiles for the batch) and between the attention grid orders
+    (batches up to 3072 tokens per sequence launch tile-major): every GEMM row, norm row,
     attention row and readout question depends only on its own request. Full depth."""
     from deciax_amd import gemma
 
